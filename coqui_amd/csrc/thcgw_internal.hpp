@@ -94,14 +94,16 @@ constexpr int GEMM_HERM_SUB = 256;
 // process-wide setting (gemm_set_complex3) says for FP32 products.
 constexpr int GEMM_G3 = 2048;
 
-// C[b] = alpha * op(A[b]) * op(B[b]) + beta * C[b] + gamma * I   (row-major, M x N)
+// C[b] = alpha * op(A[b]) * op(B[b]) + beta * C[b] + gamma * I   (row-major, M x N), for
+// op(A), op(B) = N,N or N,C or C,N
 void zgemm(hipStream_t s, int opA, int opB, int M, int N, int K, Cplx alpha, BatchPtr A, long lda,
            BatchPtr B, long ldb, Cplx beta, c128* C, long strideC, long ldc, int batch,
            Cplx gamma = Cplx{0.0, 0.0}, int tri = 0, BatchPtr hsub = BatchPtr{nullptr, 0, 1, 1, 0});
 
 // The same product in FP32 arithmetic (complex<float> MFMA, FP32 accumulation) with each
 // operand and the result stored as complex<double> or complex<float> (ta, tb, tc); alpha,
-// beta and gamma are applied in double.  Ops N/T/C for A and B in {N, C} x {N, C}.
+// beta and gamma are applied in double.  Only the products of the mixed-precision forms are
+// built (see the dispatch in zgemm.hip); the others are refused.
 void cgemm(hipStream_t s, int opA, int opB, int M, int N, int K, Cplx alpha, BatchPtr A, Dt ta, long lda,
            BatchPtr B, Dt tb, long ldb, Cplx beta, void* C, Dt tc, long strideC, long ldc, int batch,
            Cplx gamma = Cplx{0.0, 0.0}, int tri = 0, BatchPtr hsub = BatchPtr{nullptr, 0, 1, 1, 0});
@@ -164,8 +166,6 @@ void trsm_left_upper_unit(hipStream_t s, const c128* U, long sU, int ldu, c128* 
 void potrf_batched(hipStream_t s, c128* A, long sA, int lda, int n, int* info, int batch);
 void trsm_right_lower_conj(hipStream_t s, const c128* L, long sL, int ldl, c128* T, long sT, int ldt, int m, int nb,
                            int batch);
-void trsm_right_lower_conj_f32(hipStream_t s, const c128* L, long sL, int ldl, c64* T, long sT, int ldt, int m,
-                               int nb, int batch, int gemm_flags = 0);
 void trsm_right_lower_conj_f32(hipStream_t s, const c64* L, long sL, int ldl, c64* T, long sT, int ldt, int m,
                                int nb, int batch, int gemm_flags = 0);
 void zero_upper(hipStream_t s, c128* A, long sA, int n, int batch);

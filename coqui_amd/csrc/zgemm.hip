@@ -6,14 +6,24 @@
 //   C[b] = alpha * op(A[b]) * op(B[b]) + beta * C[b] + gamma * I,   op in {N, T, C}
 //
 // All matrices are row-major with explicit leading dimensions.  One 256-thread
-// workgroup (four waves, 2 x 2) computes a BM x BN tile of C; each wave owns a
-// (BM/2) x (BN/2) sub-tile made of v_mfma_f64_16x16x4_f64 blocks with separate real
-// and imaginary accumulators (a complex multiply-add is four real MFMAs, or three in the
-// G3 variant: Ar Br, Ai Bi and (Ar + Ai)(Br + Bi), combined after the K loop).  Two tile
-// shapes are built: 128 x 128 (4 x 4 MFMA blocks per wave, accumulators in 256 AGPRs,
-// one wave per SIMD) for large products and 64 x 64 (2 x 2 blocks) for small ones.
-// K is staged through LDS in chunks of 8 complex values, double buffered, so the next
-// chunk's global loads overlap the current chunk's MFMAs.
+// workgroup (four waves, 2 x 2) computes a BM x BN tile of C; each wave owns every other
+// 16 x 16 MFMA block of the tile in both directions, with separate real and imaginary
+// accumulators (a complex multiply-add is four real MFMAs, or three in the G3 variant:
+// Ar Br, Ai Bi and (Ar + Ai)(Br + Bi), combined after the K loop).  64 x 64 tiles (2 x 2
+// blocks per wave) serve every product by default; 128-wide tiles can be selected.
+// K is staged through LDS in chunks of 8 (FP64) or 16 (FP32) complex values, double buffered.
+//
+// What bounds it: the matrix cores, and in second place their issue slots.  Registers-only
+// MFMAs reach 77.4 TFLOP/s in FP64 on MI355X (154.5 in FP32); every vector instruction
+// between them takes issue cycles away, and so does a wave that waits for LDS while its
+// neighbours on the SIMD wait too.  Hence the main loop without vector instructions (TileIO),
+// the signs of conjugation and of Ai Bi in the MFMA instruction itself, and fragments
+// read one K step ahead.  Order-1600 batches, TFLOP/s of 8 M N K flops (first version, with a
+// bounds test per element, address arithmetic per chunk and fragments read when needed ->
+// now): dense N,N 66.7 -> 71.3, with three products 80.4 -> 87.9; Z Z^H (lower, K from the row,
+// Hermitian epilogue, three products) 55.6 -> 74.7; L L^H updates of order 800 53.8 -> 72.5.
+// The last two gained most from the epilogue: C (or H) used to be read, waited for and
+// written element by element, 16 memory latencies per wave.  Results are bit-identical.
 //
 // Workgroups are dispatched round-robin over the 8 XCDs; the block index is remapped
 // so that each XCD receives a contiguous range of (batch, tile) work.  The tiles of one
@@ -22,6 +32,7 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace thcgw {
@@ -35,6 +46,8 @@ constexpr int NXCD = 8;
 
 struct Args {
   int M, N, K, batch, tiles_m, tiles_n, tri;
+  int tiles;   // workgroups per matrix
+  int packed;  // 1: only the lower tiles of a square grid have workgroups
   double ar, ai, br, bi, gr, gi;
   BatchPtr A, B;
   BatchPtr H;  // GEMM_HERM_SUB: complex<double> matrix subtracted from the Hermitian result
@@ -51,8 +64,13 @@ struct Arith<double> {
   using cplx = c128;
   using acc = f64x4;
   static constexpr int BK = 8;     // K chunk staged per LDS buffer
-  static constexpr int WAVES = 3;  // waves per SIMD the register budget is held to
-  __device__ static acc mfma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+  static constexpr int WAVES = 4;  // waves per SIMD the register budget is held to (three products: one less)
+  // c + a b, with NEG c - a b: the FP64 instruction negates its A operand itself (its last
+  // immediate holds the sign bits of A, B and C; checked on gfx950)
+  template <bool NEG = false>
+  __device__ static acc mfma(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, NEG ? 1 : 0);
+  }
   // accumulator register v of lane l holds row l/16 + 4v, column l%16 (checked on gfx950)
   __device__ static int row(int lk, int v) { return lk + 4 * v; }
 };
@@ -62,7 +80,10 @@ struct Arith<float> {
   using acc = f32x4;
   static constexpr int BK = 16;
   static constexpr int WAVES = 4;
-  __device__ static acc mfma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+  template <bool NEG = false>
+  __device__ static acc mfma(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(NEG ? -a : a, b, c, 0, 0, 0);
+  }
   // accumulator register v of lane l holds row 4(l/16) + v, column l%16 (checked on gfx950)
   __device__ static int row(int lk, int v) { return 4 * lk + v; }
 };
@@ -73,20 +94,15 @@ __device__ __forceinline__ const T* batch_ptr(const BatchPtr& p, int b) {
 }
 
 template <typename RC, typename T>
-__device__ __forceinline__ RC ld_elem(const T* X, long ld, int r, int c, int R, int Cn, bool conj) {
+__device__ __forceinline__ RC cvt_elem(const T v) {
   using S = decltype(RC{}.x);
-  if (r < R && c < Cn) {
-    const T v = X[static_cast<long>(r) * ld + c];
-    return RC{static_cast<S>(v.x), static_cast<S>(conj ? -v.y : v.y)};
-  }
-  return RC{0, 0};
+  return RC{static_cast<S>(v.x), static_cast<S>(v.y)};
 }
 
 // Tile of an operand: BX elements along its free dimension x (m for op(A), n for op(B))
 // times BK along k, staged in LDS as S[k][x ^ swz(k)].  ROWS: element (x, k) is stored at X[x][k]
 // (op(A) = A, op(B) = B^T or B^H); otherwise at X[k][x] (op(A) = A^T or A^H, op(B) = B).
-// CONJ conjugates on load.  Pairs of adjacent elements along the contiguous direction
-// are loaded together; each thread loads P = BX*BK/(2*NT) pairs.
+// Conjugation is left to the signs of the products.
 // Column swizzle of LDS row k (rows are 1-2 KB apart, so every row starts in bank 0).
 //   complex<double> (16 B): a K-contiguous store group (16 lanes) writes columns 0..3 of
 //     rows 0, 2, 4, 6; XOR-ing the column with 4 (k/2) gives the 16 lanes distinct bank
@@ -101,46 +117,94 @@ __device__ __forceinline__ int swz(int k) {
   else return (((k >> 1) & 7) << 2) ^ ((k & 1) << 4);
 }
 
-template <typename RC, typename T, bool ROWS, bool CONJ, int BX, int BK>
+// Every vector instruction of a wave takes issue cycles from the matrix core of its SIMD (one
+// 32-bit operation per FP64 MFMA: 77 -> 73 TFLOP/s, two: 66), so the main loop has next to
+// none: a chunk's loads add a constant 32-bit lane offset to a uniform base that scalar
+// instructions move along, and all LDS addresses are a lane constant plus an immediate (the
+// loop is unrolled over the two buffers).
+//   ROWS: a thread takes pairs of adjacent k (one 16-byte load per pair of complex<float>).
+//   otherwise: a wave takes 64 consecutive x of one k per load.
+// Rows and columns past the operand's edge are clamped to its last one: they only feed
+// results that are not stored, so a full chunk needs no bounds test.
+template <typename RC, typename T, bool ROWS, int BX, int BK>
 struct TileIO {
-  static constexpr int P = BX * BK / (2 * NT);
-  __device__ static void coords(int t, int p, int& x, int& k) {
-    const int q = t + p * NT;  // pair id
-    if (ROWS) {                // contiguous along k: BK/2 pairs per x
-      x = q / (BK / 2);
-      k = (q % (BK / 2)) * 2;
-    } else {  // contiguous along x: BX/2 pairs per k
-      k = q / (BX / 2);
-      x = (q % (BX / 2)) * 2;
-    }
-  }
-  __device__ static void load(const T* X, long ld, int nx, int nk, int x0, int k0, RC (&r)[2 * P]) {
+  static constexpr int E = BX * BK / NT;   // elements per thread
+  static constexpr int SEG = BX / 64;      // 64-wide segments of a k row (not ROWS)
+  static constexpr int NOFF = ROWS ? E / 2 : SEG;
+  const char* base;  // uniform: the chunk's first element (of the wave's first k row if not ROWS)
+  long ldb;          // bytes between k rows (not ROWS)
+  unsigned off[NOFF];
+  int lds[E];        // element index in a buffer of this thread's element e (not ROWS) or pair e / 2
+
+  __device__ static int wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+  __device__ static int kpair(int p) { return ((threadIdx.x + p * NT) % (BK / 2)) * 2; }
+  __device__ static int krow(int e) { return (wave() + 4 * e) / SEG; }  // k of element e (not ROWS), uniform
+
+  __device__ void init(const T* X, long ld, int nx, int x0, int k0) {
+    if constexpr (ROWS) {
+      base = reinterpret_cast<const char*>(X + static_cast<long>(x0) * ld + k0);
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      int x, k;
-      coords(threadIdx.x, p, x, k);
-      if (ROWS) {
-        r[2 * p] = ld_elem<RC>(X, ld, x0 + x, k0 + k, nx, nk, CONJ);
-        r[2 * p + 1] = ld_elem<RC>(X, ld, x0 + x, k0 + k + 1, nx, nk, CONJ);
-      } else {
-        r[2 * p] = ld_elem<RC>(X, ld, k0 + k, x0 + x, nk, nx, CONJ);
-        r[2 * p + 1] = ld_elem<RC>(X, ld, k0 + k, x0 + x + 1, nk, nx, CONJ);
+      for (int p = 0; p < E / 2; ++p) {
+        const int x = (threadIdx.x + p * NT) / (BK / 2), k = kpair(p);
+        off[p] = static_cast<unsigned>((static_cast<long>(min(x, nx - 1 - x0)) * ld + k) * sizeof(T));
+        lds[2 * p] = k * BX + (x ^ swz<RC>(k));
+        lds[2 * p + 1] = (k + 1) * BX + (x ^ swz<RC>(k + 1));
+      }
+    } else {
+      ldb = ld * static_cast<long>(sizeof(T));
+      base = reinterpret_cast<const char*>(X + x0) + k0 * ldb;
+#pragma unroll
+      for (int g = 0; g < SEG; ++g)
+        off[g] = static_cast<unsigned>(min(g * 64 + static_cast<int>(threadIdx.x & 63), nx - 1 - x0) * sizeof(T));
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int k = krow(e), x = ((wave() + 4 * e) % SEG) * 64 + (threadIdx.x & 63);
+        lds[e] = k * BX + (x ^ swz<RC>(k));
       }
     }
   }
-  __device__ static void store(RC (*S)[BX], const RC (&r)[2 * P]) {
+  // The chunk with nk values of k left (a full one if TAIL is false); moves on to the next one.
+  template <bool TAIL>
+  __device__ void load(int nk, RC (&r)[E]) {
+    if constexpr (ROWS) {
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      int x, k;
-      coords(threadIdx.x, p, x, k);
-      if (ROWS) {
-        S[k][x ^ swz<RC>(k)] = r[2 * p];
-        S[k + 1][x ^ swz<RC>(k + 1)] = r[2 * p + 1];
-      } else {
-        S[k][x ^ swz<RC>(k)] = r[2 * p];
-        S[k][(x + 1) ^ swz<RC>(k)] = r[2 * p + 1];
+      for (int p = 0; p < E / 2; ++p) {
+        const char* q = base + lane_offset(off[p]);
+        if constexpr (TAIL) {
+          r[2 * p] = r[2 * p + 1] = RC{0, 0};
+          if (kpair(p) < nk) r[2 * p] = cvt_elem<RC>(reinterpret_cast<const T*>(q)[0]);
+          if (kpair(p) + 1 < nk) r[2 * p + 1] = cvt_elem<RC>(reinterpret_cast<const T*>(q)[1]);
+        } else if constexpr (sizeof(T) == 8) {
+          typedef float f4 __attribute__((ext_vector_type(4), aligned(8)));
+          const f4 v = *reinterpret_cast<const f4*>(q);
+          r[2 * p] = cvt_elem<RC>(T{v.x, v.y});
+          r[2 * p + 1] = cvt_elem<RC>(T{v.z, v.w});
+        } else {
+          r[2 * p] = cvt_elem<RC>(reinterpret_cast<const T*>(q)[0]);
+          r[2 * p + 1] = cvt_elem<RC>(reinterpret_cast<const T*>(q)[1]);
+        }
       }
+      base += BK * sizeof(T);
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const char* row = base + krow(e) * ldb;
+        r[e] = RC{0, 0};
+        const unsigned o = lane_offset(off[SEG == 1 ? 0 : (wave() + 4 * e) % SEG]);
+        if (!TAIL || krow(e) < nk) r[e] = cvt_elem<RC>(*reinterpret_cast<const T*>(row + o));
+      }
+      base += BK * ldb;
     }
+  }
+  // Keeps the offset's widening to 64 bits next to the load, where it folds into the load's
+  // scalar-base form; hoisted out of the loop it costs a register and an addition per load.
+  __device__ static unsigned lane_offset(unsigned& o) {
+    asm volatile("" : "+v"(o));
+    return o;
+  }
+  __device__ void store(RC* S, const RC (&r)[E]) const {
+#pragma unroll
+    for (int e = 0; e < E; ++e) S[lds[e]] = r[e];
   }
 };
 
@@ -150,14 +214,15 @@ struct TileIO {
 template <typename R, typename TA, typename TB, typename TC, int OPA, int OPB, int BM, int BN, bool FOLD = false,
           bool G3 = false>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(
-    BM == 64 ? (FOLD ? (G3 ? 2 : 3) : Arith<R>::WAVES) : (BN == 64 || sizeof(R) == 4 ? 2 : 1))))
+    BM == 64 ? (FOLD ? (G3 ? 2 : 3) : Arith<R>::WAVES - (G3 ? 1 : 0)) : (BN == 64 || sizeof(R) == 4 ? 2 : 1))))
 void gemm_kernel(Args p) {
   using AR = Arith<R>;
   using RC = typename AR::cplx;
   constexpr int BK = AR::BK;
   constexpr int TM = BM / 32, TN = BN / 32;  // 16x16 MFMA blocks per wave (waves are 2 x 2)
-  using IOA = TileIO<RC, TA, OPA == OP_N, OPA == OP_C, BM, BK>;  // op(A)(m,k): A[m][k] or A[k][m]
-  using IOB = TileIO<RC, TB, OPB != OP_N, OPB == OP_C, BN, BK>;  // op(B)(k,n): B[k][n] or B[n][k]
+  using IOA = TileIO<RC, TA, OPA == OP_N, BM, BK>;  // op(A)(m,k): A[m][k] or A[k][m]
+  using IOB = TileIO<RC, TB, OPB != OP_N, BN, BK>;  // op(B)(k,n): B[k][n] or B[n][k]
+  constexpr bool CA = OPA == OP_C, CB = OPB == OP_C;  // conjugated operands: signs of the products
   __shared__ RC As[2][BK][BM];
   __shared__ RC Bs[2][BK][BN];
 
@@ -168,11 +233,19 @@ void gemm_kernel(Args p) {
   const int base = nblk / NXCD, rem = nblk % NXCD;
   const int logical = xcd * base + (xcd < rem ? xcd : rem) + loc;
 
-  const int tiles = p.tiles_m * p.tiles_n;
-  const int b = logical / tiles;
-  const int tile = logical % tiles;
-  const int m0 = (tile / p.tiles_n) * BM;
-  const int n0 = (tile % p.tiles_n) * BN;
+  const int b = logical / p.tiles;
+  const int tile = logical - b * p.tiles;
+  int tm, tn;
+  if (p.packed) {  // the lower tiles of a square product, row by row
+    tm = static_cast<int>((sqrtf(8.0f * static_cast<float>(tile) + 1.0f) - 1.0f) * 0.5f);
+    while ((tm + 1) * (tm + 2) / 2 <= tile) ++tm;
+    while (tm * (tm + 1) / 2 > tile) --tm;
+    tn = tile - tm * (tm + 1) / 2;
+  } else {
+    tm = tile / p.tiles_n;
+    tn = tile - tm * p.tiles_n;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
 
   // Triangular structure (see GEMM_TRI_*): skip tiles strictly above the diagonal and
   // start the K loop where a triangular operand's band begins.
@@ -192,11 +265,15 @@ void gemm_kernel(Args p) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
   const int lr = lane & 15, lk = lane >> 4;
+  // first row / column of the wave's 16 x 16 blocks: the two waves of a direction take turns, so
+  // a tile with at most half of its rows (columns) inside the matrix is the first blocks' work
+  const auto row0 = [&](int i) { return i * 32 + wm * 16; };
+  const auto col0 = [&](int j) { return j * 32 + wn * 16; };
 
   // G3: three real products per complex product (Gauss): cr accumulates Re a Re b, ci
-  // Im a Im b and cs (Re a + Im a)(Re b + Im b); after the K loop (with FOLD: after every K
-  // chunk, before the chunk is added into the FP64 accumulators) Re c = cr - ci and
-  // Im c = cs - cr - ci.
+  // Im a Im b (unconjugated: its sign is applied afterwards) and cs (Re a + Im a)(Re b + Im b);
+  // after the K loop (with FOLD: after every K chunk, before the chunk is added into the FP64
+  // accumulators) Re c = cr - ci and Im c = cs - cr - ci.
   constexpr int GT = G3 ? TM : 1, GN = G3 ? TN : 1;
   typename AR::acc cr[TM][TN], ci[TM][TN], cs[GT][GN];
 #pragma unroll
@@ -224,106 +301,156 @@ void gemm_kernel(Args p) {
 
   const int nk = (k_hi + BK - 1) / BK;
   const int kt0 = k_lo / BK;
-  RC ra[2 * IOA::P], rb[2 * IOB::P];
-  if (kt0 < nk) {
-    IOA::load(A, p.lda, p.M, p.K, m0, k_lo, ra);
-    IOB::load(B, p.ldb, p.N, p.K, n0, k_lo, rb);
-    IOA::store(As[0], ra);
-    IOB::store(Bs[0], rb);
-  }
-  __syncthreads();
-
-  for (int kt = kt0; kt < nk; ++kt) {
-    const int cur = (kt - kt0) & 1;
-    if (kt + 1 < nk) {
-      IOA::load(A, p.lda, p.M, p.K, m0, (kt + 1) * BK, ra);
-      IOB::load(B, p.ldb, p.N, p.K, n0, (kt + 1) * BK, rb);
+  RC ra[IOA::E], rb[IOB::E];
+  IOA ia;
+  IOB ib;
+  ia.init(A, p.lda, p.M, m0, k_lo);
+  ib.init(B, p.ldb, p.N, n0, k_lo);
+  // chunk kt into registers; only the operands' last chunk can be short
+  auto fetch_full = [&] {
+    ia.template load<false>(BK, ra);
+    ib.template load<false>(BK, rb);
+  };
+  auto fetch = [&](int kt) {
+    const int left = p.K - kt * BK;
+    if (left >= BK) {
+      fetch_full();
+    } else {
+      ia.template load<true>(left, ra);
+      ib.template load<true>(left, rb);
     }
+  };
+  // LDS index of the fragment of 16-block i in K step ks, without the row part 4 ks (an
+  // immediate): swz(4 ks + lk) = swz(4 ks) ^ swz(lk), so the lane part and the constants separate.
+  const int fa0 = lk * BM + ((wm * 16 + lr) ^ swz<RC>(lk));
+  const int fb0 = lk * BN + ((wn * 16 + lr) ^ swz<RC>(lk));
+
+  // Software pipeline over K steps of 4: the fragments of the next step are read from LDS while
+  // the MFMAs of the current one run, across the chunk boundary too.  Before a chunk's last
+  // step the next chunk's values (fetched one chunk earlier) go to the other LDS buffer, the
+  // fetch of the chunk after it starts, and the chunk's only barrier follows: every read of
+  // that buffer was waited for before the previous barrier.  The scheduling barriers keep this
+  // order.  NI x NJ: the blocks per wave that hold part of the matrix (the same for the whole
+  // workgroup), the others' products are left out.
+  constexpr int NS = BK / 4;
+  auto main_loop = [&](auto ni_tag, auto nj_tag) {
+    constexpr int NI = decltype(ni_tag)::value, NJ = decltype(nj_tag)::value;
+    RC va[2][NI], vb[2][NJ];
+    auto frags = [&](int set, int buf, int ks) {
+      const RC* Sa = &As[buf][ks * 4][0];
+      const RC* Sb = &Bs[buf][ks * 4][0];
 #pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
+      for (int i = 0; i < NI; ++i) va[set][i] = Sa[fa0 ^ (swz<RC>(4 * ks) ^ (i * 32))];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) vb[set][j] = Sb[fb0 ^ (swz<RC>(4 * ks) ^ (j * 32))];
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto mfmas = [&](int set) {
       if constexpr (G3) {
-        R a_r[TM], a_i[TM], a_s[TM], b_r[TN], b_i[TN], b_s[TN];
-        const int kk = ks * 4 + lk;
+        R a_s[NI], b_s[NJ];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const RC v = As[cur][kk][(wm * (BM / 2) + i * 16 + lr) ^ swz<RC>(kk)];
-          a_r[i] = v.x;
-          a_i[i] = v.y;
-          a_s[i] = v.x + v.y;
-        }
+        for (int i = 0; i < NI; ++i) a_s[i] = CA ? va[set][i].x - va[set][i].y : va[set][i].x + va[set][i].y;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const RC v = Bs[cur][kk][(wn * (BN / 2) + j * 16 + lr) ^ swz<RC>(kk)];
-          b_r[j] = v.x;
-          b_i[j] = v.y;
-          b_s[j] = v.x + v.y;
-        }
+        for (int j = 0; j < NJ; ++j) b_s[j] = CB ? vb[set][j].x - vb[set][j].y : vb[set][j].x + vb[set][j].y;
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            cr[i][j] = AR::mfma(a_r[i], b_r[j], cr[i][j]);
-            ci[i][j] = AR::mfma(a_i[i], b_i[j], ci[i][j]);
+          for (int j = 0; j < NJ; ++j) {
+            cr[i][j] = AR::mfma(va[set][i].x, vb[set][j].x, cr[i][j]);
+            ci[i][j] = AR::mfma(va[set][i].y, vb[set][j].y, ci[i][j]);
             cs[i][j] = AR::mfma(a_s[i], b_s[j], cs[i][j]);
           }
-        continue;
-      }
-      R a_r[TM], a_i[TM], a_n[TM], b_r[TN], b_i[TN];
+      } else {
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int kk = ks * 4 + lk;
-        const RC v = As[cur][kk][(wm * (BM / 2) + i * 16 + lr) ^ swz<RC>(kk)];
-        a_r[i] = v.x;
-        a_i[i] = v.y;
-        a_n[i] = -v.y;
-      }
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int kk = ks * 4 + lk;
-        const RC v = Bs[cur][kk][(wn * (BN / 2) + j * 16 + lr) ^ swz<RC>(kk)];
-        b_r[j] = v.x;
-        b_i[j] = v.y;
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          cr[i][j] = AR::mfma(a_r[i], b_r[j], cr[i][j]);
-          ci[i][j] = AR::mfma(a_r[i], b_i[j], ci[i][j]);
-        }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          cr[i][j] = AR::mfma(a_n[i], b_i[j], cr[i][j]);
-          ci[i][j] = AR::mfma(a_i[i], b_r[j], ci[i][j]);
-        }
-    }
-    if constexpr (FOLD) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            if constexpr (G3) {
-              const R t1 = cr[i][j][v], t2 = ci[i][j][v];
-              fr[i][j][v] += static_cast<double>(t1 - t2);
-              fi[i][j][v] += static_cast<double>(cs[i][j][v] - t1 - t2);
-              cs[i][j][v] = 0;
-            } else {
-              fr[i][j][v] += static_cast<double>(cr[i][j][v]);
-              fi[i][j][v] += static_cast<double>(ci[i][j][v]);
-            }
-            cr[i][j][v] = 0;
-            ci[i][j][v] = 0;
+          for (int j = 0; j < NJ; ++j) {
+            cr[i][j] = AR::mfma(va[set][i].x, vb[set][j].x, cr[i][j]);
+            ci[i][j] = AR::template mfma<CB>(va[set][i].x, vb[set][j].y, ci[i][j]);
           }
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            cr[i][j] = AR::template mfma<CA == CB>(va[set][i].y, vb[set][j].y, cr[i][j]);
+            ci[i][j] = AR::template mfma<CA>(va[set][i].y, vb[set][j].x, ci[i][j]);
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // STEADY: chunks kt + 1 and kt + 2 exist and are full
+    auto chunk = [&](auto buf_tag, auto steady_tag, int kt) {
+      constexpr int BUF = decltype(buf_tag)::value;
+      constexpr bool STEADY = decltype(steady_tag)::value;
+#pragma unroll
+      for (int ks = 0; ks < NS; ++ks) {
+        if (ks + 1 < NS) {
+          frags((ks + 1) & 1, BUF, ks + 1);
+        } else if (STEADY || kt + 1 < nk) {
+          ia.store(&As[BUF ^ 1][0][0], ra);
+          ib.store(&Bs[BUF ^ 1][0][0], rb);
+          if constexpr (STEADY) fetch_full();
+          else if (kt + 2 < nk) fetch(kt + 2);
+          __syncthreads();
+          frags((ks + 1) & 1, BUF ^ 1, 0);
+        }
+        mfmas(ks & 1);
+      }
+      if constexpr (FOLD) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              if constexpr (G3) {
+                const R t1 = cr[i][j][v], t2 = CA != CB ? -ci[i][j][v] : ci[i][j][v];
+                fr[i][j][v] += static_cast<double>(t1 - t2);
+                fi[i][j][v] += static_cast<double>(cs[i][j][v] - t1 - t2);
+                cs[i][j][v] = 0;
+              } else {
+                fr[i][j][v] += static_cast<double>(cr[i][j][v]);
+                fi[i][j][v] += static_cast<double>(ci[i][j][v]);
+              }
+              cr[i][j][v] = 0;
+              ci[i][j][v] = 0;
+            }
+      }
+    };
+    const std::integral_constant<int, 0> buf0{};
+    const std::integral_constant<int, 1> buf1{};
+    int kt = kt0;
+    if (kt < nk) frags(0, 0, 0);
+    for (const int full = min(nk, p.K / BK); kt + 3 < full; kt += 2) {
+      chunk(buf0, std::true_type{}, kt);
+      chunk(buf1, std::true_type{}, kt + 1);
     }
-    if (kt + 1 < nk) {
-      IOA::store(As[cur ^ 1], ra);
-      IOB::store(Bs[cur ^ 1], rb);
+    for (; kt < nk; kt += 2) {
+      chunk(buf0, std::false_type{}, kt);
+      if (kt + 1 < nk) chunk(buf1, std::false_type{}, kt + 1);
     }
-    __syncthreads();
+  };
+  if (kt0 < nk) {
+    fetch(kt0);
+    ia.store(&As[0][0][0], ra);
+    ib.store(&Bs[0][0][0], rb);
+    if (kt0 + 1 < nk) fetch(kt0 + 1);
+  }
+  __syncthreads();
+  const std::integral_constant<int, TM> all_i{};
+  const std::integral_constant<int, TN> all_j{};
+  if constexpr (BM == 64 && BN == 64) {
+    const std::integral_constant<int, TM / 2> half_i{};
+    const std::integral_constant<int, TN / 2> half_j{};
+    if (p.M - m0 > BM / 2) {
+      if (p.N - n0 > BN / 2) main_loop(all_i, all_j);
+      else main_loop(all_i, half_j);
+    } else {
+      if (p.N - n0 > BN / 2) main_loop(half_i, all_j);
+      else main_loop(half_i, half_j);
+    }
+  } else {
+    main_loop(all_i, all_j);
   }
 
   if constexpr (G3 && !FOLD) {
@@ -333,7 +460,7 @@ void gemm_kernel(Args p) {
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const R t1 = cr[i][j][v], t2 = ci[i][j][v];
+          const R t1 = cr[i][j][v], t2 = CA != CB ? -ci[i][j][v] : ci[i][j][v];
           cr[i][j][v] = t1 - t2;
           ci[i][j][v] = cs[i][j][v] - t1 - t2;
         }
@@ -349,38 +476,62 @@ void gemm_kernel(Args p) {
     // element would be its own access: it goes through a wave-private 16 x 17 LDS block per
     // 16 x 16 accumulator block, so that its store and the read of H run along rows (the
     // N_mu = 1600 projections: 154.8 -> 140.1 ms per iteration).  The K loop's staging buffers
-    // are free here (its last barrier has passed): waves 0-1 use As, 2-3 Bs.
+    // are free once every wave has passed the barrier below: waves 0-1 use As, 2-3 Bs.
     using S = decltype(TC{}.x);
     const c128* Hb = p.H.p ? batch_ptr<c128>(p.H, b) : nullptr;
     if constexpr (sizeof(R) == 8) {
+      // Per 16 x 16 block all reads of H first, then the stores: one wait instead of one per
+      // element.  The reads are clamped into the matrix instead of predicated.
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j) {
+          c128 h[4], ht[4];
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
-            const int r = m0 + wm * (BM / 2) + i * 16 + AR::row(lk, v);
-            const int c = n0 + wn * (BN / 2) + j * 16 + lr;
-            if (r < p.M && c < p.N && r >= c) {
-              const double xr = cr[i][j][v], xi = ci[i][j][v];
-              const double outr = p.ar * xr - p.ai * xi, outi = p.ar * xi + p.ai * xr;
-              const c128 h = Hb ? Hb[static_cast<long>(r) * p.ldc + c] : c128{0.0, 0.0};
-              C[static_cast<long>(r) * p.ldc + c] = TC{static_cast<S>(outr - h.x), static_cast<S>(outi - h.y)};
-              if (r > c) {
-                const c128 ht = Hb ? Hb[static_cast<long>(c) * p.ldc + r] : c128{0.0, 0.0};
-                C[static_cast<long>(c) * p.ldc + r] = TC{static_cast<S>(outr - ht.x), static_cast<S>(-outi - ht.y)};
-              }
+            h[v] = ht[v] = c128{0.0, 0.0};
+            if (Hb) {
+              const int r = min(m0 + row0(i) + AR::row(lk, v), p.M - 1);
+              const int c = min(n0 + col0(j) + lr, p.N - 1);
+              h[v] = Hb[static_cast<long>(r) * p.ldc + c];
+              ht[v] = Hb[static_cast<long>(c) * p.ldc + r];
             }
           }
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int r = m0 + row0(i) + AR::row(lk, v);
+            const int c = n0 + col0(j) + lr;
+            const double xr = cr[i][j][v], xi = ci[i][j][v];
+            const double outr = p.ar * xr - p.ai * xi, outi = p.ar * xi + p.ai * xr;
+            if (r < p.M && c < p.N && r >= c)
+              C[static_cast<long>(r) * p.ldc + c] = TC{static_cast<S>(outr - h[v].x), static_cast<S>(outi - h[v].y)};
+            if (r < p.M && c < p.N && r > c)
+              C[static_cast<long>(c) * p.ldc + r] = TC{static_cast<S>(outr - ht[v].x), static_cast<S>(-outi - ht[v].y)};
+          }
+        }
       return;
     }
-    c128* T = reinterpret_cast<c128*>(wave < 2 ? static_cast<void*>(&As[0][0][0]) : static_cast<void*>(&Bs[0][0][0])) +
-              (wave & 1) * (16 * 17);
+    __syncthreads();
+    // With H the block is kept in double (H is subtracted there), else as stored.  Only the wave
+    // itself reads what it wrote, and a wave's LDS accesses are in order: no barrier.
+    using TT = typename std::conditional<sizeof(TC) == 16, c128, TC>::type;
+    using SS = decltype(TT{}.x);
+    TT* T = reinterpret_cast<TT*>(wave < 2 ? static_cast<void*>(&As[0][0][0]) : static_cast<void*>(&Bs[0][0][0])) +
+            (wave & 1) * (16 * 17);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const int R0 = m0 + wm * (BM / 2) + i * 16, C0 = n0 + wn * (BN / 2) + j * 16;
+        const int R0 = m0 + row0(i), C0 = n0 + col0(j);
+        c128 h[4], ht[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          h[v] = ht[v] = c128{0.0, 0.0};
+          if (Hb) {
+            h[v] = Hb[static_cast<long>(min(R0 + AR::row(lk, v), p.M - 1)) * p.ldc + min(C0 + lr, p.N - 1)];
+            ht[v] = Hb[static_cast<long>(min(C0 + lk + 4 * v, p.N - 1)) * p.ldc + min(R0 + lr, p.M - 1)];
+          }
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int rl = AR::row(lk, v), r = R0 + rl, c = C0 + lr;
@@ -390,60 +541,69 @@ void gemm_kernel(Args p) {
             xi += fi[i][j][v];
           }
           const double outr = p.ar * xr - p.ai * xi, outi = p.ar * xi + p.ai * xr;
-          if (r < p.M && c < p.N && r >= c) {
-            const c128 h = Hb ? Hb[static_cast<long>(r) * p.ldc + c] : c128{0.0, 0.0};
-            C[static_cast<long>(r) * p.ldc + c] = TC{static_cast<S>(outr - h.x), static_cast<S>(outi - h.y)};
-          }
-          T[lr * 17 + rl] = c128{outr, -outi};  // T[col][row] = conj(X[row][col])
+          if (r < p.M && c < p.N && r >= c)
+            C[static_cast<long>(r) * p.ldc + c] = TC{static_cast<S>(outr - h[v].x), static_cast<S>(outi - h[v].y)};
+          T[lr * 17 + rl] = TT{static_cast<SS>(outr), static_cast<SS>(-outi)};  // T[col][row] = conj(X[row][col])
         }
-        __syncthreads();
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int cl = lk + 4 * v;  // source column: destination row C0 + cl
           const int r = R0 + lr, c = C0 + cl;
+          const TT x = T[cl * 17 + lr];
           if (r < p.M && c < p.N && r > c) {
-            const c128 x = T[cl * 17 + lr];
-            const c128 ht = Hb ? Hb[static_cast<long>(c) * p.ldc + r] : c128{0.0, 0.0};
-            C[static_cast<long>(c) * p.ldc + r] = TC{static_cast<S>(x.x - ht.x), static_cast<S>(x.y - ht.y)};
+            if (sizeof(TC) == 16) C[static_cast<long>(c) * p.ldc + r] = TC{static_cast<S>(x.x - ht[v].x), static_cast<S>(x.y - ht[v].y)};
+            else C[static_cast<long>(c) * p.ldc + r] = TC{static_cast<S>(x.x), static_cast<S>(x.y)};
           }
         }
-        __syncthreads();
+        __builtin_amdgcn_wave_barrier();
       }
     return;
   }
+  // beta C: the old values of a 16-row block are read together (clamped into the matrix, not
+  // predicated) before any of them is used.  Read, waited for and stored one element at a
+  // time, a wave's 16 values cost 16 memory latencies, as long as the main loop of K = 64.
   const bool beta0 = (p.br == 0.0 && p.bi == 0.0);
   const bool gamma0 = (p.gr == 0.0 && p.gi == 0.0);
+  using S = decltype(TC{}.x);
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < TM; ++i) {
+    TC old[TN][4];
+    if (!beta0) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int r = min(m0 + row0(i) + AR::row(lk, v), p.M - 1);
+          const int c = min(n0 + col0(j) + lr, p.N - 1);
+          old[j][v] = C[static_cast<long>(r) * p.ldc + c];
+        }
+    }
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int r = m0 + wm * (BM / 2) + i * 16 + AR::row(lk, v);
-        const int c = n0 + wn * (BN / 2) + j * 16 + lr;
-        if (r < p.M && c < p.N) {
-          double xr = cr[i][j][v], xi = ci[i][j][v];
-          if constexpr (FOLD) {
-            xr += fr[i][j][v];
-            xi += fi[i][j][v];
-          }
-          double outr = p.ar * xr - p.ai * xi;
-          double outi = p.ar * xi + p.ai * xr;
-          TC* dst = C + static_cast<long>(r) * p.ldc + c;
-          using S = decltype(TC{}.x);
-          if (!beta0) {
-            const TC old = *dst;
-            const double o_r = old.x, o_i = old.y;
-            outr += p.br * o_r - p.bi * o_i;
-            outi += p.br * o_i + p.bi * o_r;
-          }
-          if (!gamma0 && r == c) {
-            outr += p.gr;
-            outi += p.gi;
-          }
-          *dst = TC{static_cast<S>(outr), static_cast<S>(outi)};
+        const int r = m0 + row0(i) + AR::row(lk, v);
+        const int c = n0 + col0(j) + lr;
+        double xr = cr[i][j][v], xi = ci[i][j][v];
+        if constexpr (FOLD) {
+          xr += fr[i][j][v];
+          xi += fi[i][j][v];
         }
+        double outr = p.ar * xr - p.ai * xi;
+        double outi = p.ar * xi + p.ai * xr;
+        if (!beta0) {
+          const double o_r = old[j][v].x, o_i = old[j][v].y;
+          outr += p.br * o_r - p.bi * o_i;
+          outi += p.br * o_i + p.bi * o_r;
+        }
+        if (!gamma0 && r == c) {
+          outr += p.gr;
+          outi += p.gi;
+        }
+        if (r < p.M && c < p.N) C[static_cast<long>(r) * p.ldc + c] = TC{static_cast<S>(outr), static_cast<S>(outi)};
       }
+  }
 }
 
 // ---------------------------------------------------------------------------------
@@ -738,13 +898,21 @@ hipEvent_t pool_event() {
 // read by the callers (the FP32 projections of G for Sigma, through GEMM_G3).
 std::atomic<int> g_complex3{0};
 
+// Tile grid of a product: one workgroup per tile, or per lower tile of a square lower product.
+// Returns the number of workgroups.
+long set_tiles(Args& a, int bm, int bn) {
+  a.tiles_m = (a.M + bm - 1) / bm;
+  a.tiles_n = (a.N + bn - 1) / bn;
+  a.packed = (a.tri & GEMM_TRI_LOWER) && bm == bn && a.tiles_m == a.tiles_n && !(a.tri & GEMM_SPLIT_BF16);
+  a.tiles = a.packed ? a.tiles_m * (a.tiles_m + 1) / 2 : a.tiles_m * a.tiles_n;
+  return static_cast<long>(a.batch) * a.tiles;
+}
+
 // Tile shapes: 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128 (complex<double> only).
 template <int OPA, int OPB>
 void launch(hipStream_t s, Args a, int shape) {
   const int bm = shape == 0 ? 64 : 128, bn = shape == 2 ? 128 : 64;
-  a.tiles_m = (a.M + bm - 1) / bm;
-  a.tiles_n = (a.N + bn - 1) / bn;
-  const long nblocks = static_cast<long>(a.batch) * a.tiles_m * a.tiles_n;
+  const long nblocks = set_tiles(a, bm, bn);
   THCGW_REQUIRE(nblocks < (1L << 31), "zgemm: grid too large");
   const dim3 g(static_cast<unsigned>(nblocks)), t(NT);
   if (shape == 0 && (g_complex3.load() & 1))
@@ -759,40 +927,29 @@ void launch(hipStream_t s, Args a, int shape) {
 
 std::atomic<int> g_tile_mode32{0};  // FP32 tile: 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128
 
-template <typename TA, typename TB, typename TC, int OPA, int OPB>
+// FOLD: the products the callers run with GEMM_FOLD64 (always or never, by operand types and
+// ops: see cgemm).
+template <typename TA, typename TB, typename TC, int OPA, int OPB, bool FOLD>
 void launch_f32(hipStream_t s, Args a) {
+  const bool bf = (a.tri & GEMM_SPLIT_BF16) != 0;
   const int tb = (a.tri >> GEMM_TILE32_SHIFT) & 3;
-  const int mode = ((a.tri & (GEMM_SPLIT_BF16 | GEMM_FOLD64)) == 0) ? (tb ? tb - 1 : g_tile_mode32.load()) : 0;
-  const int bm = mode == 0 ? 64 : 128, bn = mode == 2 ? 128 : 64;
-  a.tiles_m = (a.M + bm - 1) / bm;
-  a.tiles_n = (a.N + bn - 1) / bn;
-  const long nblocks = static_cast<long>(a.batch) * a.tiles_m * a.tiles_n;
+  const int mode = (!bf && !FOLD) ? (tb ? tb - 1 : g_tile_mode32.load()) : 0;
+  const long nblocks = set_tiles(a, mode == 0 ? 64 : 128, mode == 2 ? 128 : 64);
   THCGW_REQUIRE(nblocks < (1L << 31), "cgemm: grid too large");
-  if (mode == 1) {
-    hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 128, 64>), dim3(static_cast<unsigned>(nblocks)),
-                       dim3(NT), 0, s, a);
-  } else if (mode == 2) {
-    hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 128, 128>), dim3(static_cast<unsigned>(nblocks)),
-                       dim3(NT), 0, s, a);
-  } else if (a.tri & GEMM_SPLIT_BF16) {
-    if (a.tri & GEMM_FOLD64)
-      hipLaunchKernelGGL((gemm_bf16x6_kernel<TA, TB, TC, OPA, OPB, true>), dim3(static_cast<unsigned>(nblocks)),
-                         dim3(NT), 0, s, a);
+  const dim3 g(static_cast<unsigned>(nblocks)), t(NT);
+  const bool g3 = (g_complex3.load() & (FOLD ? 4 : 2)) || (a.tri & GEMM_G3);
+  if (bf)
+    hipLaunchKernelGGL((gemm_bf16x6_kernel<TA, TB, TC, OPA, OPB, FOLD>), g, t, 0, s, a);
+  else if (mode == 0 && g3)
+    hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 64, 64, FOLD, true>), g, t, 0, s, a);
+  else if (mode == 0)
+    hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 64, 64, FOLD>), g, t, 0, s, a);
+  else if constexpr (!FOLD) {
+    if (mode == 1)
+      hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 128, 64>), g, t, 0, s, a);
     else
-      hipLaunchKernelGGL((gemm_bf16x6_kernel<TA, TB, TC, OPA, OPB, false>), dim3(static_cast<unsigned>(nblocks)),
-                         dim3(NT), 0, s, a);
-  } else if ((a.tri & GEMM_FOLD64) && ((g_complex3.load() & 4) || (a.tri & GEMM_G3)))
-    hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 64, 64, true, true>),
-                       dim3(static_cast<unsigned>(nblocks)), dim3(NT), 0, s, a);
-  else if (a.tri & GEMM_FOLD64)
-    hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 64, 64, true>), dim3(static_cast<unsigned>(nblocks)),
-                       dim3(NT), 0, s, a);
-  else if ((g_complex3.load() & 2) || (a.tri & GEMM_G3))
-    hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 64, 64, false, true>),
-                       dim3(static_cast<unsigned>(nblocks)), dim3(NT), 0, s, a);
-  else
-    hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 64, 64>), dim3(static_cast<unsigned>(nblocks)),
-                       dim3(NT), 0, s, a);
+      hipLaunchKernelGGL((gemm_kernel<float, TA, TB, TC, OPA, OPB, 128, 128>), g, t, 0, s, a);
+  }
 }
 
 std::atomic<int> g_tile_mode{0};  // 0 = automatic, else shape + 1
@@ -809,11 +966,13 @@ int tile_shape(int, int, int) {
 namespace {
 
 Args make_args(int M, int N, int K, Cplx alpha, BatchPtr A, long lda, BatchPtr B, long ldb, Cplx beta, void* C,
-               long strideC, long ldc, int batch, Cplx gamma, int tri, BatchPtr hsub) {
+               long strideC, long ldc, int batch, Cplx gamma, int tri, BatchPtr hsub, bool a_rows, bool b_rows) {
   THCGW_REQUIRE(!(tri & GEMM_HERM_SUB) || (M == N && beta.re == 0.0 && beta.im == 0.0 &&
                                            gamma.re == 0.0 && gamma.im == 0.0 && (tri & GEMM_TRI_LOWER) &&
                                            !(tri & GEMM_SPLIT_BF16)),
                 "gemm: GEMM_HERM_SUB needs a square lower product without beta, gamma or split BF16");
+  // a tile's rows are addressed by 32-bit offsets where K is contiguous (TileIO)
+  THCGW_REQUIRE((!a_rows || lda < (1L << 21)) && (!b_rows || ldb < (1L << 21)), "gemm: leading dimension too large");
   Args a;
   a.H = hsub;
   a.M = M;
@@ -881,44 +1040,22 @@ void timed(hipStream_t s, double flops, double bytes, int cls, F&& launch_fn) {
   g_flops_milli.fetch_add(static_cast<long long>(flops / 1000.0));
 }
 
-template <typename TA, typename TB, typename TC>
-void dispatch_f32_ops(hipStream_t s, int opA, int opB, const Args& a) {
-  if (opA == OP_N && opB == OP_N) launch_f32<TA, TB, TC, OP_N, OP_N>(s, a);
-  else if (opA == OP_N && opB == OP_C) launch_f32<TA, TB, TC, OP_N, OP_C>(s, a);
-  else if (opA == OP_C && opB == OP_N) launch_f32<TA, TB, TC, OP_C, OP_N>(s, a);
-  else if (opA == OP_C && opB == OP_C) launch_f32<TA, TB, TC, OP_C, OP_C>(s, a);
-  else throw Error(THCGW_ERR_UNSUPPORTED, "cgemm: transpose without conjugation is not built");
-}
-
-template <typename TA, typename TB>
-void dispatch_f32_c(hipStream_t s, int opA, int opB, Dt tc, const Args& a) {
-  if (tc == DT_C128) dispatch_f32_ops<TA, TB, c128>(s, opA, opB, a);
-  else dispatch_f32_ops<TA, TB, c64>(s, opA, opB, a);
-}
-
 }  // namespace
 
 void zgemm(hipStream_t s, int opA, int opB, int M, int N, int K, Cplx alpha, BatchPtr A, long lda,
            BatchPtr B, long ldb, Cplx beta, c128* C, long strideC, long ldc, int batch, Cplx gamma, int tri,
            BatchPtr hsub) {
   THCGW_REQUIRE(M >= 0 && N >= 0 && K >= 0 && batch >= 0, "zgemm: negative size");
-  THCGW_REQUIRE(opA >= 0 && opA <= 2 && opB >= 0 && opB <= 2, "zgemm: bad op");
+  THCGW_REQUIRE((opA == OP_N && (opB == OP_N || opB == OP_C)) || (opA == OP_C && opB == OP_N), "zgemm: ops not built");
   if (M == 0 || N == 0 || batch == 0) return;
-  const Args a = make_args(M, N, K, alpha, A, lda, B, ldb, beta, C, strideC, ldc, batch, gamma, tri, hsub);
+  const Args a = make_args(M, N, K, alpha, A, lda, B, ldb, beta, C, strideC, ldc, batch, gamma, tri, hsub, opA == OP_N,
+                           opB != OP_N);
   const int nb = tile_shape(M, N, K);
   const bool bnz = beta.re != 0.0 || beta.im != 0.0;
   timed(s, model_flops(M, N, K, batch, tri), model_bytes(M, N, K, batch, tri, bnz, 16, 16, 16), opA * 3 + opB, [&] {
-    switch (opA * 3 + opB) {
-      case 0: launch<OP_N, OP_N>(s, a, nb); break;
-      case 1: launch<OP_N, OP_T>(s, a, nb); break;
-      case 2: launch<OP_N, OP_C>(s, a, nb); break;
-      case 3: launch<OP_T, OP_N>(s, a, nb); break;
-      case 4: launch<OP_T, OP_T>(s, a, nb); break;
-      case 5: launch<OP_T, OP_C>(s, a, nb); break;
-      case 6: launch<OP_C, OP_N>(s, a, nb); break;
-      case 7: launch<OP_C, OP_T>(s, a, nb); break;
-      default: launch<OP_C, OP_C>(s, a, nb); break;
-    }
+    if (opA == OP_N && opB == OP_N) launch<OP_N, OP_N>(s, a, nb);
+    else if (opA == OP_N) launch<OP_N, OP_C>(s, a, nb);
+    else launch<OP_C, OP_N>(s, a, nb);
   });
 }
 
@@ -929,15 +1066,24 @@ void cgemm(hipStream_t s, int opA, int opB, int M, int N, int K, Cplx alpha, Bat
   if (M == 0 || N == 0 || batch == 0) return;
   THCGW_REQUIRE(!(tri & GEMM_HERM_SUB) || tc == DT_C128 || !hsub.p,
                 "cgemm: GEMM_HERM_SUB with a subtracted matrix writes complex<double>");
-  const Args a = make_args(M, N, K, alpha, A, lda, B, ldb, beta, C, strideC, ldc, batch, gamma, tri, hsub);
+  const Args a = make_args(M, N, K, alpha, A, lda, B, ldb, beta, C, strideC, ldc, batch, gamma, tri, hsub, opA == OP_N,
+                           opB != OP_N);
   const int cls = ((tri & GEMM_SPLIT_BF16) ? 13 : 9) + (opA == OP_C ? 2 : 0) + (opB == OP_C ? 1 : 0);
   const bool bnz = beta.re != 0.0 || beta.im != 0.0;
   const int ea = ta == DT_C128 ? 16 : 8, eb = tb == DT_C128 ? 16 : 8, ec = tc == DT_C128 ? 16 : 8;
   timed(s, model_flops(M, N, K, batch, tri), model_bytes(M, N, K, batch, tri, bnz, ea, eb, ec), cls, [&] {
-    if (ta == DT_C128 && tb == DT_C128) dispatch_f32_c<c128, c128>(s, opA, opB, tc, a);
-    else if (ta == DT_C128) dispatch_f32_c<c128, c64>(s, opA, opB, tc, a);
-    else if (tb == DT_C128) dispatch_f32_c<c64, c128>(s, opA, opB, tc, a);
-    else dispatch_f32_c<c64, c64>(s, opA, opB, tc, a);
+    // the products of the mixed-precision forms, and only those, are built
+    const bool c64s = ta == DT_C64 && tb == DT_C64, fold = (tri & GEMM_FOLD64) != 0;
+    const bool nn = opA == OP_N && opB == OP_N, nc = opA == OP_N && opB == OP_C, cn = opA == OP_C && opB == OP_N;
+    if (nn && !fold && ta == DT_C64 && tb == DT_C128 && tc == DT_C64)
+      launch_f32<c64, c128, c64, OP_N, OP_N, false>(s, a);
+    else if (nc && !fold && c64s && tc == DT_C64) launch_f32<c64, c64, c64, OP_N, OP_C, false>(s, a);
+    else if (nc && !fold && c64s) launch_f32<c64, c64, c128, OP_N, OP_C, false>(s, a);
+    else if (nn && fold && c64s && tc == DT_C64) launch_f32<c64, c64, c64, OP_N, OP_N, true>(s, a);
+    else if (nn && fold && c64s) launch_f32<c64, c64, c128, OP_N, OP_N, true>(s, a);
+    else if (cn && fold && c64s && tc == DT_C64) launch_f32<c64, c64, c64, OP_C, OP_N, true>(s, a);
+    else if (cn && fold && c64s) launch_f32<c64, c64, c128, OP_C, OP_N, true>(s, a);
+    else throw Error(THCGW_ERR_UNSUPPORTED, "cgemm: this combination of ops, types and folding is not built");
   });
 }
 
