@@ -1379,24 +1379,7 @@ c128* sigma_to_w(thcgw_ctx* ctx, const c128* Sigma, hipStream_t s) {
   return Sw;
 }
 
-// Out[n,k] = [(iw_n + mu) S - H0 - F - Sw]^-1 Rhs, Rhs = S_k (with_s) or I, for all (n, k) by
-// batched LU (A = Lt Ut Pt), two triangular solves and the row gather that undoes the swaps.
-void matsubara_solve(thcgw_ctx* ctx, const c128* H0, const c128* F, const c128* S, const c128* Sw, double mu,
-                     bool rhs_s, c128* Out, hipStream_t s) {
-  const int nw = ctx->d.nw_f, nk = ctx->nk, no = ctx->d.no;
-  const long m = static_cast<long>(no) * no;
-  const long count = static_cast<long>(nw) * nk;
-  THCGW_REQUIRE(count < (1L << 30), "Dyson for G: too many matrices");
-  c128* X = ctx->buf<c128>("dg_x", static_cast<size_t>(count) * m);
-  c128* Y = ctx->buf<c128>("dg_y", static_cast<size_t>(count) * m);
-  int* ipiv = ctx->buf<int>("dg_ipiv", static_cast<size_t>(count) * no);
-  int* info = ctx->buf<int>("dg_info", static_cast<size_t>(count));
-  thcgw::matsubara_dyson(s, H0, F, S, Sw, ctx->d_wn_f, ctx->d.beta, mu, nw, nk, no, X);
-  thcgw::getrf_batched(s, X, m, no, no, ipiv, info, static_cast<int>(count));
-  thcgw::rhs_batch(s, rhs_s ? S : nullptr, nk, no, count, Y);
-  thcgw::trsm_left_lower(s, X, m, no, Y, m, no, no, no, static_cast<int>(count));
-  thcgw::trsm_left_upper_unit(s, X, m, no, Y, m, no, no, no, static_cast<int>(count));
-  thcgw::dyson_finish(s, Y, m, nullptr, 0, 1, ipiv, no, Out, m, 0, static_cast<int>(count));
+void check_matsubara_info(const int* info, long count, int nk, hipStream_t s) {
   std::vector<int> h(count);
   THCGW_HIP(hipMemcpyAsync(h.data(), info, sizeof(int) * count, hipMemcpyDeviceToHost, s));
   THCGW_HIP(hipStreamSynchronize(s));
@@ -1406,18 +1389,44 @@ void matsubara_solve(thcgw_ctx* ctx, const c128* H0, const c128* F, const c128* 
                                                  std::to_string(b / nk) + ", " + std::to_string(b % nk) + ")");
 }
 
+// X^-1 of X[n,k] = (iw_n + mu) S - H0 - F - Sw for all (n, k) into Out, or with tr only
+// Tr[X^-1 S_k].  Up to order 128 one kernel forms and inverts each matrix in registers (matsubara.hip);
+// beyond, batched LU (A = Lt Ut Pt), two triangular solves with the right-hand side I (S_k
+// for the traces) and the row gather that undoes the swaps.
+void matsubara_solve(thcgw_ctx* ctx, const c128* H0, const c128* F, const c128* S, const c128* Sw, double mu,
+                     c128* Out, c128* tr, hipStream_t s) {
+  const int nw = ctx->d.nw_f, nk = ctx->nk, no = ctx->d.no;
+  const long m = static_cast<long>(no) * no;
+  const long count = static_cast<long>(nw) * nk;
+  THCGW_REQUIRE(count < (1L << 30), "Dyson for G: too many matrices");
+  int* info = ctx->buf<int>("dg_info", static_cast<size_t>(count));
+  if (thcgw::matsubara_inverse_fits(no)) {
+    thcgw::matsubara_inverse(s, H0, F, S, Sw, ctx->d_wn_f, ctx->d.beta, mu, nw, nk, no, tr ? nullptr : Out, tr, info);
+    return check_matsubara_info(info, count, nk, s);
+  }
+  c128* X = ctx->buf<c128>("dg_x", static_cast<size_t>(count) * m);
+  c128* Y = ctx->buf<c128>("dg_y", static_cast<size_t>(count) * m);
+  if (!Out) Out = ctx->buf<c128>("dg_r", static_cast<size_t>(count) * m);
+  int* ipiv = ctx->buf<int>("dg_ipiv", static_cast<size_t>(count) * no);
+  thcgw::matsubara_dyson(s, H0, F, S, Sw, ctx->d_wn_f, ctx->d.beta, mu, nw, nk, no, X);
+  thcgw::getrf_batched(s, X, m, no, no, ipiv, info, static_cast<int>(count));
+  thcgw::rhs_batch(s, tr ? S : nullptr, nk, no, count, Y);
+  thcgw::trsm_left_lower(s, X, m, no, Y, m, no, no, no, static_cast<int>(count));
+  thcgw::trsm_left_upper_unit(s, X, m, no, Y, m, no, no, no, static_cast<int>(count));
+  thcgw::dyson_finish(s, Y, m, nullptr, 0, 1, ipiv, no, Out, m, 0, static_cast<int>(count));
+  check_matsubara_info(info, count, nk, s);
+  if (tr) thcgw::batched_trace(s, Out, m, no, tr, static_cast<int>(count));
+}
+
 // Electron number at mu (compute_Nelec, scf_common.cpp:10-42) with the spectral sum of
 // compute_eigenspectra (simple_dyson.cpp:130-172) taken as the resolvent trace
 // sum_b 1/(iw_n + mu - lambda_b) = Tr[((iw_n + mu) S - H0 - F - Sigma)^-1 S].
 double nelec_at(thcgw_ctx* ctx, const c128* H0, const c128* F, const c128* S, const c128* Sw, double mu,
                 hipStream_t s) {
-  const int nw = ctx->d.nw_f, nk = ctx->nk, no = ctx->d.no, nt = ctx->d.nt;
-  const long m = static_cast<long>(no) * no;
+  const int nw = ctx->d.nw_f, nk = ctx->nk, nt = ctx->d.nt;
   const long count = static_cast<long>(nw) * nk;
-  c128* R = ctx->buf<c128>("dg_r", static_cast<size_t>(count) * m);
   c128* tr = ctx->buf<c128>("dg_tr", static_cast<size_t>(count));
-  matsubara_solve(ctx, H0, F, S, Sw, mu, true, R, s);
-  thcgw::batched_trace(s, R, m, no, tr, static_cast<int>(count));
+  matsubara_solve(ctx, H0, F, S, Sw, mu, nullptr, tr, s);
   std::vector<std::complex<double>> h(count);
   THCGW_HIP(hipMemcpyAsync(h.data(), tr, sizeof(c128) * count, hipMemcpyDeviceToHost, s));
   THCGW_HIP(hipStreamSynchronize(s));
@@ -2051,7 +2060,7 @@ int thcgw_dyson_g(thcgw_ctx* ctx, const double* H0, const double* F, const doubl
     const long dim = static_cast<long>(ctx->nk) * ctx->d.no * ctx->d.no;
     c128* Sw = sigma_to_w(ctx, C(Sigma), s);
     c128* Gw = ctx->buf<c128>("dg_r", static_cast<size_t>(nw) * dim);
-    matsubara_solve(ctx, C(H0), C(F), C(Sov), Sw, mu, false, Gw, s);  // simple_dyson.cpp:65-78
+    matsubara_solve(ctx, C(H0), C(F), C(Sov), Sw, mu, Gw, nullptr, s);  // simple_dyson.cpp:65-78
     // G(tau) = w_to_tau(G(iw), fermi)  (simple_dyson.cpp:97-98)
     thcgw::zgemm(s, thcgw::OP_N, thcgw::OP_N, nt, static_cast<int>(dim), nw, kOne, thcgw::bp(ctx->d_Ttw_ff, 0), nw,
                  thcgw::bp(Gw, 0), dim, kZero, Cm(G), 0, dim, 1);

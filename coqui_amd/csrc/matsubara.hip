@@ -1,0 +1,278 @@
+// Inverses of the Matsubara matrices X(n, k) = (iw_n + mu) S_k - H0_k - F_k - Sigma(iw_n, k) of
+// order <= 128, one workgroup per matrix, or only the traces Tr[X^-1 S_k] that the electron
+// number needs (simple_dyson.cpp:65-78,130-172).
+//
+// The matrix is formed in registers and inverted there in place by Gauss-Jordan elimination
+// with partial pivoting: thread (r, c) of T x T holds the E x E elements (r + a T, c + b T).
+// Per column: its values and one pivot candidate per wave (published at the end of the
+// step before) are in LDS; barrier; every thread takes the same maximum; the pivot row's
+// owners scale it by the pivot and publish it; barrier; rank-1 update.  Rows are not
+// exchanged: the pivot row of column k stays where it is (row p_k), and X^-1[k][p_j] = B[p_k][j]
+// at the end.  A candidate is |Re| + |Im| with its row number in the lowest 7 of the 52
+// mantissa bits, so that one floating-point maximum yields both (lowest row on ties).
+// The division of a pivot row by its pivot is put off to the end: row p_k is scale[p_k] times
+// the stored row, whose own later updates need just its stored column values, and the identity's
+// element (p_k, k) is added there too.  So no register row is picked for writing in a column step.
+//
+// What bounds it: FP64 vector arithmetic (8 n^3 flops per matrix) and two barriers per column.
+// Memory traffic is one read of Sigma(iw) and one write of the inverse.  T = 16 with E = n / 16
+// rounded up wastes little padding and leaves 2-8 workgroups per CU to hide the barriers; up to
+// E = 6 (n <= 96) the elements fit the registers (E = 7 spills 90 of them in every column step),
+// and n <= 128 takes T = 32, E = 4.
+// N(mu) over N_k = 64 and 80 frequencies (5120 inverses with the transform and the transfer of the
+// traces), batched LU with triangular solves and a row gather through memory -> this kernel:
+// order 16 1.34 -> 0.22 ms, 26 2.18 -> 0.33, 52 5.17 -> 1.00, 78 9.83 -> 2.12, 96 13.2 -> 2.99,
+// 104 15.5 -> 5.6, 128 20.7 -> 7.2.  At order 78 the inversion takes 1.26 ms, 15 TFLOP/s of
+// vector arithmetic: two workgroups per CU (200 registers) hide half of the column step's
+// chain of barrier, maximum, reciprocal, barrier; a budget of three workgroups spills (1.65 ms).
+#include "thcgw_internal.hpp"
+
+#include <cfloat>
+#include <type_traits>
+#include <utility>
+
+namespace thcgw {
+namespace {
+
+__device__ __forceinline__ c128 cmul(c128 a, c128 b) { return c128{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
+
+// max(x, x of the lane D away): rows of 16 or halves of 32 lanes exchanged in the vector unit
+// (a shuffle through LDS would add two of its latencies to every column step)
+template <int D>
+__device__ __forceinline__ double swap_max(double x) {
+  const unsigned lo = static_cast<unsigned>(__double2loint(x)), hi = static_cast<unsigned>(__double2hiint(x));
+  const auto l = D == 16 ? __builtin_amdgcn_permlane16_swap(lo, lo, false, false)
+                         : __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto h = D == 16 ? __builtin_amdgcn_permlane16_swap(hi, hi, false, false)
+                         : __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return fmax(__hiloint2double(static_cast<int>(h[0]), static_cast<int>(l[0])),
+              __hiloint2double(static_cast<int>(h[1]), static_cast<int>(l[1])));
+}
+
+// f(0), ..., f(E - 1) with compile-time arguments, for work on the one register row that is picked at
+// run time.  The empty statement at the end of each such branch differs from branch to branch and so
+// keeps the compiler from merging them into one indexed access, which would move the array to memory.
+template <class F, int... A>
+__device__ __forceinline__ void each(F&& f, std::integer_sequence<int, A...>) {
+  (f(std::integral_constant<int, A>{}), ...);
+}
+
+template <int T, int E, bool TRACE>
+__global__ __launch_bounds__(T* T) __attribute__((amdgpu_waves_per_eu(T == 32 ? 4 : E <= 4 ? 4 : 2)))
+void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn, double beta,
+                              double mu, int nk, int n, c128* Out, c128* tr_out, int* info) {
+  constexpr int N = T * E;
+  __shared__ c128 colv[2][N], rowv[N], scale[N];
+  __shared__ double key[2][T * T / 64];
+  __shared__ int perm[N], rowpos[N];
+  __shared__ double red[2][T * T / 64];
+  __shared__ int bad;  // first zero or non-finite pivot column + 1
+  const long b = blockIdx.x, m = static_cast<long>(n) * n;
+  const long kofs = (b % nk) * m;
+  const int r = threadIdx.x / T, c = threadIdx.x % T;
+
+  c128 v[E][E];
+  {
+    const double wi = static_cast<double>(wn[b / nk]) * M_PI / beta;
+#pragma unroll
+    for (int a = 0; a < E; ++a)
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const int i = r + a * T, j = c + q * T;
+        v[a][q] = c128{0.0, 0.0};
+        if (i < n && j < n) {
+          const long e = static_cast<long>(i) * n + j;
+          const c128 sij = S ? S[kofs + e] : c128{i == j ? 1.0 : 0.0, 0.0};
+          const c128 h = H0 ? H0[kofs + e] : c128{0.0, 0.0};
+          const c128 f = F[kofs + e], sw = Sw[b * m + e];
+          v[a][q] = c128{mu * sij.x - wi * sij.y - h.x - f.x - sw.x, mu * sij.y + wi * sij.x - h.y - f.y - sw.y};
+        }
+      }
+  }
+  unsigned used = 0;  // bit a: row r + a T was a pivot row or lies outside the matrix
+#pragma unroll
+  for (int a = 0; a < E; ++a) used |= static_cast<unsigned>(r + a * T >= n) << a;
+
+  // Column values of element block q of thread column cc to LDS, which leaves zeros (the column
+  // of the identity), and the largest candidate of the wave's rows.
+  auto publish = [&](auto q_tag, int cc, int buf) __attribute__((always_inline)) {
+    constexpr int q = decltype(q_tag)::value;
+    double best = -1.0;
+#pragma unroll
+    for (int a = 0; a < E; ++a) {
+      // fmin: a NaN or an infinity becomes a pivot by its place and is found by its value then
+      const double mag = fmin(fabs(v[a][q].x) + fabs(v[a][q].y), DBL_MAX);
+      const unsigned off = (used << (31 - a)) & 0x80000000u;  // negative: loses every maximum
+      const unsigned lo = (static_cast<unsigned>(__double2loint(mag)) & ~127u) | static_cast<unsigned>(127 - (r + a * T));
+      best = fmax(best, __hiloint2double(static_cast<int>(static_cast<unsigned>(__double2hiint(mag)) | off),
+                                         static_cast<int>(lo)));
+    }
+    if (T == 16) best = swap_max<16>(best);  // four thread rows per wave, at lanes c, c + 16, c + 32, c + 48
+    best = swap_max<32>(best);
+    if (c == cc) {
+#pragma unroll
+      for (int a = 0; a < E; ++a) {
+        colv[buf][r + a * T] = v[a][q];
+        v[a][q] = c128{0.0, 0.0};
+      }
+      if (r % (64 / T) == 0) key[buf][threadIdx.x >> 6] = best;
+    }
+  };
+
+  if (threadIdx.x == 0) bad = 0;
+  publish(std::integral_constant<int, 0>{}, 0, 0);
+  auto column = [&](auto q_tag, int kk) __attribute__((always_inline)) {  // column k = q T + kk
+    constexpr int q = decltype(q_tag)::value;
+    const int k = q * T + kk, buf = k & 1;
+    __syncthreads();
+    double best = key[buf][0];
+#pragma unroll
+    for (int t = 1; t < T * T / 64; ++t) best = fmax(best, key[buf][t]);
+    const int p = __builtin_amdgcn_readfirstlane(127 - (__double2loint(best) & 127));
+    const int pr = p % T, pa = p / T;
+    if (r == pr) {  // the pivot row's owners (one wave) publish w = row / pivot
+      const c128 piv = colv[buf][p];
+      const double den = 1.0 / (piv.x * piv.x + piv.y * piv.y);
+      const c128 s{piv.x * den, -piv.y * den};
+      used |= 1u << pa;
+      each([&](auto a) __attribute__((always_inline)) {
+        if (a == pa) {
+#pragma unroll
+          for (int j = 0; j < E; ++j) rowv[c + j * T] = (j == q && c == kk) ? s : cmul(v[a][j], s);
+          asm volatile("; row block %0" ::"n"(decltype(a)::value));
+        }
+      }, std::make_integer_sequence<int, E>{});
+      if (c == 0) {
+        colv[buf][p] = c128{0.0, 0.0};  // the stored row stays as it is
+        scale[p] = s;
+        const bool ok = isfinite(piv.x) && isfinite(piv.y) && (piv.x != 0.0 || piv.y != 0.0);
+        if (!ok && bad == 0) bad = k + 1;
+        perm[k] = p;
+        rowpos[p] = k;
+      }
+    }
+    __syncthreads();
+    c128 w[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) w[j] = rowv[c + j * T];
+#pragma unroll
+    for (int a = 0; a < E; ++a) {
+      asm volatile("" ::: "memory");  // one row's factor at a time in registers
+      const c128 f = colv[buf][r + a * T];
+#pragma unroll
+      for (int j = 0; j < E; ++j) {
+        v[a][j].x = fma(f.y, w[j].y, fma(-f.x, w[j].x, v[a][j].x));
+        v[a][j].y = fma(-f.y, w[j].x, fma(-f.x, w[j].y, v[a][j].y));
+      }
+    }
+    if (kk + 1 < T) publish(q_tag, kk + 1, buf ^ 1);
+    else if constexpr (q + 1 < E) publish(std::integral_constant<int, q + 1>{}, 0, buf ^ 1);
+  };
+  auto columns = [&](auto q_tag) __attribute__((always_inline)) {
+    for (int kk = 0; kk < T && decltype(q_tag)::value * T + kk < n; ++kk) column(q_tag, kk);
+  };
+  columns(std::integral_constant<int, 0>{});
+  if constexpr (E > 1) columns(std::integral_constant<int, 1>{});
+  if constexpr (E > 2) columns(std::integral_constant<int, 2>{});
+  if constexpr (E > 3) columns(std::integral_constant<int, 3>{});
+  if constexpr (E > 4) columns(std::integral_constant<int, 4>{});
+  if constexpr (E > 5) columns(std::integral_constant<int, 5>{});
+  __syncthreads();
+  if (threadIdx.x == 0) info[b] = bad;
+  // the scaled rows, with the ones left out so far
+#pragma unroll
+  for (int a = 0; a < E; ++a) {
+    const int i = r + a * T;
+    if (i < n) {
+      const c128 s = scale[i];
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const int j = c + q * T;
+        if (j < n) v[a][q] = cmul(c128{v[a][q].x + (perm[j] == i ? 1.0 : 0.0), v[a][q].y}, s);
+      }
+    }
+  }
+
+  if constexpr (TRACE) {  // Tr[X^-1 S] = sum over this matrix of X^-1[k][p_j] S[p_j][k]
+    double re = 0.0, im = 0.0;
+#pragma unroll
+    for (int a = 0; a < E; ++a)
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const int i = r + a * T, j = c + q * T;
+        if (i < n && j < n) {
+          const int row = rowpos[i], col = perm[j];
+          if (S) {
+            const c128 t = cmul(v[a][q], S[kofs + static_cast<long>(col) * n + row]);
+            re += t.x;
+            im += t.y;
+          } else if (row == col) {
+            re += v[a][q].x;
+            im += v[a][q].y;
+          }
+        }
+      }
+    for (int o = 32; o >= 1; o >>= 1) {
+      re += __shfl_xor(re, o);
+      im += __shfl_xor(im, o);
+    }
+    if ((threadIdx.x & 63) == 0) {
+      red[0][threadIdx.x >> 6] = re;
+      red[1][threadIdx.x >> 6] = im;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int q = 1; q < T * T / 64; ++q) {
+        re += red[0][q];
+        im += red[1][q];
+      }
+      tr_out[b] = c128{re, im};
+    }
+  } else {
+    c128* Ob = Out + b * m;
+#pragma unroll
+    for (int a = 0; a < E; ++a)
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const int i = r + a * T, j = c + q * T;
+        if (i < n && j < n) Ob[static_cast<long>(rowpos[i]) * n + perm[j]] = v[a][q];
+      }
+  }
+}
+
+template <int T, int E>
+void launch_inverse(hipStream_t s, const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn,
+                    double beta, double mu, int nk, int n, int count, c128* Out, c128* tr, int* info) {
+  if (tr)
+    hipLaunchKernelGGL((matsubara_inverse_kernel<T, E, true>), dim3(count), dim3(T * T), 0, s, H0, F, S, Sw, wn, beta, mu,
+                       nk, n, Out, tr, info);
+  else
+    hipLaunchKernelGGL((matsubara_inverse_kernel<T, E, false>), dim3(count), dim3(T * T), 0, s, H0, F, S, Sw, wn, beta,
+                       mu, nk, n, Out, tr, info);
+  THCGW_HIP(hipGetLastError());
+}
+
+}  // namespace
+
+bool matsubara_inverse_fits(int no) { return no >= 1 && no <= 128; }
+
+void matsubara_inverse(hipStream_t s, const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn,
+                       double beta, double mu, int nw, int nk, int no, c128* Out, c128* tr, int* info) {
+  THCGW_REQUIRE(matsubara_inverse_fits(no), "matsubara_inverse: order must be in [1, 128]");
+  THCGW_REQUIRE((Out != nullptr) != (tr != nullptr), "matsubara_inverse: either the inverses or the traces");
+  const long count = static_cast<long>(nw) * nk;
+  THCGW_REQUIRE(count < (1L << 30), "Dyson for G: too many matrices");
+  if (count == 0) return;
+  const int nb = static_cast<int>(count);
+  switch ((no + 15) / 16) {
+    case 1: launch_inverse<16, 1>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
+    case 2: launch_inverse<16, 2>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
+    case 3: launch_inverse<16, 3>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
+    case 4: launch_inverse<16, 4>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
+    case 5: launch_inverse<16, 5>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
+    case 6: launch_inverse<16, 6>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
+    default: launch_inverse<32, 4>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
+  }
+}
+
+}  // namespace thcgw

@@ -189,6 +189,13 @@ bool ir_transform_fits(int R, int I);
 void ir_transform(hipStream_t s, const c128* T, int R, int I, const c128* in, long ld_in, long bs_in, c128* out,
                   long ld_out, long bs_out, long cols, int batch, bool real_t = false);
 
+// matsubara.hip: Out[n, k] = [(iw_n + mu) S_k - H0_k - F_k - Sw[n, k]]^-1 or tr[n, k] = Tr of that
+// inverse times S_k (exactly one of Out and tr; S and H0 nullable) for orders up to 128;
+// info[n nk + k] = first zero or non-finite pivot column + 1, or 0
+bool matsubara_inverse_fits(int no);
+void matsubara_inverse(hipStream_t s, const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn,
+                       double beta, double mu, int nw, int nk, int no, c128* Out, c128* tr, int* info);
+
 // misc.hip
 void scale_mo(hipStream_t s, const c128* C, const double* E, const double* tau, double mu, double beta, int nt, int nk,
               int no, c128* CG);
