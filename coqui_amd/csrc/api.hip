@@ -264,18 +264,27 @@ size_t free_device_bytes() {
   return fr;
 }
 
+// What a projection of Hermitian matrices forms: the whole product, its lower tiles mirrored to the
+// upper half, or its lower tiles only (for readers of the lower triangle; the rest of O_out
+// keeps what it held).  Sigma's k-grid transform reads the lower triangle only, and the
+// projections are bound by their stores (K = N_orb): without the mirrored ones Sigma at N_k = 64,
+// N_mu = 405, N_orb = 52 and 60 tau points takes 11.7 ms instead of 12.8, the mixed iteration at
+// N_mu = 480 61.7 instead of 62.7.
+enum Proj { PROJ_FULL, PROJ_MIRROR, PROJ_LOWER };
+int proj_flags(Proj p) {
+  return p == PROJ_FULL ? 0 : p == PROJ_MIRROR ? (thcgw::GEMM_TRI_LOWER | thcgw::GEMM_HERM_SUB) : thcgw::GEMM_TRI_LOWER;
+}
+
 // O_out[b,k] = X_k O_in[b,k] X_k^H for nbk = nb*nk matrices (thc_solver_comm.hpp:422,427).
-// herm: O_in is Hermitian, so is O_out; its lower tiles are formed and mirrored.
 void project_p2a(thcgw_ctx* ctx, hipStream_t s, const c128* X, const c128* Oin, c128* Oout, long nbk, c128* Abuf,
-                 bool herm = false, int xmod = 0) {
+                 Proj proj = PROJ_FULL, int xmod = 0) {
   const int nk = xmod > 0 ? xmod : ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu;
   const long sX = static_cast<long>(nmu) * no;
   THCGW_REQUIRE(nbk < (1L << 30), "primary_to_aux: batch too large");
   thcgw::zgemm(s, thcgw::OP_N, thcgw::OP_N, nmu, no, no, kOne, thcgw::bp(X, sX, nk), no,
                thcgw::bp(Oin, static_cast<long>(no) * no), no, kZero, Abuf, sX, no, static_cast<int>(nbk));
   thcgw::zgemm(s, thcgw::OP_N, thcgw::OP_C, nmu, nmu, no, kOne, thcgw::bp(Abuf, sX), no, thcgw::bp(X, sX, nk), no,
-               kZero, Oout, ctx->M, nmu, static_cast<int>(nbk), kZero,
-               herm ? (thcgw::GEMM_TRI_LOWER | thcgw::GEMM_HERM_SUB) : 0);
+               kZero, Oout, ctx->M, nmu, static_cast<int>(nbk), kZero, proj_flags(proj));
 }
 
 // O_out[b,k] = X_k^H O_in[b,k] X_k (thc_solver_comm.hpp:560,563).
@@ -314,20 +323,21 @@ const c64* x_c64(thcgw_ctx* ctx, const c128* X, hipStream_t s) {
   return X64;
 }
 
-// O_out[b,k] = X_k O_in[b,k] X_k^H with O_in complex<double>, result complex<float>; herm as
-// for project_p2a.
+// O_out[b,k] = X_k O_in[b,k] X_k^H with O_in complex<double>, result complex<float>.
 void project_p2a_f32(thcgw_ctx* ctx, hipStream_t s, const c64* X64, const c128* Oin, c64* Oout, long nbk, c64* Abuf,
-                     bool herm = false, bool g3 = false) {
+                     Proj proj = PROJ_FULL, bool g3 = false) {
   const int f = ctx->pf() | (g3 ? thcgw::GEMM_G3 : 0);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu;
   const long sX = static_cast<long>(nmu) * no;
   THCGW_REQUIRE(nbk < (1L << 30), "primary_to_aux: batch too large");
+  THCGW_REQUIRE(proj == PROJ_FULL || ctx->precision != 2,
+                "Hermitian projections (flag 10) are not built for split BF16 (flag 7 = 2)");
   thcgw::cgemm(s, thcgw::OP_N, thcgw::OP_N, nmu, no, no, kOne, thcgw::bp(X64, sX, nk), DT_C64, no,
                thcgw::bp(Oin, static_cast<long>(no) * no), DT_C128, no, kZero, Abuf, DT_C64, sX, no,
                static_cast<int>(nbk), kZero, f);
   thcgw::cgemm(s, thcgw::OP_N, thcgw::OP_C, nmu, nmu, no, kOne, thcgw::bp(Abuf, sX), DT_C64, no,
                thcgw::bp(X64, sX, nk), DT_C64, no, kZero, Oout, DT_C64, ctx->M, nmu, static_cast<int>(nbk), kZero,
-               f | (herm ? (thcgw::GEMM_TRI_LOWER | thcgw::GEMM_HERM_SUB) : 0));
+               f | proj_flags(proj));
 }
 
 // O_out[b,k] = X_k^H O_in[b,k] X_k with O_in complex<float>, result complex<double>; herm: O_in
@@ -382,6 +392,7 @@ void check_herm_g(thcgw_ctx* ctx, const c128* G, hipStream_t s, int nk_g = 0) {
 void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s) {
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
+  const Proj proj = ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
   const long gs = static_cast<long>(nk) * no * no;
   const int P = choose_pair_chunk(ctx, 1);
   const c64* X64 = x_c64(ctx, X, s);
@@ -391,8 +402,8 @@ void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStrea
   const double scale = -2.0 / (double(nk) * nk);
   for (int i0 = 0; i0 < nth; i0 += P) {
     const int c = std::min(P, nth - i0);
-    project_p2a_f32(ctx, s, X64, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, ctx->herm_g);
-    project_p2a_f32(ctx, s, X64, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, ctx->herm_g);
+    project_p2a_f32(ctx, s, X64, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
+    project_p2a_f32(ctx, s, X64, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, proj);
     for (int j = 0; j < c; ++j)
       thcgw::pi_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP + static_cast<long>(j) * nk * M,
                          GN + static_cast<long>(c - 1 - j) * nk * M, Pi + static_cast<long>(i0 + j) * nk * M, M, scale);
@@ -404,6 +415,7 @@ void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t 
   if (ctx->precision != 0) return run_pi_f32(ctx, G, X, Pi, s);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
+  const Proj proj = ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
   const long gs = static_cast<long>(nk) * no * no;  // one tau slice of G
   const int P = choose_pair_chunk(ctx, 2);
   c128* GP = ctx->buf<c128>("pi_gp", static_cast<size_t>(P) * nk * M);
@@ -412,9 +424,9 @@ void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t 
   const double scale = -2.0 / (double(nk) * nk);  // sp = -2 for ns = 1 (rpa_pi.icc:46)
   for (int i0 = 0; i0 < nth; i0 += P) {
     const int c = std::min(P, nth - i0);
-    project_p2a(ctx, s, X, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, ctx->herm_g);
+    project_p2a(ctx, s, X, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
     // G(beta - tau_i) = G[nt-1-i] for i in [i0, i0+c): tau slots [nt-i0-c, nt-i0), reversed
-    project_p2a(ctx, s, X, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, ctx->herm_g);
+    project_p2a(ctx, s, X, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, proj);
     for (int j = 0; j < c; ++j)
       thcgw::pi_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP + static_cast<long>(j) * nk * M,
                      GN + static_cast<long>(c - 1 - j) * nk * M, Pi + static_cast<long>(i0 + j) * nk * M, M, scale);
@@ -1002,12 +1014,13 @@ void run_sigma_f32(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X
   const double scale = -1.0 / (double(nk) * nk);
   // flag 12 bit 3: these projections (Sigma's only, not chi0's) by three real products
   const bool g3 = (thcgw::gemm_complex3() & 8) != 0;
+  const Proj proj = ctx->herm_g ? PROJ_LOWER : PROJ_FULL;
   for (int i0 = 0; i0 < nth; i0 += P) {
     const int c = std::min(P, nth - i0);
     const int c2 = std::max(0, std::min(c, nt / 2 - i0));
-    project_p2a_f32(ctx, s, X64, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, ctx->herm_g, g3);
+    project_p2a_f32(ctx, s, X64, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj, g3);
     if (c2 > 0)
-      project_p2a_f32(ctx, s, X64, G + (nt - i0 - c2) * gs, GN, static_cast<long>(c2) * nk, Ab, ctx->herm_g, g3);
+      project_p2a_f32(ctx, s, X64, G + (nt - i0 - c2) * gs, GN, static_cast<long>(c2) * nk, Ab, proj, g3);
     for (int j = 0; j < c; ++j) {
       const int i = i0 + j;
       const bool second = j < c2;
@@ -1039,12 +1052,13 @@ void run_sigma(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c1
   c128* SN = ctx->buf<c128>("sg_sn", static_cast<size_t>(P) * nk * M);
   c128* Ab = ctx->buf<c128>("proj_ab", static_cast<size_t>(P) * nk * nmu * no);
   const double scale = -1.0 / (double(nk) * nk);
+  const Proj proj = ctx->herm_g ? PROJ_LOWER : PROJ_FULL;
   for (int i0 = 0; i0 < nth; i0 += P) {
     const int c = std::min(P, nth - i0);
     // second pass only for i < nt/2 (thc_gw.icc:53-62 writes Sigma(beta - tau_i) at nt-1-i)
     const int c2 = std::max(0, std::min(c, nt / 2 - i0));
-    project_p2a(ctx, s, X, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, ctx->herm_g);
-    if (c2 > 0) project_p2a(ctx, s, X, G + (nt - i0 - c2) * gs, GN, static_cast<long>(c2) * nk, Ab, ctx->herm_g);
+    project_p2a(ctx, s, X, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
+    if (c2 > 0) project_p2a(ctx, s, X, G + (nt - i0 - c2) * gs, GN, static_cast<long>(c2) * nk, Ab, proj);
     for (int j = 0; j < c; ++j) {
       const int i = i0 + j;
       const bool second = j < c2;
@@ -1148,6 +1162,7 @@ void require_bz(const thcgw_ctx* ctx, const std::string& entry) {
 // k-grid kernel of the full grid and the irreducible q gathered from its result
 // (rpa_pi.icc:160-169).  Projections are batched over tau pairs.
 void run_pi_ibz(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s) {
+  const Proj proj = ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
   check_herm_g(ctx, G, s, ctx->bz_nk_ibz);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const int nqi = ctx->bz_nq_ibz;
@@ -1169,9 +1184,9 @@ void run_pi_ibz(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStrea
   for (int i0 = 0; i0 < nth; i0 += P) {
     const int c = std::min(P, nth - i0);
     for (int j = 0; j < c; ++j) gather(i0 + j, Gg + j * per);
-    project_p2a(ctx, s, Xg, Gg, GP, static_cast<long>(c) * nk, Ab, ctx->herm_g);
+    project_p2a(ctx, s, Xg, Gg, GP, static_cast<long>(c) * nk, Ab, proj);
     for (int j = 0; j < c; ++j) gather(nt - 1 - (i0 + j), Gg + j * per);
-    project_p2a(ctx, s, Xg, Gg, GN, static_cast<long>(c) * nk, Ab, ctx->herm_g);
+    project_p2a(ctx, s, Xg, Gg, GN, static_cast<long>(c) * nk, Ab, proj);
     for (int j = 0; j < c; ++j) {
       thcgw::pi_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP + j * nk * M, GN + j * nk * M, PF, M, scale);
       thcgw::gather_rows(s, PF, M, bz_tab(ctx, BZ_Q_GRID), nullptr, nqi, M, Pi + static_cast<long>(i0 + j) * nqi * M,
@@ -1204,6 +1219,7 @@ const c128* bz_xd(thcgw_ctx* ctx, const c128* X, hipStream_t s) {
 // are batched over tau.
 void run_sigma_ibz(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c128* Sig, bool herm,
                    hipStream_t s) {
+  const Proj proj = ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
   check_herm_g(ctx, G, s, ctx->bz_nk_ibz);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const int nki = ctx->bz_nk_ibz, nqi = ctx->bz_nq_ibz, nkn = ctx->bz_nk_nt, nsym = ctx->bz_nsym;
@@ -1225,7 +1241,7 @@ void run_sigma_ibz(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X
       for (int j = 0; j < c; ++j)
         thcgw::gather_blocks(s, G + itg(j) * gs, bz_tab(ctx, BZ_G_SRC), bz_tab(ctx, BZ_G_TRANS), nullptr, no, nkn,
                              Gg + j * per);
-      project_p2a(ctx, s, X, Gg, B, static_cast<long>(c) * nkn, Ab, ctx->herm_g, nkn);
+      project_p2a(ctx, s, X, Gg, B, static_cast<long>(c) * nkn, Ab, proj, nkn);
       // with flag 10 every Sigma_PQ of an operation is Hermitian (Hadamard sums of Hermitian G
       // and W): its lower half L goes back as X^H L X + (X^H L X)^H, a triangular first product
       const int hn = ctx->herm_g ? nmu : 0;
