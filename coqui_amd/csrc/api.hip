@@ -404,9 +404,7 @@ void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStrea
     const int c = std::min(P, nth - i0);
     project_p2a_f32(ctx, s, X64, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
     project_p2a_f32(ctx, s, X64, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, proj);
-    for (int j = 0; j < c; ++j)
-      thcgw::pi_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP + static_cast<long>(j) * nk * M,
-                         GN + static_cast<long>(c - 1 - j) * nk * M, Pi + static_cast<long>(i0 + j) * nk * M, M, scale);
+    thcgw::pi_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP, GN, Pi + static_cast<long>(i0) * nk * M, M, scale, c);
   }
 }
 
@@ -427,9 +425,7 @@ void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t 
     project_p2a(ctx, s, X, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
     // G(beta - tau_i) = G[nt-1-i] for i in [i0, i0+c): tau slots [nt-i0-c, nt-i0), reversed
     project_p2a(ctx, s, X, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, proj);
-    for (int j = 0; j < c; ++j)
-      thcgw::pi_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP + static_cast<long>(j) * nk * M,
-                     GN + static_cast<long>(c - 1 - j) * nk * M, Pi + static_cast<long>(i0 + j) * nk * M, M, scale);
+    thcgw::pi_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP, GN, Pi + static_cast<long>(i0) * nk * M, M, scale, c);
   }
 }
 
@@ -1021,16 +1017,9 @@ void run_sigma_f32(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X
     project_p2a_f32(ctx, s, X64, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj, g3);
     if (c2 > 0)
       project_p2a_f32(ctx, s, X64, G + (nt - i0 - c2) * gs, GN, static_cast<long>(c2) * nk, Ab, proj, g3);
-    for (int j = 0; j < c; ++j) {
-      const int i = i0 + j;
-      const bool second = j < c2;
-      thcgw::sigma_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP + static_cast<long>(j) * nk * M,
-                            second ? GN + static_cast<long>(c2 - 1 - j) * nk * M : nullptr,
-                            Wqt + static_cast<long>(i) * M, static_cast<long>(nth) * M,
-                            SP + static_cast<long>(j) * nk * M,
-                            second ? SN + static_cast<long>(c2 - 1 - j) * nk * M : nullptr, M, scale,
-                            ctx->herm_g ? nmu : 0);
-    }
+    thcgw::sigma_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP, c2 > 0 ? GN : nullptr,
+                      Wqt + static_cast<long>(i0) * M, static_cast<long>(nth) * M, SP, c2 > 0 ? SN : nullptr, M, scale,
+                      ctx->herm_g ? nmu : 0, c, c2);
     project_a2p_f32(ctx, s, X64, SP, Sig + i0 * gs, static_cast<long>(c) * nk, Ab, ctx->herm_g);
     if (c2 > 0)
       project_a2p_f32(ctx, s, X64, SN, Sig + (nt - i0 - c2) * gs, static_cast<long>(c2) * nk, Ab, ctx->herm_g);
@@ -1059,15 +1048,9 @@ void run_sigma(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c1
     const int c2 = std::max(0, std::min(c, nt / 2 - i0));
     project_p2a(ctx, s, X, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
     if (c2 > 0) project_p2a(ctx, s, X, G + (nt - i0 - c2) * gs, GN, static_cast<long>(c2) * nk, Ab, proj);
-    for (int j = 0; j < c; ++j) {
-      const int i = i0 + j;
-      const bool second = j < c2;
-      thcgw::sigma_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP + static_cast<long>(j) * nk * M,
-                        second ? GN + static_cast<long>(c2 - 1 - j) * nk * M : nullptr, Wqt + static_cast<long>(i) * M,
-                        static_cast<long>(nth) * M, SP + static_cast<long>(j) * nk * M,
-                        second ? SN + static_cast<long>(c2 - 1 - j) * nk * M : nullptr, M, scale,
-                        ctx->herm_g ? nmu : 0);
-    }
+    thcgw::sigma_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP, c2 > 0 ? GN : nullptr,
+                      Wqt + static_cast<long>(i0) * M, static_cast<long>(nth) * M, SP, c2 > 0 ? SN : nullptr, M, scale,
+                      ctx->herm_g ? nmu : 0, c, c2);
     if (ctx->herm_g) {
       project_a2p_herm(ctx, s, X, SP, Sig + i0 * gs, static_cast<long>(c) * nk, Ab);
       if (c2 > 0) project_a2p_herm(ctx, s, X, SN, Sig + (nt - i0 - c2) * gs, static_cast<long>(c2) * nk, Ab);

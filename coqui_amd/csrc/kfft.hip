@@ -172,11 +172,16 @@ constexpr int KT = 256;
 
 // Pi(:, col) = scale * F+[ F-'[Gp] o conj(F-'[Gn]) ], F-' the unscaled forward DFT; the
 // caller passes scale = sp / N_k^2.  Arithmetic in the scalar type of RC; TG and TO are
-// the storage types of G and Pi.
+// the storage types of G and Pi.  One launch covers a batch of tau slices (grid.y): a launch per
+// slice left the chip half empty at small N_mu and drained at the end of every slice.
 template <int N1, int N2, int N3, int S, typename RC, typename TG, typename TO>
 __global__ __launch_bounds__(KT) void pi_kfft_kernel(const TG* __restrict__ Gp, const TG* __restrict__ Gn,
                                                      TO* __restrict__ Pi, long M, double scale) {
   constexpr int L = (N1 / S) * N2 * N3;
+  const long ts = N1 * N2 * N3 * M;  // between tau slices; Gn's run backwards
+  Gp += blockIdx.y * ts;
+  Gn += (gridDim.y - 1 - blockIdx.y) * ts;
+  Pi += blockIdx.y * ts;
   const long gid = static_cast<long>(blockIdx.x) * KT + threadIdx.x;
   const long col = gid / S;
   const int h = static_cast<int>(gid % S);
@@ -194,6 +199,8 @@ __global__ __launch_bounds__(KT) void pi_kfft_kernel(const TG* __restrict__ Gp, 
 }
 
 // S(:, col) = scale * F+[ F-'[G] o F-'[W] ] for up to two G arrays sharing W; scale = -1/N_k^2.
+// Slice j of the batch (grid.y): G1 and S1 forwards, W's slices M apart, and for j < n2 the second
+// arrays backwards from slice n2 - 1.
 // herm_n > 0 (Hermitian S, order herm_n): only the lower half L of S = L + L^H is written: the
 // columns above the diagonal are not formed (zeros are written only inside the diagonal
 // 128 x 128 blocks, the part that a product with K from the tile column reads with tiles up
@@ -202,8 +209,19 @@ template <int N1, int N2, int N3, int S, typename RC, typename TG, typename TW, 
 __global__ __launch_bounds__(KT) void sigma_kfft_kernel(const TG* __restrict__ G1, const TG* __restrict__ G2,
                                                         const TW* __restrict__ W, long w_kstride,
                                                         TO* __restrict__ S1, TO* __restrict__ S2, long M,
-                                                        double scale, int herm_n) {
+                                                        double scale, int herm_n, int n2) {
   constexpr int L = (N1 / S) * N2 * N3;
+  const long ts = N1 * N2 * N3 * M;
+  const int slice = blockIdx.y;
+  G1 += slice * ts;
+  S1 += slice * ts;
+  W += slice * M;
+  if (slice < n2) {
+    G2 += (n2 - 1 - slice) * ts;
+    S2 += (n2 - 1 - slice) * ts;
+  } else {
+    G2 = nullptr;
+  }
   const long gid = static_cast<long>(blockIdx.x) * KT + threadIdx.x;
   const long col = gid / S;
   const int h = static_cast<int>(gid % S);
@@ -247,86 +265,118 @@ __global__ __launch_bounds__(KT) void sigma_kfft_kernel(const TG* __restrict__ G
 }
 
 // ---------------------------------------------------------------------------------
-// Fallback for any grid with N_k <= 16: one thread per column, the column staged in
-// LDS, direct separable DFTs with twiddles from sincospi.  Used for grids without a
-// specialised kernel and as an independent check of the specialised ones.
+// Any grid with N_k <= 16, in FP64: a workgroup takes 16 columns, one thread per (k, column), the
+// columns in LDS and direct separable DFTs with a table of twiddles (sincospi).  Used for grids
+// without a specialised kernel and as an independent check of the specialised ones.  Bound by
+// the LDS reads, one complex value per term.  One thread per column with a sincospi per term took
+// 20 us for one tau slice of the 2 x 2 x 1 grid at N_mu = 24 (nine workgroups); the 20 slices of
+// a 40-point table now take 6.8 us in one launch, and the N_mu = 24 iteration 0.37 ms instead of 1.18.
 // ---------------------------------------------------------------------------------
-constexpr int FB_T = 64;
-constexpr int FB_NK = 16;
+constexpr int FB_C = 16;   // columns per workgroup
+constexpr int FB_NK = 16;  // largest N_k
 
-__device__ void dft3_lds(c128* x /*stride FB_T*/, c128* tmp, int n1, int n2, int n3, int sign) {
-  const int dims[3] = {n1, n2, n3};
-  const int strides[3] = {n2 * n3, n3, 1};
-  const int nk = n1 * n2 * n3;
+struct FbGrid {
+  int n[3], st[3], nk;
+};
+
+// In place DFT of sign SIGN along every dimension of NX arrays x[i][k][column].
+template <int SIGN, int NX>
+__device__ void dft3_lds(c128 (*x)[FB_NK][FB_C], const c128 (*tw)[FB_NK], const FbGrid& g, int k, int c) {
+#pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const int n = dims[d], st = strides[d];
+    const int n = g.n[d], st = g.st[d];
     if (n == 1) continue;
-    for (int e = 0; e < nk; ++e) tmp[e * FB_T] = x[e * FB_T];
-    for (int e = 0; e < nk; ++e) {
-      const int m = (e / st) % n;
-      const int base = e - m * st;
-      c128 acc{0.0, 0.0};
+    c128 acc[NX];
+#pragma unroll
+    for (int i = 0; i < NX; ++i) acc[i] = c128{0.0, 0.0};
+    if (k < g.nk) {
+      const int m = (k / st) % n, base = k - m * st;
+      int t = 0;  // j m mod n
       for (int j = 0; j < n; ++j) {
-        double s, c;
-        sincospi(2.0 * double(sign) * double((j * m) % n) / double(n), &s, &c);
-        acc = cadd(acc, cmul(tmp[(base + j * st) * FB_T], c128{c, s}));
+        const c128 w = tw[d][t];
+#pragma unroll
+        for (int i = 0; i < NX; ++i)
+          acc[i] = cadd(acc[i], cmul(x[i][base + j * st][c], c128{w.x, SIGN > 0 ? w.y : -w.y}));
+        t += m;
+        if (t >= n) t -= n;
       }
-      x[e * FB_T] = acc;
     }
+    __syncthreads();
+    if (k < g.nk)
+#pragma unroll
+      for (int i = 0; i < NX; ++i) x[i][k][c] = acc[i];
+    __syncthreads();
   }
 }
 
+// mode 0 (chi0): O1 = scale F+[F-[A1] o conj(F-[A2])]; mode 1 (Sigma): as sigma_kfft_kernel.
 template <typename TG, typename TW, typename TO>
-__global__ __launch_bounds__(FB_T) void kfft_fallback_kernel(int mode, int n1, int n2, int n3, const TG* A1,
-                                                             const TG* A2, const TW* W, long w_kstride, TO* O1,
-                                                             TO* O2, long M, double scale) {
-  __shared__ c128 xs[FB_NK * FB_T], ys[FB_NK * FB_T], ts[FB_NK * FB_T];
-  const long col = static_cast<long>(blockIdx.x) * FB_T + threadIdx.x;
-  const int nk = n1 * n2 * n3;
-  c128* x = xs + threadIdx.x;
-  c128* y = ys + threadIdx.x;
-  c128* t = ts + threadIdx.x;
-  if (col >= M) return;
-  if (mode == 0) {  // chi0
-    for (int k = 0; k < nk; ++k) {
-      x[k * FB_T] = cvt<c128>(A1[k * M + col]);
-      y[k * FB_T] = cvt<c128>(A2[k * M + col]);
-    }
-    dft3_lds(x, t, n1, n2, n3, -1);
-    dft3_lds(y, t, n1, n2, n3, -1);
-    for (int k = 0; k < nk; ++k) x[k * FB_T] = cscale(cmulconj(x[k * FB_T], y[k * FB_T]), scale);
-    dft3_lds(x, t, n1, n2, n3, +1);
-    for (int k = 0; k < nk; ++k) O1[k * M + col] = cvt<TO>(x[k * FB_T]);
-  } else {  // Sigma
-    for (int k = 0; k < nk; ++k) y[k * FB_T] = cvt<c128>(W[k * w_kstride + col]);
-    dft3_lds(y, t, n1, n2, n3, -1);
-    for (int pass = 0; pass < 2; ++pass) {
-      const TG* G = pass == 0 ? A1 : A2;
-      TO* O = pass == 0 ? O1 : O2;
-      if (G == nullptr) break;
-      for (int k = 0; k < nk; ++k) x[k * FB_T] = cvt<c128>(G[k * M + col]);
-      dft3_lds(x, t, n1, n2, n3, -1);
-      for (int k = 0; k < nk; ++k) x[k * FB_T] = cscale(cmul(x[k * FB_T], y[k * FB_T]), scale);
-      dft3_lds(x, t, n1, n2, n3, +1);
-      for (int k = 0; k < nk; ++k) O[k * M + col] = cvt<TO>(x[k * FB_T]);
-    }
+__global__ __launch_bounds__(FB_NK* FB_C) void kfft_fallback_kernel(int mode, FbGrid g, const TG* A1, const TG* A2,
+                                                                    const TW* W, long w_kstride, TO* O1, TO* O2,
+                                                                    long M, double scale, int herm_n, int n2) {
+  __shared__ c128 x[2][FB_NK][FB_C], tw[3][FB_NK];
+  const int c = threadIdx.x % FB_C, k = threadIdx.x / FB_C;
+  const long col = static_cast<long>(blockIdx.x) * FB_C + c, ts = g.nk * M;
+  const int slice = blockIdx.y;
+  const bool in = k < g.nk && col < M;
+  if (threadIdx.x < 3 * FB_NK) {
+    const int d = threadIdx.x / FB_NK, t = threadIdx.x % FB_NK;
+    double sn = 0.0, cs = 1.0;
+    if (t < g.n[d]) sincospi(2.0 * double(t) / double(g.n[d]), &sn, &cs);
+    tw[d][t] = c128{cs, sn};
+  }
+  const long e = k * M + col + slice * ts;  // element of an array of slices
+  if (mode == 0) {
+    x[0][k][c] = in ? cvt<c128>(A1[e]) : c128{0.0, 0.0};
+    x[1][k][c] = in ? cvt<c128>(A2[k * M + col + (gridDim.y - 1 - slice) * ts]) : c128{0.0, 0.0};
+    __syncthreads();
+    dft3_lds<-1, 2>(x, tw, g, k, c);
+    x[0][k][c] = cscale(cmulconj(x[0][k][c], x[1][k][c]), scale);
+    __syncthreads();
+    dft3_lds<+1, 1>(x, tw, g, k, c);
+    if (in) O1[e] = cvt<TO>(x[0][k][c]);
+    return;
+  }
+  bool keep = true, half = false;  // herm_n: the lower half with the diagonal halved
+  if (herm_n > 0 && col < M) {
+    const int P = static_cast<int>(col / herm_n), Q = static_cast<int>(col % herm_n);
+    keep = Q <= P;
+    half = Q == P;
+  }
+  c128(*y)[FB_NK][FB_C] = x + 1;
+  y[0][k][c] = in ? cvt<c128>(W[k * w_kstride + slice * M + col]) : c128{0.0, 0.0};
+  __syncthreads();
+  dft3_lds<-1, 1>(y, tw, g, k, c);
+  for (int pass = 0; pass < (slice < n2 ? 2 : 1); ++pass) {
+    const long eo = pass == 0 ? e : k * M + col + (n2 - 1 - slice) * ts;
+    const TG* G = pass == 0 ? A1 : A2;
+    TO* O = pass == 0 ? O1 : O2;
+    x[0][k][c] = in && keep ? cvt<c128>(G[eo]) : c128{0.0, 0.0};
+    __syncthreads();
+    dft3_lds<-1, 1>(x, tw, g, k, c);
+    x[0][k][c] = cscale(cmul(x[0][k][c], y[0][k][c]), scale);
+    __syncthreads();
+    dft3_lds<+1, 1>(x, tw, g, k, c);
+    if (in) O[eo] = keep ? cvt<TO>(half ? cscale(x[0][k][c], 0.5) : x[0][k][c]) : TO{0, 0};
+    __syncthreads();
   }
 }
 
 template <int N1, int N2, int N3, int S, typename RC, typename TG, typename TO>
-void launch_pi(hipStream_t s, const TG* Gp, const TG* Gn, TO* Pi, long M, double scale) {
+void launch_pi(hipStream_t s, const TG* Gp, const TG* Gn, TO* Pi, long M, double scale, int slices) {
   const long threads = M * S;
   const unsigned grid = static_cast<unsigned>((threads + KT - 1) / KT);
-  hipLaunchKernelGGL((pi_kfft_kernel<N1, N2, N3, S, RC, TG, TO>), dim3(grid), dim3(KT), 0, s, Gp, Gn, Pi, M, scale);
+  hipLaunchKernelGGL((pi_kfft_kernel<N1, N2, N3, S, RC, TG, TO>), dim3(grid, slices), dim3(KT), 0, s, Gp, Gn, Pi, M,
+                     scale);
 }
 
 template <int N1, int N2, int N3, int S, typename RC, typename TG, typename TW, typename TO>
 void launch_sigma(hipStream_t s, const TG* G1, const TG* G2, const TW* W, long wks, TO* S1, TO* S2, long M,
-                  double scale, int herm_n) {
+                  double scale, int herm_n, int slices, int n2) {
   const long threads = M * S;
   const unsigned grid = static_cast<unsigned>((threads + KT - 1) / KT);
-  hipLaunchKernelGGL((sigma_kfft_kernel<N1, N2, N3, S, RC, TG, TW, TO>), dim3(grid), dim3(KT), 0, s, G1, G2, W, wks,
-                     S1, S2, M, scale, herm_n);
+  hipLaunchKernelGGL((sigma_kfft_kernel<N1, N2, N3, S, RC, TG, TW, TO>), dim3(grid, slices), dim3(KT), 0, s, G1, G2, W,
+                     wks, S1, S2, M, scale, herm_n, n2);
 }
 
 int grid_code(const int* kg) {
@@ -343,22 +393,27 @@ bool kfft_supported(const int* kgrid) {
 
 namespace {
 
+FbGrid fallback_grid(const int* kg) {
+  const int nk = kg[0] * kg[1] * kg[2];
+  THCGW_REQUIRE(nk <= FB_NK, "k-grid not supported by the fused transform kernels");
+  return FbGrid{{kg[0], kg[1], kg[2]}, {kg[1] * kg[2], kg[2], 1}, nk};
+}
+
 template <typename RC, typename TG, typename TO>
 void pi_kfft_t(hipStream_t s, const int* kgrid, bool force_fallback, const TG* Gp, const TG* Gn, TO* Pi, long M,
-               double scale) {
+               double scale, int slices) {
+  if (slices <= 0) return;
   const int code = force_fallback ? 0 : grid_code(kgrid);
   switch (code) {
-    case 1: launch_pi<1, 1, 1, 1, RC>(s, Gp, Gn, Pi, M, scale); break;
-    case 2: launch_pi<2, 2, 2, 1, RC>(s, Gp, Gn, Pi, M, scale); break;
-    case 3: launch_pi<3, 3, 3, 1, RC>(s, Gp, Gn, Pi, M, scale); break;
-    case 4: launch_pi<4, 4, 4, 4, RC>(s, Gp, Gn, Pi, M, scale); break;
+    case 1: launch_pi<1, 1, 1, 1, RC>(s, Gp, Gn, Pi, M, scale, slices); break;
+    case 2: launch_pi<2, 2, 2, 1, RC>(s, Gp, Gn, Pi, M, scale, slices); break;
+    case 3: launch_pi<3, 3, 3, 1, RC>(s, Gp, Gn, Pi, M, scale, slices); break;
+    case 4: launch_pi<4, 4, 4, 4, RC>(s, Gp, Gn, Pi, M, scale, slices); break;
     default: {
-      const int nk = kgrid[0] * kgrid[1] * kgrid[2];
-      THCGW_REQUIRE(nk <= FB_NK, "k-grid not supported by the fused transform kernels");
-      const unsigned grid = static_cast<unsigned>((M + FB_T - 1) / FB_T);
-      hipLaunchKernelGGL((kfft_fallback_kernel<TG, TG, TO>), dim3(grid), dim3(FB_T), 0, s, 0, kgrid[0], kgrid[1],
-                         kgrid[2], Gp, Gn, static_cast<const TG*>(nullptr), 0L, Pi, static_cast<TO*>(nullptr), M,
-                         scale);
+      const unsigned grid = static_cast<unsigned>((M + FB_C - 1) / FB_C);
+      hipLaunchKernelGGL((kfft_fallback_kernel<TG, TG, TO>), dim3(grid, slices), dim3(FB_NK * FB_C), 0, s, 0,
+                         fallback_grid(kgrid), Gp, Gn, static_cast<const TG*>(nullptr), 0L, Pi,
+                         static_cast<TO*>(nullptr), M, scale, 0, 0);
     }
   }
   THCGW_HIP(hipGetLastError());
@@ -366,24 +421,19 @@ void pi_kfft_t(hipStream_t s, const int* kgrid, bool force_fallback, const TG* G
 
 template <typename RC, typename TG, typename TW, typename TO>
 void sigma_kfft_t(hipStream_t s, const int* kgrid, bool force_fallback, const TG* G1, const TG* G2, const TW* W,
-                  long w_kstride, TO* S1, TO* S2, long M, double scale, int herm_n) {
+                  long w_kstride, TO* S1, TO* S2, long M, double scale, int herm_n, int slices, int n2) {
+  if (slices <= 0) return;
+  if (G2 == nullptr) n2 = 0;
   const int code = force_fallback ? 0 : grid_code(kgrid);
   switch (code) {
-    case 1: launch_sigma<1, 1, 1, 1, RC>(s, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n); break;
-    case 2: launch_sigma<2, 2, 2, 1, RC>(s, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n); break;
-    case 3: launch_sigma<3, 3, 3, 1, RC>(s, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n); break;
-    case 4: launch_sigma<4, 4, 4, 4, RC>(s, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n); break;
+    case 1: launch_sigma<1, 1, 1, 1, RC>(s, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n, slices, n2); break;
+    case 2: launch_sigma<2, 2, 2, 1, RC>(s, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n, slices, n2); break;
+    case 3: launch_sigma<3, 3, 3, 1, RC>(s, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n, slices, n2); break;
+    case 4: launch_sigma<4, 4, 4, 4, RC>(s, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n, slices, n2); break;
     default: {
-      const int nk = kgrid[0] * kgrid[1] * kgrid[2];
-      THCGW_REQUIRE(nk <= FB_NK, "k-grid not supported by the fused transform kernels");
-      const unsigned grid = static_cast<unsigned>((M + FB_T - 1) / FB_T);
-      hipLaunchKernelGGL((kfft_fallback_kernel<TG, TW, TO>), dim3(grid), dim3(FB_T), 0, s, 1, kgrid[0], kgrid[1],
-                         kgrid[2], G1, G2, W, w_kstride, S1, S2, M, scale);
-      THCGW_HIP(hipGetLastError());
-      if (herm_n > 0) {  // the lower half of the full result
-        lower_half(s, S1, herm_n, nk);
-        if (G2 != nullptr) lower_half(s, S2, herm_n, nk);
-      }
+      const unsigned grid = static_cast<unsigned>((M + FB_C - 1) / FB_C);
+      hipLaunchKernelGGL((kfft_fallback_kernel<TG, TW, TO>), dim3(grid, slices), dim3(FB_NK * FB_C), 0, s, 1,
+                         fallback_grid(kgrid), G1, G2, W, w_kstride, S1, S2, M, scale, herm_n, n2);
     }
   }
   THCGW_HIP(hipGetLastError());
@@ -392,23 +442,24 @@ void sigma_kfft_t(hipStream_t s, const int* kgrid, bool force_fallback, const TG
 }  // namespace
 
 void pi_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128* Gp, const c128* Gn, c128* Pi,
-             long M, double scale) {
-  pi_kfft_t<c128>(s, kgrid, force_fallback, Gp, Gn, Pi, M, scale);
+             long M, double scale, int slices) {
+  pi_kfft_t<c128>(s, kgrid, force_fallback, Gp, Gn, Pi, M, scale, slices);
 }
 
 void sigma_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128* G1, const c128* G2,
-                const c128* W, long w_kstride, c128* S1, c128* S2, long M, double scale, int herm_n) {
-  sigma_kfft_t<c128>(s, kgrid, force_fallback, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n);
+                const c128* W, long w_kstride, c128* S1, c128* S2, long M, double scale, int herm_n, int slices, int n2) {
+  sigma_kfft_t<c128>(s, kgrid, force_fallback, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n, slices, n2);
 }
 
 void pi_kfft_f32(hipStream_t s, const int* kgrid, bool force_fallback, const c64* Gp, const c64* Gn, c128* Pi,
-                 long M, double scale) {
-  pi_kfft_t<c64>(s, kgrid, force_fallback, Gp, Gn, Pi, M, scale);
+                 long M, double scale, int slices) {
+  pi_kfft_t<c64>(s, kgrid, force_fallback, Gp, Gn, Pi, M, scale, slices);
 }
 
 void sigma_kfft_f32(hipStream_t s, const int* kgrid, bool force_fallback, const c64* G1, const c64* G2,
-                    const c128* W, long w_kstride, c64* S1, c64* S2, long M, double scale, int herm_n) {
-  sigma_kfft_t<c64>(s, kgrid, force_fallback, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n);
+                    const c128* W, long w_kstride, c64* S1, c64* S2, long M, double scale, int herm_n, int slices,
+                    int n2) {
+  sigma_kfft_t<c64>(s, kgrid, force_fallback, G1, G2, W, w_kstride, S1, S2, M, scale, herm_n, slices, n2);
 }
 
 }  // namespace thcgw

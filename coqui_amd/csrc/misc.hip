@@ -552,32 +552,6 @@ void hermitize(hipStream_t s, c128* A, int n, long nb, double scale) {
   THCGW_HIP(hipGetLastError());
 }
 
-// Lower half of a Hermitian matrix, L with A = L + L^H: the strict upper triangle set to zero
-// and the diagonal halved, for nb n x n matrices in place.
-template <typename T>
-__global__ __launch_bounds__(T256) void lower_half_kernel(T* A, int n, long nb) {
-  const long per = static_cast<long>(n) * n;
-  const long e = static_cast<long>(blockIdx.x) * T256 + threadIdx.x;
-  if (e >= per * nb) return;
-  const int i = static_cast<int>((e % per) / n), j = static_cast<int>(e % n);
-  if (i > j) return;
-  using S = decltype(T{}.x);
-  const T x = A[e];
-  A[e] = (i == j) ? T{static_cast<S>(0.5) * x.x, static_cast<S>(0.5) * x.y} : T{0, 0};
-}
-
-template <typename T>
-void lower_half_t(hipStream_t s, T* A, int n, long nb) {
-  const long total = static_cast<long>(n) * n * nb;
-  if (total == 0) return;
-  THCGW_REQUIRE((total + T256 - 1) / T256 < (1L << 31), "lower_half: too many elements");
-  hipLaunchKernelGGL(lower_half_kernel<T>, dim3(static_cast<unsigned>((total + T256 - 1) / T256)), dim3(T256), 0, s, A,
-                     n, nb);
-  THCGW_HIP(hipGetLastError());
-}
-
-void lower_half(hipStream_t s, c128* A, int n, long nb) { lower_half_t(s, A, n, nb); }
-void lower_half(hipStream_t s, c64* A, int n, long nb) { lower_half_t(s, A, n, nb); }
 
 void one_minus_trace(hipStream_t s, const c128* A, long sA, int n, c128* trace, int batch) {
   hipLaunchKernelGGL(one_minus_trace_kernel, dim3(batch), dim3(T256), 0, s, A, sA, n, trace);

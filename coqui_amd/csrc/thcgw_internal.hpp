@@ -126,16 +126,21 @@ void gemm_profile_read(double* ms, double* flops, double* bytes, long* launches)
 
 // kfft.hip
 bool kfft_supported(const int* kgrid);
+// `slices` tau slices per call, N_k M elements apart (W's M apart): Gp, Pi, G1 and S1 forwards, Gn
+// backwards from the last slice, and G2, S2 for the first n2 slices, backwards from slice n2 - 1
 void pi_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128* Gp, const c128* Gn, c128* Pi,
-             long M, double scale);
-// herm_n > 0: S Hermitian of order herm_n, only its lower half L (S = L + L^H) is written
+             long M, double scale, int slices = 1);
+// herm_n > 0: S Hermitian of order herm_n, only its lower half L (S = L + L^H) is written, and only
+// the lower triangle of G and W is used
 void sigma_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128* G1, const c128* G2,
-                const c128* W, long w_kstride, c128* S1, c128* S2, long M, double scale, int herm_n = 0);
+                const c128* W, long w_kstride, c128* S1, c128* S2, long M, double scale, int herm_n = 0,
+                int slices = 1, int n2 = 1);
 // FP32 arithmetic (the generic-grid fallback computes in FP64), complex<float> G and Sigma.
 void pi_kfft_f32(hipStream_t s, const int* kgrid, bool force_fallback, const c64* Gp, const c64* Gn, c128* Pi,
-                 long M, double scale);
+                 long M, double scale, int slices = 1);
 void sigma_kfft_f32(hipStream_t s, const int* kgrid, bool force_fallback, const c64* G1, const c64* G2,
-                    const c128* W, long w_kstride, c64* S1, c64* S2, long M, double scale, int herm_n = 0);
+                    const c128* W, long w_kstride, c64* S1, c64* S2, long M, double scale, int herm_n = 0,
+                    int slices = 1, int n2 = 1);
 
 // kconv.hip: k-space convolutions (chi0 uses the [q][k] table, Sigma the [k][q] one)
 std::vector<int> kminus_table(const int* kgrid);  // t[a * nk + b] = index of k_a - k_b
@@ -200,9 +205,6 @@ void matsubara_inverse(hipStream_t s, const c128* H0, const c128* F, const c128*
 void scale_mo(hipStream_t s, const c128* C, const double* E, const double* tau, double mu, double beta, int nt, int nk,
               int no, c128* CG);
 void hermitize(hipStream_t s, c128* A, int n, long nb, double scale = 1.0);
-// L with A = L + L^H in place (strict upper triangle zeroed, diagonal halved)
-void lower_half(hipStream_t s, c128* A, int n, long nb);
-void lower_half(hipStream_t s, c64* A, int n, long nb);
 void one_minus_trace(hipStream_t s, const c128* A, long sA, int n, c128* trace, int batch);
 void log_re_det(hipStream_t s, const c128* A, long sA, int n, const int* ipiv, double* ldet, int batch);
 // W = P Z - V: rows of Z in the order that undoes the LU column swaps, minus V (nullable).
