@@ -373,7 +373,7 @@ std::string sci(double v);
 // 1e-12 of max |G| (G built from a Hermitian H(k) is Hermitian to rounding).
 void check_herm_g(thcgw_ctx* ctx, const c128* G, hipStream_t s, int nk_g = 0) {
   if (!ctx->herm_g || ctx->deferred) return;
-  const int nbx = 256;
+  const int nbx = 2048;
   double* d = ctx->buf<double>("hg_chk", static_cast<size_t>(2) * nbx);
   thcgw::herm_diff(s, G, ctx->d.no, static_cast<long>(ctx->d.nt) * (nk_g > 0 ? nk_g : ctx->nk), nbx, d);
   std::vector<double> h(static_cast<size_t>(2) * nbx);
@@ -913,7 +913,7 @@ struct FiniteArg {
   long ncplx;  // complex elements
   const char* name;
 };
-constexpr int kNonfiniteBlocks = 512;
+constexpr int kNonfiniteBlocks = 1024;  // 16 waves per CU
 
 void check_finite(thcgw_ctx* ctx, const char* entry, std::initializer_list<FiniteArg> args, hipStream_t s) {
   std::vector<FiniteArg> a;
@@ -921,9 +921,13 @@ void check_finite(thcgw_ctx* ctx, const char* entry, std::initializer_list<Finit
     if (x.p && x.ncplx > 0) a.push_back(x);
   if (a.empty()) return;
   int* cnt = ctx->buf<int>("nf_cnt", a.size() * kNonfiniteBlocks);
-  for (size_t i = 0; i < a.size(); ++i)
-    thcgw::nonfinite_count(s, static_cast<const double*>(a[i].p), 2 * a[i].ncplx, kNonfiniteBlocks,
-                           cnt + i * kNonfiniteBlocks);
+  THCGW_REQUIRE(a.size() <= thcgw::FINITE_MAX, "check_finite: too many arrays");
+  thcgw::FiniteArrays arr{};
+  for (size_t i = 0; i < a.size(); ++i) {
+    arr.p[i] = a[i].p;
+    arr.ncplx[i] = a[i].ncplx;
+  }
+  thcgw::nonfinite_count(s, arr, static_cast<int>(a.size()), kNonfiniteBlocks, cnt);
   if (ctx->deferred) {
     ctx->nf_arrays = static_cast<int>(a.size());
     return;
@@ -1028,8 +1032,10 @@ void run_sigma_f32(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X
   if (herm && !ctx->herm_g) thcgw::hermitize(s, Sig, no, static_cast<long>(nt) * nk);
 }
 
-void run_sigma(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c128* Sig, bool herm, hipStream_t s) {
-  check_herm_g(ctx, G, s);
+// g_checked: the caller's run_pi has checked the same G for flag 10.
+void run_sigma(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c128* Sig, bool herm, hipStream_t s,
+               bool g_checked = false) {
+  if (!g_checked) check_herm_g(ctx, G, s);
   if (ctx->precision != 0) return run_sigma_f32(ctx, G, Wqt, X, Sig, herm, s);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
@@ -1201,9 +1207,9 @@ const c128* bz_xd(thcgw_ctx* ctx, const c128* X, hipStream_t s) {
 // by D (one product with X_{kS} D), and the sum over S.  Projections and back-projections
 // are batched over tau.
 void run_sigma_ibz(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c128* Sig, bool herm,
-                   hipStream_t s) {
+                   hipStream_t s, bool g_checked = false) {
   const Proj proj = ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
-  check_herm_g(ctx, G, s, ctx->bz_nk_ibz);
+  if (!g_checked) check_herm_g(ctx, G, s, ctx->bz_nk_ibz);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const int nki = ctx->bz_nk_ibz, nqi = ctx->bz_nq_ibz, nkn = ctx->bz_nk_nt, nsym = ctx->bz_nsym;
   const int nout = nsym * nki;
@@ -1274,7 +1280,7 @@ void run_iteration_ibz(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
                                                    std::to_string(b / nqi) + ", " + std::to_string(b % nqi) + ")");
   }
   run_w_to_tau(ctx, Piw, Wqt, s, nqi);
-  run_sigma_ibz(ctx, G, Wqt, X, Sig, herm, s);
+  run_sigma_ibz(ctx, G, Wqt, X, Sig, herm, s, true);
   if (Ec) {
     std::vector<std::complex<double>> tr(total);
     std::vector<double> ld(total);
@@ -1312,7 +1318,7 @@ void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
   run_tau_to_w(ctx, Pit, Piw, s);
   run_dyson(ctx, Piw, V, dtr, dld, true, false, s);
   run_w_to_tau(ctx, Piw, Wqt, s);
-  run_sigma(ctx, G, Wqt, X, Sig, herm, s);
+  run_sigma(ctx, G, Wqt, X, Sig, herm, s, true);
 }
 
 // After a deferred enqueue has completed: Cholesky / LU flags of the Dyson step.

@@ -182,33 +182,43 @@ __global__ __launch_bounds__(T256) void batched_trace_kernel(const c128* A, long
   if (threadIdx.x == 0) tr[blockIdx.x] = c128{re, im};
 }
 
-// d[Q] = (2 / nk) sum_k DP[k][Q][Q]: twice the R = 0 diagonal of the projected density.
+// d[Q] = (2 / nk) sum_k DP[k][Q][Q]: twice the R = 0 diagonal of the projected density.  A wave per
+// Q, its lanes over k: the reads are nk scattered elements, so latency, not bandwidth, counts.
 __global__ __launch_bounds__(T256) void hf_diag_kernel(const c128* DP, int nk, int nmu, c128* d) {
-  const int Q = blockIdx.x * T256 + threadIdx.x;
+  const int Q = blockIdx.x * (T256 / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (Q >= nmu) return;
   const long M = static_cast<long>(nmu) * nmu;
   double re = 0.0, im = 0.0;
-  for (int k = 0; k < nk; ++k) {
+  for (int k = lane; k < nk; k += 64) {
     const c128 v = DP[k * M + static_cast<long>(Q) * nmu + Q];
     re += v.x;
     im += v.y;
   }
-  d[Q] = c128{2.0 * re / nk, 2.0 * im / nk};
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    re += __shfl_xor(re, off);
+    im += __shfl_xor(im, off);
+  }
+  if (lane == 0) d[Q] = c128{2.0 * re / nk, 2.0 * im / nk};
 }
 
-// J_P = sum_Q V0[P][Q] d[Q];  FP[k][P][P] += J_P for every k.
+// J_P = sum_Q V0[P][Q] d[Q];  FP[k][P][P] += J_P for every k.  A workgroup per row P, which reads the
+// row in order; one thread per row took 259 us at N_mu = 800 (strided reads by four
+// workgroups) and its input 41 us, now 7 and 5.
 __global__ __launch_bounds__(T256) void hf_hartree_kernel(const c128* V0, const c128* d, c128* FP, int nk, int nmu) {
-  const int P = blockIdx.x * T256 + threadIdx.x;
-  if (P >= nmu) return;
+  __shared__ double sh[T256 / 64];
+  const int P = blockIdx.x;
   const long M = static_cast<long>(nmu) * nmu;
   double re = 0.0, im = 0.0;
   const c128* row = V0 + static_cast<long>(P) * nmu;
-  for (int Q = 0; Q < nmu; ++Q) {
+  for (int Q = threadIdx.x; Q < nmu; Q += T256) {
     const c128 v = row[Q], x = d[Q];
     re += v.x * x.x - v.y * x.y;
     im += v.x * x.y + v.y * x.x;
   }
-  for (int k = 0; k < nk; ++k) {
+  re = block_sum(re, sh);
+  im = block_sum(im, sh);
+  for (int k = threadIdx.x; k < nk; k += T256) {
     c128* f = FP + k * M + static_cast<long>(P) * nmu + P;
     *f = c128{f->x + re, f->y + im};
   }
@@ -316,21 +326,30 @@ __global__ void scatter_ir_terms_kernel(const c128* __restrict__ trs, const doub
   }
 }
 
-// out[2 (q nbx + bx)] = max |A[mq(q)] - conj A[q]|, out[... + 1] = max |A[q]| over the block's slice
-// out[2 b'] = max |A_ij - conj(A_ji)|, out[2 b' + 1] = max |A_ij| over the elements that block
-// b' visits (grid stride over all nb matrices of order n).
+// out[2 b'] = max |A_ij - conj(A_ji)|, out[2 b' + 1] = max |A_ij| over block b's share of nb matrices
+// of order n: a workgroup takes a matrix at a time and each pair of elements once.  The
+// transposed reads come out of the caches; a 64-bit division per element and 256 workgroups
+// took 201 us for 5120 matrices of order 60 (295 MB), this takes 83.
 __global__ __launch_bounds__(T256) void herm_diff_kernel(const c128* __restrict__ A, int n, long nb,
                                                          double* __restrict__ out) {
   __shared__ double r0[T256], r1[T256];
-  const long nn = static_cast<long>(n) * n, total = nn * nb;
+  const long nn = static_cast<long>(n) * n;
   double d = 0.0, m = 0.0;
-  for (long e = static_cast<long>(blockIdx.x) * T256 + threadIdx.x; e < total;
-       e += static_cast<long>(gridDim.x) * T256) {
-    const long b = e / nn;
-    const int ij = static_cast<int>(e - b * nn), i = ij / n, j = ij % n;
-    const c128 u = A[e], v = A[b * nn + static_cast<long>(j) * n + i];
-    d = fmax(d, fmax(fabs(u.x - v.x), fabs(u.y + v.y)));
-    m = fmax(m, fmax(fabs(u.x), fabs(u.y)));
+  for (long b = blockIdx.x; b < nb; b += gridDim.x) {
+    const c128* Ab = A + b * nn;
+    int i = threadIdx.x / n, j = threadIdx.x % n;
+    while (i < n) {
+      if (j <= i) {
+        const c128 u = Ab[static_cast<long>(i) * n + j], v = Ab[static_cast<long>(j) * n + i];
+        d = fmax(d, fmax(fabs(u.x - v.x), fabs(u.y + v.y)));
+        m = fmax(m, fmax(fmax(fabs(u.x), fabs(u.y)), fmax(fabs(v.x), fabs(v.y))));
+      }
+      j += T256;  // the next element of this thread, row-major
+      while (j >= n) {
+        j -= n;
+        ++i;
+      }
+    }
   }
   r0[threadIdx.x] = d;
   r1[threadIdx.x] = m;
@@ -348,6 +367,7 @@ __global__ __launch_bounds__(T256) void herm_diff_kernel(const c128* __restrict_
   }
 }
 
+// out[2 (q nbx + bx)] = max |A[mq(q)] - conj A[q]|, out[... + 1] = max |A[q]| over the block's slice
 __global__ __launch_bounds__(T256) void trev_diff_kernel(const c128* __restrict__ A, long M, const int* __restrict__ mq,
                                                          double* __restrict__ out) {
   __shared__ double r0[T256], r1[T256];
@@ -378,20 +398,29 @@ __global__ __launch_bounds__(T256) void trev_diff_kernel(const c128* __restrict_
 }
 
 
-// Input guard: out[block] = number of NaN / infinite doubles among x[0, n) in the block's
-// grid-stride share (blocks read 256 consecutive doubles per step).
-__global__ __launch_bounds__(T256) void nonfinite_kernel(const double* __restrict__ x, long n, int* __restrict__ out) {
-  __shared__ int r[T256];
+// Input guard: out[a * gridDim.x + block] = number of NaN / infinite doubles in the block's
+// grid-stride share of array a = blockIdx.y.  Bound by HBM: four 16-byte reads per lane in flight
+// (read one 8-byte value at a time by 512 workgroups it ran at 2.3 TB/s, one launch per array).
+__global__ __launch_bounds__(T256) void nonfinite_kernel(FiniteArrays arr, int* __restrict__ out) {
+  const double2* __restrict__ x = static_cast<const double2*>(arr.p[blockIdx.y]);
+  const long n = arr.ncplx[blockIdx.y], stride = static_cast<long>(gridDim.x) * T256;
   int c = 0;
-  for (long e = static_cast<long>(blockIdx.x) * T256 + threadIdx.x; e < n; e += static_cast<long>(gridDim.x) * T256)
-    c += isfinite(x[e]) ? 0 : 1;
-  r[threadIdx.x] = c;
-  __syncthreads();
-  for (int w = T256 / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) r[threadIdx.x] += r[threadIdx.x + w];
-    __syncthreads();
+  auto bad = [](double2 v) { return (isfinite(v.x) ? 0 : 1) + (isfinite(v.y) ? 0 : 1); };
+  long e = static_cast<long>(blockIdx.x) * T256 + threadIdx.x;
+  for (; e + 3 * stride < n; e += 4 * stride) {
+    const double2 a0 = x[e], a1 = x[e + stride], a2 = x[e + 2 * stride], a3 = x[e + 3 * stride];
+    c += bad(a0) + bad(a1) + bad(a2) + bad(a3);
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = r[0];
+  for (; e < n; e += stride) c += bad(x[e]);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) c += __shfl_xor(c, off);
+  __shared__ int r[T256 / 64];
+  if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < T256 / 64; ++w) c += r[w];
+    out[static_cast<long>(blockIdx.y) * gridDim.x + blockIdx.x] = c;
+  }
 }
 
 // ---- long-wavelength (Gygi) correction ----
@@ -605,10 +634,10 @@ void batched_trace(hipStream_t s, const c128* A, long sA, int n, c128* tr, int b
 }
 
 void hf_hartree(hipStream_t s, const c128* DP, const c128* V0, c128* d, c128* FP, int nk, int nmu) {
-  const unsigned g = static_cast<unsigned>((nmu + T256 - 1) / T256);
+  const unsigned g = static_cast<unsigned>((nmu + T256 / 64 - 1) / (T256 / 64));
   hipLaunchKernelGGL(hf_diag_kernel, dim3(g), dim3(T256), 0, s, DP, nk, nmu, d);
   THCGW_HIP(hipGetLastError());
-  hipLaunchKernelGGL(hf_hartree_kernel, dim3(g), dim3(T256), 0, s, V0, static_cast<const c128*>(d), FP, nk, nmu);
+  hipLaunchKernelGGL(hf_hartree_kernel, dim3(nmu), dim3(T256), 0, s, V0, static_cast<const c128*>(d), FP, nk, nmu);
   THCGW_HIP(hipGetLastError());
 }
 
@@ -693,8 +722,9 @@ void herm_diff(hipStream_t s, const c128* A, int n, long nb, int nbx, double* ou
   THCGW_HIP(hipGetLastError());
 }
 
-void nonfinite_count(hipStream_t s, const double* x, long n, int nbx, int* out) {
-  hipLaunchKernelGGL(nonfinite_kernel, dim3(nbx), dim3(T256), 0, s, x, n, out);
+void nonfinite_count(hipStream_t s, const FiniteArrays& arr, int count, int nbx, int* out) {
+  THCGW_REQUIRE(count >= 1 && count <= FINITE_MAX, "nonfinite_count: too many arrays");
+  hipLaunchKernelGGL(nonfinite_kernel, dim3(nbx, count), dim3(T256), 0, s, arr, out);
   THCGW_HIP(hipGetLastError());
 }
 

@@ -233,8 +233,13 @@ void scatter_ir(hipStream_t s, const c128* S, long M, int n0, int nq, const int*
 void scatter_ir_terms(hipStream_t s, const c128* trs, const double* lds, const int* infos, int n0, int nq,
                       const int* qir, const int* mq, int nqi, int cnt, c128* tr, double* ld, int* info);
 void trev_diff(hipStream_t s, const c128* A, long M, const int* mq, int nq, int nbx, double* out);
-// out[b] (b < nbx) = number of non-finite doubles among x[0, n) in block b's grid-stride share
-void nonfinite_count(hipStream_t s, const double* x, long n, int nbx, int* out);
+// out[a nbx + b] = number of non-finite doubles in block b's share of array a (a < count)
+constexpr int FINITE_MAX = 4;
+struct FiniteArrays {
+  const void* p[FINITE_MAX];
+  long ncplx[FINITE_MAX];
+};
+void nonfinite_count(hipStream_t s, const FiniteArrays& arr, int count, int nbx, int* out);
 
 // Quasiparticle equation per (k, n) state on the device (qp.hip): Pade fit frequencies as
 // rows of Twt_ff (w) with z_i = i * zim[i].
