@@ -26,6 +26,7 @@
 // vector arithmetic: two workgroups per CU (200 registers) hide half of the column step's
 // chain of barrier, maximum, reciprocal, barrier; a budget of three workgroups spills (1.65 ms).
 #include "thcgw_internal.hpp"
+#include "wave.hpp"
 
 #include <cfloat>
 #include <type_traits>
@@ -35,27 +36,6 @@ namespace thcgw {
 namespace {
 
 __device__ __forceinline__ c128 cmul(c128 a, c128 b) { return c128{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
-
-// max(x, x of the lane D away): rows of 16 or halves of 32 lanes exchanged in the vector unit
-// (a shuffle through LDS would add two of its latencies to every column step)
-template <int D>
-__device__ __forceinline__ double swap_max(double x) {
-  const unsigned lo = static_cast<unsigned>(__double2loint(x)), hi = static_cast<unsigned>(__double2hiint(x));
-  const auto l = D == 16 ? __builtin_amdgcn_permlane16_swap(lo, lo, false, false)
-                         : __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-  const auto h = D == 16 ? __builtin_amdgcn_permlane16_swap(hi, hi, false, false)
-                         : __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-  return fmax(__hiloint2double(static_cast<int>(h[0]), static_cast<int>(l[0])),
-              __hiloint2double(static_cast<int>(h[1]), static_cast<int>(l[1])));
-}
-
-// f(0), ..., f(E - 1) with compile-time arguments, for work on the one register row that is picked at
-// run time.  The empty statement at the end of each such branch differs from branch to branch and so
-// keeps the compiler from merging them into one indexed access, which would move the array to memory.
-template <class F, int... A>
-__device__ __forceinline__ void each(F&& f, std::integer_sequence<int, A...>) {
-  (f(std::integral_constant<int, A>{}), ...);
-}
 
 template <int T, int E, bool TRACE>
 __global__ __launch_bounds__(T* T) __attribute__((amdgpu_waves_per_eu(T == 32 ? 4 : E <= 4 ? 4 : 2)))
