@@ -19,6 +19,7 @@
 // matrix is defined.
 #include "lri.hpp"
 #include "thcgw_internal.hpp"
+#include "tri_leaf.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -173,60 +174,6 @@ __global__ __launch_bounds__(256) void zero_block_kernel(c128* A, long sA, int l
   if (e >= static_cast<long>(rows) * cols) return;
   const int r = static_cast<int>(e / cols), c = static_cast<int>(e % cols);
   A[static_cast<long>(blockIdx.y) * sA + static_cast<long>(r) * ld + c] = c128{0.0, 0.0};
-}
-
-// X L^H = T for the lower non-unit nb x nb block L (nb <= CBL); one thread per row of T.
-// RC is the complex arithmetic type; T and L may be stored in another precision.
-template <typename RC, typename TT, typename TL, int CBL = CB>
-__global__ __launch_bounds__(256) void trsm_rlc_leaf_kernel(const TL* L, long sL, int ldl, TT* T, long sT, int ldt,
-                                                            int m, int nb) {
-  using S = decltype(RC{}.x);
-  constexpr int CB = CBL;
-  __shared__ RC Ls[CB][CB];
-  const int b = blockIdx.y;
-  const TL* Lb = L + static_cast<long>(b) * sL;
-  for (int e = threadIdx.x; e < CB * CB; e += 256) {
-    const int r = e / CB, c = e % CB;
-    if (r < nb && c <= r) {
-      const TL v = Lb[static_cast<long>(r) * ldl + c];
-      Ls[r][c] = RC{static_cast<S>(v.x), static_cast<S>(v.y)};
-    } else {
-      Ls[r][c] = RC{0, 0};
-    }
-  }
-  __syncthreads();
-  const int row = blockIdx.x * 256 + threadIdx.x;
-  if (row >= m) return;
-  TT* Tr = T + static_cast<long>(b) * sT + static_cast<long>(row) * ldt;
-  RC x[CB];
-#pragma unroll
-  for (int c = 0; c < CB; ++c) {
-    if (c < nb) {
-      const TT v = Tr[c];
-      x[c] = RC{static_cast<S>(v.x), static_cast<S>(v.y)};
-    } else {
-      x[c] = RC{0, 0};
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < CB; ++c) {
-    if (c < nb) {
-      RC s = x[c];
-#pragma unroll
-      for (int cp = 0; cp < c; ++cp) {  // s -= x[cp] * conj(L[c][cp])
-        const RC a = x[cp], l = Ls[c][cp];
-        s = RC{s.x - (a.x * l.x + a.y * l.y), s.y - (a.y * l.x - a.x * l.y)};
-      }
-      // divide by conj(L[c][c])
-      const RC d = Ls[c][c];
-      const S inv = S(1) / (d.x * d.x + d.y * d.y);
-      x[c] = RC{(s.x * d.x - s.y * d.y) * inv, (s.y * d.x + s.x * d.y) * inv};
-    }
-  }
-  using ST = decltype(TT{}.x);
-#pragma unroll
-  for (int c = 0; c < CB; ++c)
-    if (c < nb) Tr[c] = TT{static_cast<ST>(x[c].x), static_cast<ST>(x[c].y)};
 }
 
 __global__ void fill_int0_kernel(int* p, int n) {
@@ -492,9 +439,7 @@ void trsm_right_lower_conj(hipStream_t s, const c128* L, long sL, int ldl, c128*
                            int batch) {
   if (m <= 0 || nb <= 0 || batch <= 0) return;
   if (nb <= CB) {
-    hipLaunchKernelGGL((trsm_rlc_leaf_kernel<c128, c128, c128>), dim3((m + 255) / 256, batch), dim3(256), 0, s, L, sL,
-                       ldl, T, sT, ldt, m, nb);
-    THCGW_HIP(hipGetLastError());
+    tri_leaf<TRI_ROW_LOWER_CONJ, CB>(s, L, sL, ldl, T, sT, ldt, m, nb, batch);
     return;
   }
   const int n1 = tile_split(nb, CB), n2 = nb - n1;
@@ -513,9 +458,7 @@ void trsm_rlc_utri(hipStream_t s, const c128* L, long sL, int ldl, c128* T, long
                    int batch) {
   const int m = c0 + nb;
   if (nb <= CB) {
-    hipLaunchKernelGGL((trsm_rlc_leaf_kernel<c128, c128, c128>), dim3((m + 255) / 256, batch), dim3(256), 0, s, L, sL,
-                       ldl, T, sT, ldt, m, nb);
-    THCGW_HIP(hipGetLastError());
+    tri_leaf<TRI_ROW_LOWER_CONJ, CB>(s, L, sL, ldl, T, sT, ldt, m, nb, batch);
     return;
   }
   const int n1 = tile_split(nb, CB), n2 = nb - n1;
@@ -546,9 +489,7 @@ void trsm_right_lower_conj_f32(hipStream_t s, const c64* L, long sL, int ldl, c6
                                int nb, int batch, int gemm_flags) {
   if (m <= 0 || nb <= 0 || batch <= 0) return;
   if (nb <= CB32) {
-    hipLaunchKernelGGL((trsm_rlc_leaf_kernel<c64, c64, c64, CB32>), dim3((m + 255) / 256, batch), dim3(256), 0, s, L,
-                       sL, ldl, T, sT, ldt, m, nb);
-    THCGW_HIP(hipGetLastError());
+    tri_leaf<TRI_ROW_LOWER_CONJ, CB32>(s, L, sL, ldl, T, sT, ldt, m, nb, batch);
     return;
   }
   const int n1 = split_point(nb, CB32), n2 = nb - n1;

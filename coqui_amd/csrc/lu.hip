@@ -18,7 +18,7 @@
 // are 16-wide panels factored in registers by one workgroup per matrix.
 #include "thcgw_internal.hpp"
 
-#include "wave.hpp"
+#include "tri_leaf.hpp"
 
 #include <cfloat>
 
@@ -28,7 +28,6 @@ namespace {
 __device__ __forceinline__ c128 cmul(c128 a, c128 b) {
   return c128{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
-__device__ __forceinline__ c128 csub(c128 a, c128 b) { return c128{a.x - b.x, a.y - b.y}; }
 __device__ __forceinline__ c128 crecip(c128 d) {
   const double s = 1.0 / (d.x * d.x + d.y * d.y);
   return c128{d.x * s, -d.y * s};
@@ -130,7 +129,13 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(T * R <= 256 
             const c128 l = cmul(v[s][c], inv);
             v[s][c] = l;
 #pragma unroll
-            for (int cc = c + 1; cc < W; ++cc) v[s][cc] = csub(v[s][cc], cmul(l, prow[cc]));
+            for (int cc = c + 1; cc < W; ++cc) {
+              const c128 u = prow[cc];
+              v[s][cc].x -= l.x * u.x;
+              v[s][cc].y -= l.x * u.y;
+              v[s][cc].x += l.y * u.y;
+              v[s][cc].y -= l.y * u.x;
+            }
           }
       }
     }
@@ -175,83 +180,6 @@ __global__ __launch_bounds__(256) void laswp_kernel(c128* A, long sA, int lda, i
 
 constexpr int LB = 32;  // triangular-solve leaf size
 
-// X U = T for the unit upper nb x nb block U; thread per row of T (m rows).
-__global__ __launch_bounds__(256) void trsm_ruu_leaf(const c128* U, long sU, int ldu, c128* T, long sT, int ldt,
-                                                     int m, int nb) {
-  __shared__ c128 Us[LB][LB];
-  const int b = blockIdx.y;
-  const c128* Ub = U + static_cast<long>(b) * sU;
-  for (int e = threadIdx.x; e < LB * LB; e += 256) {
-    const int i = e / LB, j = e % LB;
-    Us[i][j] = (i < nb && j < nb) ? Ub[static_cast<long>(i) * ldu + j] : c128{0.0, 0.0};
-  }
-  __syncthreads();
-  const int row = blockIdx.x * 256 + threadIdx.x;
-  if (row >= m) return;
-  c128* Tr = T + static_cast<long>(b) * sT + static_cast<long>(row) * ldt;
-  c128 x[LB];
-#pragma unroll
-  for (int c = 0; c < LB; ++c) x[c] = (c < nb) ? Tr[c] : c128{0.0, 0.0};
-#pragma unroll
-  for (int c = 1; c < LB; ++c) {
-    if (c < nb) {
-      c128 s = x[c];
-#pragma unroll
-      for (int cp = 0; cp < c; ++cp) s = csub(s, cmul(x[cp], Us[cp][c]));
-      x[c] = s;
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < LB; ++c)
-    if (c < nb) Tr[c] = x[c];
-}
-
-// L X = B, L lower non-unit (LOWER = true) or U X = B, U upper unit (LOWER = false);
-// nb x nb triangle, thread per right-hand-side column (ncol columns).
-template <bool LOWER>
-__global__ __launch_bounds__(256) void trsm_left_leaf(const c128* Tm, long sTm, int ldm, c128* B, long sB, int ldb,
-                                                      int nb, int ncol) {
-  __shared__ c128 Ts[LB][LB];
-  const int b = blockIdx.y;
-  const c128* Tb = Tm + static_cast<long>(b) * sTm;
-  for (int e = threadIdx.x; e < LB * LB; e += 256) {
-    const int i = e / LB, j = e % LB;
-    Ts[i][j] = (i < nb && j < nb) ? Tb[static_cast<long>(i) * ldm + j] : c128{0.0, 0.0};
-  }
-  __syncthreads();
-  const int col = blockIdx.x * 256 + threadIdx.x;
-  if (col >= ncol) return;
-  c128* Bc = B + static_cast<long>(b) * sB + col;
-  c128 x[LB];
-#pragma unroll
-  for (int r = 0; r < LB; ++r) x[r] = (r < nb) ? Bc[static_cast<long>(r) * ldb] : c128{0.0, 0.0};
-  if (LOWER) {
-#pragma unroll
-    for (int r = 0; r < LB; ++r) {
-      if (r < nb) {
-        c128 s = x[r];
-#pragma unroll
-        for (int c = 0; c < r; ++c) s = csub(s, cmul(Ts[r][c], x[c]));
-        x[r] = cmul(s, crecip(Ts[r][r]));
-      }
-    }
-  } else {
-#pragma unroll
-    for (int r = LB - 1; r >= 0; --r) {
-      if (r < nb) {
-        c128 s = x[r];
-#pragma unroll
-        for (int c = r + 1; c < LB; ++c)
-          if (c < nb) s = csub(s, cmul(Ts[r][c], x[c]));
-        x[r] = s;
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < LB; ++r)
-    if (r < nb) Bc[static_cast<long>(r) * ldb] = x[r];
-}
-
 const Cplx kOne{1.0, 0.0};
 const Cplx kMinusOne{-1.0, 0.0};
 
@@ -273,8 +201,7 @@ void trsm_right_upper_unit(hipStream_t s, const c128* U, long sU, int ldu, c128*
                            int batch) {
   if (m <= 0 || nb <= 0 || batch <= 0) return;
   if (nb <= LB) {
-    hipLaunchKernelGGL(trsm_ruu_leaf, dim3((m + 255) / 256, batch), dim3(256), 0, s, U, sU, ldu, T, sT, ldt, m, nb);
-    THCGW_HIP(hipGetLastError());
+    tri_leaf<TRI_ROW_UPPER_UNIT, LB>(s, U, sU, ldu, T, sT, ldt, m, nb, batch);
     return;
   }
   const int n1 = tile_split(nb, LB), n2 = nb - n1;
@@ -289,9 +216,7 @@ void trsm_left_lower(hipStream_t s, const c128* L, long sL, int ldl, c128* B, lo
                      int batch) {
   if (n <= 0 || ncol <= 0 || batch <= 0) return;
   if (n <= LB) {
-    hipLaunchKernelGGL((trsm_left_leaf<true>), dim3((ncol + 255) / 256, batch), dim3(256), 0, s, L, sL, ldl, B, sB,
-                       ldb, n, ncol);
-    THCGW_HIP(hipGetLastError());
+    tri_leaf<TRI_COL_LOWER, LB>(s, L, sL, ldl, B, sB, ldb, ncol, n, batch);
     return;
   }
   const int n1 = tile_split(n, LB), n2 = n - n1;
@@ -307,9 +232,7 @@ void trsm_left_upper_unit(hipStream_t s, const c128* U, long sU, int ldu, c128* 
                           int batch) {
   if (n <= 0 || ncol <= 0 || batch <= 0) return;
   if (n <= LB) {
-    hipLaunchKernelGGL((trsm_left_leaf<false>), dim3((ncol + 255) / 256, batch), dim3(256), 0, s, U, sU, ldu, B, sB,
-                       ldb, n, ncol);
-    THCGW_HIP(hipGetLastError());
+    tri_leaf<TRI_COL_UPPER_UNIT, LB>(s, U, sU, ldu, B, sB, ldb, ncol, n, batch);
     return;
   }
   const int n1 = tile_split(n, LB), n2 = n - n1;

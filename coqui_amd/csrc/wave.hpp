@@ -38,6 +38,18 @@ __device__ __forceinline__ double wave_max(double x) {
   return swap_max<32>(swap_max<16>(x));
 }
 
+// x of lane N of the row of 16 lanes
+template <int N>
+__device__ __forceinline__ float row_bcast(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x150 + N, 0xF, 0xF, false));
+}
+template <int N>
+__device__ __forceinline__ double row_bcast(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0x150 + N, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0x150 + N, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+
 // f(0), ..., f(E - 1) with compile-time arguments, for register arrays whose loops the compiler
 // unrolls too late or whose row is picked at run time.  A branch on such a row ends in an empty
 // statement that differs from row to row and so keeps the compiler from merging the branches into one

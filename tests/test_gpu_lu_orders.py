@@ -51,3 +51,30 @@ def test_singular_last_column_is_reported(n):
         ctx.dyson_w(PiW, np.eye(n)[None].astype(complex))
     assert e.value.code == 3
     ctx.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n", [1, 16, 17, 33, 63, 65, 130, 900])
+def test_hermitian_form_orders(n, precision):
+    """The same by Cholesky (Hermitian V and Pi), whose triangular leaves are 32 wide in double and
+    64 wide in single precision, with one or four vectors per 16 lanes (up to 16384 rows or more).
+    M = 1 - L^H Pi L has its eigenvalues in [1, 1 + 1]: its factors lose 16 n eps at most."""
+    import torch
+
+    from coqui_amd import IAFT, ThcGW
+
+    rng = np.random.default_rng(n)
+    ia = IAFT.from_table(1000.0, "1e2.1e-15")
+    ctx = ThcGW((1, 1, 1), 2, n, ia)
+    ctx.set_flag(6, 1)
+    ctx.set_flag(7, precision)
+    a = rng.standard_normal((2, n, n)) + 1j * rng.standard_normal((2, n, n))
+    B = a @ np.conj(np.swapaxes(a, 1, 2)) / (4 * n)
+    V = B[0] + 0.5 * np.eye(n)
+    Pi = -B[1] / np.linalg.norm(B[1], 2) / np.linalg.norm(V, 2)
+    PiW = torch.from_numpy(np.broadcast_to(Pi, (ia.nw_half, 1, n, n)).copy()).cuda()
+    ctx.dyson_w(PiW, V[None])
+    ref = np.linalg.solve(np.eye(n) - V @ Pi, V) - V
+    tol = 16 * n * (EPS if precision == 0 else np.finfo(np.float32).eps)
+    assert np.max(np.abs(PiW.cpu().numpy() - ref)) <= tol * np.linalg.norm(V, 2)
+    ctx.close()
