@@ -27,145 +27,183 @@
 namespace thcgw {
 namespace {
 
-__device__ __forceinline__ c128 cmul(c128 a, c128 b) { return c128{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
-// a * conj(b)
-__device__ __forceinline__ c128 cmulc(c128 a, c128 b) { return c128{a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y}; }
-
 constexpr int CB = 32;  // leaf order
 
-// In-place Cholesky of the nb x nb (nb <= 32) diagonal block at A[j0][j0] of each matrix.
-// info[b] receives j0 + j + 1 for the first non-positive (or NaN) pivot j; the factor then
-// continues with a unit pivot so that the launch stays finite.
-__global__ __launch_bounds__(CB* CB) void potrf_leaf_kernel(c128* A, long sA, int lda, int j0, int nb, int* info) {
-  __shared__ c128 S[CB][CB + 1];
-  __shared__ double s_inv;
-  const int b = blockIdx.x;
-  c128* Ab = A + static_cast<long>(b) * sA + static_cast<long>(j0) * lda + j0;
-  const int t = threadIdx.x;
-  const int i = t / CB, k = t % CB;
-  S[i][k] = (i < nb && k <= i) ? Ab[static_cast<long>(i) * lda + k] : c128{0.0, 0.0};
-  __syncthreads();
-  for (int j = 0; j < nb; ++j) {
-    if (t == 0) {
-      double d = S[j][j].x;
+// Cholesky leaves, order nb <= 32, one workgroup of 256 threads per matrix: thread (ti, tk) holds the
+// elements (ti + 16 a, tk + 16 b), a, b < 2, of the diagonal block at [j0][j0] in registers.  A column
+// step has one barrier: the owners of column j have stored it to LDS, every thread reads its
+// two rows' and two columns' elements of it and updates its own four, and the owners of column j + 1
+// store theirs in the other buffer.  No thread waits for another's square root, reciprocal or scaling:
+// each forms them for itself.  info[b] receives j0 + j + 1 for the first non-positive (or NaN) pivot
+// j; the factor then continues with a unit pivot so that the launch stays finite.
+//
+// What bounds them: the chain of a step (barrier, LDS read, square root and division, update, LDS
+// write) for a few matrices, vector instructions for thousands; four waves and few registers keep
+// several workgroups on a CU.  The roundings are written out, because the forms that hold V^-1
+// multiply a change in the last bits of V's factor by the condition of V.
+struct LeafThread {
+  int ti, tk;
+  __device__ LeafThread() : ti(threadIdx.x >> 4), tk(threadIdx.x & 15) {}
+  __device__ int row(int a) const { return ti + 16 * a; }
+  __device__ int col(int b) const { return tk + 16 * b; }
+};
+
+// In-place Cholesky of the block, lower triangle.
+// 16.9 us per call on 4 matrices with 1024 threads, the block in LDS and three barriers per column,
+// now 12.8: most of it is the chain of a square root and a division per column.
+__global__ __launch_bounds__(256) void potrf_leaf_kernel(c128* A, long sA, int lda, int j0, int nb, int* info) {
+  __shared__ c128 column[2][CB];
+  const LeafThread th;
+  const int mat = blockIdx.x;
+  c128* Ab = A + static_cast<long>(mat) * sA + static_cast<long>(j0) * lda + j0;
+  c128 s[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int i = th.row(a), k = th.col(b);
+      s[a][b] = (i < nb && k <= i) ? Ab[static_cast<long>(i) * lda + k] : c128{0.0, 0.0};
+    }
+  if (th.tk == 0)
+#pragma unroll
+    for (int a = 0; a < 2; ++a) column[0][th.row(a)] = s[a][0];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {  // columns 16 h .. 16 h + 15
+    for (int jj = 0; jj < 16 && 16 * h + jj < nb; ++jj) {
+      const int j = 16 * h + jj;
+      const c128* c = column[j & 1];
+      __syncthreads();
+      double d = c[j].x;
+      c128 ci[2], ck[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        ci[a] = c[th.row(a)];
+        ck[a] = c[th.col(a)];
+      }
       if (!(d > 0.0)) {
-        if (info[b] == 0) info[b] = j0 + j + 1;
+        if (threadIdx.x == 0 && info[mat] == 0) info[mat] = j0 + j + 1;
         d = 1.0;
       }
-      const double l = sqrt(d);
-      S[j][j] = c128{l, 0.0};
-      s_inv = 1.0 / l;
+      const double l = sqrt(d), r = 1.0 / l;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        ci[a] = c128{ci[a].x * r, ci[a].y * r};
+        ck[a] = c128{ck[a].x * r, ck[a].y * r};
+      }
+#pragma unroll
+      for (int a = h; a < 2; ++a) {
+        if (th.tk == jj) s[a][h] = th.row(a) == j ? c128{l, 0.0} : ci[a];
+#pragma unroll
+        for (int b = h; b <= a; ++b)
+          if (th.col(b) > j && th.col(b) <= th.row(a)) {
+            const c128 p = ci[a], q = ck[b];
+            s[a][b].x -= fma(p.x, q.x, p.y * q.y);
+            s[a][b].y -= fma(p.y, q.x, -(p.x * q.y));
+          }
+      }
+      c128* next = column[(j + 1) & 1];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        if (th.tk == jj + 1) next[th.row(a)] = s[a][h];
+        if (h == 0 && jj == 15 && th.tk == 0) next[th.row(a)] = s[a][1];
+      }
     }
-    __syncthreads();
-    if (k == j && i > j && i < nb) {
-      const double r = s_inv;
-      S[i][j] = c128{S[i][j].x * r, S[i][j].y * r};
-    }
-    __syncthreads();
-    if (i > j && k > j && k <= i && i < nb) {
-      const c128 u = cmulc(S[i][j], S[k][j]);
-      S[i][k] = c128{S[i][k].x - u.x, S[i][k].y - u.y};
-    }
-    __syncthreads();
   }
-  if (i < nb && k <= i) Ab[static_cast<long>(i) * lda + k] = S[i][k];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b <= a; ++b) {
+      const int i = th.row(a), k = th.col(b);
+      if (i < nb && k <= i) Ab[static_cast<long>(i) * lda + k] = s[a][b];
+    }
 }
 
-// The leaf of the Cholesky-inverse recursion, order nb <= NB, one workgroup of 1024
-// threads per matrix block with NB * NB / 1024 elements each: the diagonal block at
-// [j0][j0] is factored in place (A = L L^H, lower) and the block of Z at [j0][j0] receives
-// L^-H (upper triangular, zeros below the diagonal).  One LDS array holds the block: in and
-// below the diagonal the factorisation's working values S, above it T = the unscaled rows
-// of L^-1, transposed (T[r][c] at [c][r]; T[j][j] = 1).  Column j of S and row j of T are
-// used unscaled, divided by the pivot d_j = S[j][j] on the fly, so that each column costs
-// one barrier (no thread waits for another's square root or scaling):
+// The leaf of the Cholesky-inverse recursion: the block is factored in place (A = L L^H, lower)
+// and the block of Z at [j0][j0] receives L^-H (upper triangular, zeros below the diagonal).  In
+// and below the diagonal a thread's elements are the factorisation's working values S, above it T = the
+// unscaled rows of L^-1, transposed (T[r][c] at [c][r]; T[j][j] = 1), so that column j of the block
+// holds all that step j uses.  Column j of S and row j of T are used unscaled, divided by the
+// pivot d_j = S[j][j] on the fly:
 //   i >= k > j:  S[i][k] -= S[i][j] conj(S[k][j]) / d_j        (right-looking Cholesky)
 //   r > j >= c:  T[r][c] -= S[r][j] T[j][c] / d_j               (right-looking L^-1)
 // Neither reads an element written in the same step.  At the end L[i][k] = S[i][k] / sqrt(d_k)
-// (L[k][k] = sqrt(d_k)) and L^-1[r][c] = T[r][c] / sqrt(d_r).  info as for potrf_leaf_kernel
-// (a non-positive or NaN pivot is recorded and replaced by 1).  Order 32: 20.7 us per call on
-// 200 matrices, against 46.1 us for a leaf that scales column j and forms L^-1 by one
-// thread's forward substitution per column (three barriers per column).  Order-64 leaves
-// took 89 us (this scheme, four elements per thread, 66.5 KB of LDS) and 78 us (the block
-// in registers, one published column per step): VALU issue, not LDS, bounds them, and
-// either only matched the order-32 leaf together with the products of the level it
-// replaces.
-template <int NB>
-__global__ __launch_bounds__(1024) void cholinv_leaf_kernel(c128* A, long sA, int lda, c128* Z, long sZ, int ldz,
-                                                            int j0, int nb, int* info) {
-  constexpr int EPT = NB * NB / 1024;
-  static_assert(EPT >= 1 && NB * NB == EPT * 1024, "NB * NB must be a multiple of 1024");
-  __shared__ c128 S[NB][NB + 1];
-  const int b = blockIdx.x, t = threadIdx.x;
-  c128* Ab = A + static_cast<long>(b) * sA + static_cast<long>(j0) * lda + j0;
-  c128* Zb = Z + static_cast<long>(b) * sZ + static_cast<long>(j0) * ldz + j0;
-  int ei[EPT], ek[EPT];
+// (L[k][k] = sqrt(d_k)) and L^-1[r][c] = T[r][c] / sqrt(d_r).
+// 2624 matrices: 134.8 us with 1024 threads and the block in LDS, now 59.1; 164 matrices 20.1, now 16.8.
+// Order-64 leaves took 89 us on 200 matrices where order 32 took 20.7 (LDS, 1024 threads) and so only
+// matched it together with the products of the level they replace.
+__global__ __launch_bounds__(256) void cholinv_leaf_kernel(c128* A, long sA, int lda, c128* Z, long sZ, int ldz, int j0,
+                                                           int nb, int* info) {
+  __shared__ c128 column[2][CB];
+  __shared__ double diag[CB];
+  const LeafThread th;
+  const int mat = blockIdx.x;
+  c128* Ab = A + static_cast<long>(mat) * sA + static_cast<long>(j0) * lda + j0;
+  c128* Zb = Z + static_cast<long>(mat) * sZ + static_cast<long>(j0) * ldz + j0;
+  c128 s[2][2];
 #pragma unroll
-  for (int m = 0; m < EPT; ++m) {
-    const int e = t + 1024 * m;
-    ei[m] = e / NB;
-    ek[m] = e % NB;
-    const int i = ei[m], k = ek[m];
-    S[i][k] = (i < nb && k <= i) ? Ab[static_cast<long>(i) * lda + k] : c128{0.0, 0.0};
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int i = th.row(a), k = th.col(b);
+      s[a][b] = (i < nb && k <= i) ? Ab[static_cast<long>(i) * lda + k] : c128{0.0, 0.0};
+    }
+  if (th.tk == 0)
+#pragma unroll
+    for (int a = 0; a < 2; ++a) column[0][th.row(a)] = s[a][0];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    for (int jj = 0; jj < 16 && 16 * h + jj < nb; ++jj) {
+      const int j = 16 * h + jj;
+      const c128* c = column[j & 1];
+      __syncthreads();
+      double d = c[j].x;
+      c128 ci[2], ck[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        ci[a] = c[th.row(a)];
+        ck[a] = c[th.col(a)];
+      }
+      if (!(d > 0.0)) {
+        if (threadIdx.x == 0 && info[mat] == 0) info[mat] = j0 + j + 1;
+        d = 1.0;
+      }
+      if (threadIdx.x == 0) diag[j] = d;  // the pivot as the factorisation uses it
+      const double inv = 1.0 / d;
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = h; b < 2; ++b) {
+          const int i = th.row(a), k = th.col(b);
+          const bool lo = k <= i;
+          if (k > j && (lo || i <= j)) {
+            const c128 p = lo ? ci[a] : ck[b];
+            const c128 q = lo ? c128{ck[b].x, -ck[b].y} : i == j ? c128{1.0, 0.0} : ci[a];
+            s[a][b].x = fma(-inv, fma(p.x, q.x, -(p.y * q.y)), s[a][b].x);
+            s[a][b].y = fma(-inv, fma(p.x, q.y, p.y * q.x), s[a][b].y);
+          }
+        }
+      c128* next = column[(j + 1) & 1];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        if (th.tk == jj + 1) next[th.row(a)] = s[a][h];
+        if (h == 0 && jj == 15 && th.tk == 0) next[th.row(a)] = s[a][1];
+      }
+    }
   }
   __syncthreads();
-  for (int j = 0; j < nb; ++j) {
-    double d = S[j][j].x;
-    if (!(d > 0.0)) {
-      if (t == 0 && info[b] == 0) info[b] = j0 + j + 1;
-      d = 1.0;
-    }
-    const double inv = 1.0 / d;
-    // every read of this step before any write (no element read here is written here), so
-    // that the LDS reads of the thread's elements are in flight together
-    c128 p[EPT], q[EPT], o[EPT];
-    bool upd[EPT];
 #pragma unroll
-    for (int m = 0; m < EPT; ++m) {
-      const int i = ei[m], k = ek[m];
-      const bool in = i < nb && k < nb;
-      const bool lo = in && k <= i && k > j;            // S[i][k], i >= k > j
-      const bool hi = in && k > i && k > j && i <= j;   // T[r][c], r = k > j >= c = i
-      upd[m] = lo || hi;
-      p[m] = q[m] = o[m] = c128{0.0, 0.0};
-      if (lo) {
-        p[m] = S[i][j];
-        const c128 v = S[k][j];
-        q[m] = c128{v.x, -v.y};
-      } else if (hi) {
-        p[m] = S[k][j];
-        q[m] = (i == j) ? c128{1.0, 0.0} : S[i][j];
-      }
-      if (upd[m]) o[m] = S[i][k];
-    }
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int m = 0; m < EPT; ++m)
-      if (upd[m]) {
-        const c128 u = cmul(p[m], q[m]);
-        S[ei[m]][ek[m]] = c128{o[m].x - u.x * inv, o[m].y - u.y * inv};
-      }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int m = 0; m < EPT; ++m) {
-    const int i = ei[m], k = ek[m];
-    if (i >= nb || k >= nb) continue;
-    // the pivots as the factorisation used them
-    const double di = S[i][i].x > 0.0 ? S[i][i].x : 1.0;
-    const double dk = S[k][k].x > 0.0 ? S[k][k].x : 1.0;
-    if (k <= i) {
-      const double sk = sqrt(dk);
-      Ab[static_cast<long>(i) * lda + k] = (k == i) ? c128{sk, 0.0} : c128{S[i][k].x / sk, S[i][k].y / sk};
+    for (int b = 0; b < 2; ++b) {
+      const int i = th.row(a), k = th.col(b);
+      if (i >= nb || k >= nb) continue;
+      const double sk = sqrt(diag[k]), r = 1.0 / sk;
+      const c128 v = s[a][b];
+      if (k <= i) Ab[static_cast<long>(i) * lda + k] = (k == i) ? c128{sk, 0.0} : c128{v.x / sk, v.y / sk};
+      // Z[i][k] = conj(L^-1[k][i]) on and above the diagonal, 0 below
+      Zb[static_cast<long>(i) * ldz + k] =
+          (k == i) ? c128{r, 0.0} : (k > i) ? c128{v.x * r, -v.y * r} : c128{0.0, 0.0};
     }
-    // Z[i][k] = conj(L^-1[k][i]) on and above the diagonal, 0 below
-    c128 z{0.0, 0.0};
-    if (k == i) z = c128{1.0 / sqrt(di), 0.0};
-    else if (k > i) {
-      const double r = 1.0 / sqrt(dk);
-      z = c128{S[i][k].x * r, -S[i][k].y * r};
-    }
-    Zb[static_cast<long>(i) * ldz + k] = z;
-  }
 }
 
 // Zero a rows x cols block (leading dimension ld) of each matrix.
@@ -354,7 +392,7 @@ int tile_split(int n, int unit) { return split_point(n, n > 128 ? 64 : unit); }
 
 void potrf_rec(hipStream_t s, c128* A, long sA, int lda, int j0, int n, int* info, int batch) {
   if (n <= CB) {
-    hipLaunchKernelGGL(potrf_leaf_kernel, dim3(batch), dim3(CB * CB), 0, s, A, sA, lda, j0, n, info);
+    hipLaunchKernelGGL(potrf_leaf_kernel, dim3(batch), dim3(256), 0, s, A, sA, lda, j0, n, info);
     THCGW_HIP(hipGetLastError());
     return;
   }
@@ -384,7 +422,7 @@ void potrf_rec(hipStream_t s, c128* A, long sA, int lda, int j0, int n, int* inf
 void cholinv_rec(hipStream_t s, c128* A, long sA, int lda, c128* Z, long sZ, int ldz, int j0, int n, int* info,
                  int batch) {
   if (n <= CB) {
-    hipLaunchKernelGGL(cholinv_leaf_kernel<CB>, dim3(batch), dim3(1024), 0, s, A, sA, lda, Z, sZ, ldz, j0, n, info);
+    hipLaunchKernelGGL(cholinv_leaf_kernel, dim3(batch), dim3(256), 0, s, A, sA, lda, Z, sZ, ldz, j0, n, info);
     THCGW_HIP(hipGetLastError());
     return;
   }

@@ -47,7 +47,7 @@ constexpr int MAX_ORDER = 2048;
 // lowest 11 mantissa bits, so that one floating-point maximum yields the value and the place
 // (lowest column on ties).  NaN counts as zero and infinity as the largest number; what the
 // pivot really holds is looked at when it has been read.
-// Panels of 328 matrices of order 200, on average: 50.6 us with 1024 threads for any order, now 18.4;
+// Panels of 168 matrices of order 200, on average: 50.6 us with 1024 threads for any order, now 18.4;
 // of 164 matrices of order 800: 57.5 us, now 25.8.
 template <int T, int R, int W>
 __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(T * R <= 256 ? 4 : R * W > 16 ? 2 : 4))) void getf2_panel_kernel(

@@ -25,7 +25,7 @@ enum TriLeaf {
 // With L^H the product is rounded before it is subtracted: the forms that hold V^-1 multiply a
 // change in the last bits of V's factor by the condition of V.
 // Against one thread per vector with the triangle read from LDS for each (per launch, order 32):
-// L^H with at most 1600 rows on 4 matrices 23.3 -> 6.2 us; all leaves of the LU form on 328 matrices
+// L^H with at most 1600 rows on 4 matrices 23.3 -> 6.2 us; all leaves of the LU form on 168 matrices
 // of order 200 616 -> 337 us, on 164 of order 800 4.30 -> 2.87 ms.  Order-64 leaves (100 us where two of
 // order 32 take 32 each and the product between them the rest) gained 1% on the latter and lost 4%
 // on order 24.
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void tri_leaf_kernel(const RC* A, long sA, int
 
 // Four vectors per 16 lanes read the triangle once for all four; below 16384 vectors (4 waves per SIMD
 // with one each) more waves are worth more: L^H with at most 1600 rows on 4 matrices 6.2 us with
-// one, 10.4 with four; order 24 on 40 matrices 4.8 and 6.7; order 200 on 328 matrices, the narrow blocks
+// one, 10.4 with four; order 24 on 84 matrices 4.8 and 6.7; order 200 on 168 matrices, the narrow blocks
 // below the line included, 337 us by this rule, 355 with four everywhere.
 template <TriLeaf KIND, int NB, typename RC>
 void tri_leaf(hipStream_t s, const RC* A, long sA, int lda, RC* T, long sT, int ldt, int m, int nb, int batch) {
