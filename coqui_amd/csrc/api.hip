@@ -1423,12 +1423,24 @@ void matsubara_solve(thcgw_ctx* ctx, const c128* H0, const c128* F, const c128* 
   if (tr) thcgw::batched_trace(s, Out, m, no, tr, static_cast<int>(count));
 }
 
+// -2 Re G(beta) summed over the orbitals, from the traces of G(iw_n) averaged over k
+double nelec_from_traces(const thcgw_ctx* ctx, const std::vector<std::complex<double>>& Xw) {
+  const int nw = ctx->d.nw_f, nt = ctx->d.nt;
+  std::complex<double> nel = 0.0;
+  for (int t = 0; t < nt; ++t) {
+    std::complex<double> xt = 0.0;
+    for (int n = 0; n < nw; ++n) xt += ctx->tab.Ttw_ff[static_cast<size_t>(t) * nw + n] * Xw[n];
+    nel += ctx->tab.T_beta[t] * xt;
+  }
+  return -2.0 * nel.real();  // spin factor 2 for ns = npol = 1
+}
+
 // Electron number at mu (compute_Nelec, scf_common.cpp:10-42) with the spectral sum of
 // compute_eigenspectra (simple_dyson.cpp:130-172) taken as the resolvent trace
 // sum_b 1/(iw_n + mu - lambda_b) = Tr[((iw_n + mu) S - H0 - F - Sigma)^-1 S].
 double nelec_at(thcgw_ctx* ctx, const c128* H0, const c128* F, const c128* S, const c128* Sw, double mu,
                 hipStream_t s) {
-  const int nw = ctx->d.nw_f, nk = ctx->nk, nt = ctx->d.nt;
+  const int nw = ctx->d.nw_f, nk = ctx->nk;
   const long count = static_cast<long>(nw) * nk;
   c128* tr = ctx->buf<c128>("dg_tr", static_cast<size_t>(count));
   matsubara_solve(ctx, H0, F, S, Sw, mu, nullptr, tr, s);
@@ -1438,13 +1450,25 @@ double nelec_at(thcgw_ctx* ctx, const c128* H0, const c128* F, const c128* S, co
   std::vector<std::complex<double>> Xw(nw, 0.0);
   for (int n = 0; n < nw; ++n)
     for (int k = 0; k < nk; ++k) Xw[n] += h[static_cast<size_t>(n) * nk + k] / double(nk);  // k weights 1/N_k
-  std::complex<double> nel = 0.0;
-  for (int t = 0; t < nt; ++t) {
-    std::complex<double> xt = 0.0;
-    for (int n = 0; n < nw; ++n) xt += ctx->tab.Ttw_ff[static_cast<size_t>(t) * nw + n] * Xw[n];
-    nel += ctx->tab.T_beta[t] * xt;
-  }
-  return -2.0 * nel.real();  // spin factor 2 for ns = npol = 1
+  return nelec_from_traces(ctx, Xw);
+}
+
+// The same from the Hessenberg forms of H0 + F + Sigma(iw_n) in the orthonormal basis (hessenberg.hip);
+// false when some pivot is zero or not finite.
+bool nelec_from_hessenberg(thcgw_ctx* ctx, const c128* H, double mu, double* nel, hipStream_t s) {
+  const int nw = ctx->d.nw_f, nk = ctx->nk;
+  const size_t count = static_cast<size_t>(nw) * nk;
+  c128* tr = ctx->buf<c128>("dg_tr", count);
+  int* bad = ctx->buf<int>("dg_info", count);
+  c128* sums = ctx->buf<c128>("dg_sum", static_cast<size_t>(nw) + 1);
+  thcgw::hessenberg_traces(s, H, ctx->d_wn_f, ctx->d.beta, mu, nw, nk, ctx->d.no, tr, bad, sums);
+  std::vector<std::complex<double>> h(nw + 1);
+  THCGW_HIP(hipMemcpyAsync(h.data(), sums, sizeof(c128) * h.size(), hipMemcpyDeviceToHost, s));
+  THCGW_HIP(hipStreamSynchronize(s));
+  if (h[nw] != 0.0) return false;
+  h.pop_back();
+  *nel = nelec_from_traces(ctx, h);
+  return true;
 }
 
 }  // namespace
@@ -2096,7 +2120,20 @@ int thcgw_update_mu(thcgw_ctx* ctx, const double* H0, const double* F, const dou
     hipStream_t s = S(stream);
     check_dyson_g_inputs(ctx, "thcgw_update_mu", H0, F, Sov, Sigma, s);
     c128* Sw = sigma_to_w(ctx, C(Sigma), s);
-    auto N = [&](double mu) { return nelec_at(ctx, C(H0), C(F), C(Sov), Sw, mu, s); };
+    // The Hessenberg forms cost about one evaluation by inverses and make each of the 3 to 200
+    // that follow cheap; with an overlap, beyond their order, or should a pivot be lost, by inverses.
+    const c128* H = nullptr;
+    if (!Sov && thcgw::hessenberg_fits(ctx->d.no)) {
+      const int nw = ctx->d.nw_f, no = ctx->d.no;
+      c128* Hb = ctx->buf<c128>("dg_h", static_cast<size_t>(nw) * ctx->nk * no * no);
+      thcgw::hessenberg_reduce(s, C(H0), C(F), Sw, nw, ctx->nk, no, Hb);
+      H = Hb;
+    }
+    auto N = [&](double mu) {
+      double nel;
+      if (H && nelec_from_hessenberg(ctx, H, mu, &nel, s)) return nel;
+      return nelec_at(ctx, C(H0), C(F), C(Sov), Sw, mu, s);
+    };
     // scf_common.cpp:147-202: bracket in steps of 0.2, then bisect to |nel - target| < mu_tol
     const double delta = 0.2;
     double nel = N(old_mu), mu = old_mu;

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(T * R <= 256 
         const unsigned hi = static_cast<unsigned>(__double2hiint(mag)) | ((used << (31 - s)) & 0x80000000u);
         best = fmax(best, __hiloint2double(static_cast<int>(hi), static_cast<int>(lo)));
       }
-      best = wave_max(best);
+      best = wave_reduce(best, MaxOp{});
       if ((t & 63) == 0) key[c & 1][t >> 6] = best;
       __syncthreads();
       best = key[c & 1][0];

@@ -87,8 +87,8 @@ void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, cons
       best = fmax(best, __hiloint2double(static_cast<int>(static_cast<unsigned>(__double2hiint(mag)) | off),
                                          static_cast<int>(lo)));
     }
-    if (T == 16) best = swap_max<16>(best);  // four thread rows per wave, at lanes c, c + 16, c + 32, c + 48
-    best = swap_max<32>(best);
+    if (T == 16) best = swap_with<16>(best, MaxOp{});  // four thread rows per wave, at lanes c, c + 16, c + 32, c + 48
+    best = swap_with<32>(best, MaxOp{});
     if (c == cc) {
 #pragma unroll
       for (int a = 0; a < E; ++a) {

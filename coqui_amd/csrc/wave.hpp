@@ -7,35 +7,46 @@
 
 namespace thcgw {
 
-// max(x, x of the lane D away): rows of 16 or halves of 32 lanes exchanged in the vector unit
-// (a shuffle through LDS adds two of its latencies to a serial step)
-template <int D>
-__device__ __forceinline__ double swap_max(double x) {
+// op(x, x of the lane D away): rows of 16 or halves of 32 lanes exchanged in the vector unit
+// (a shuffle through LDS adds two of its latencies to a serial step).  op is commutative, so that
+// both lanes get the same bits.
+template <int D, class Op>
+__device__ __forceinline__ double swap_with(double x, Op op) {
   static_assert(D == 16 || D == 32, "rows of 16 or halves of 32");
   const unsigned lo = static_cast<unsigned>(__double2loint(x)), hi = static_cast<unsigned>(__double2hiint(x));
   const auto l = D == 16 ? __builtin_amdgcn_permlane16_swap(lo, lo, false, false)
                          : __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
   const auto h = D == 16 ? __builtin_amdgcn_permlane16_swap(hi, hi, false, false)
                          : __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-  return fmax(__hiloint2double(static_cast<int>(h[0]), static_cast<int>(l[0])),
-              __hiloint2double(static_cast<int>(h[1]), static_cast<int>(l[1])));
+  return op(__hiloint2double(static_cast<int>(h[0]), static_cast<int>(l[0])),
+            __hiloint2double(static_cast<int>(h[1]), static_cast<int>(l[1])));
 }
 
-// max(x, x of the lane N to the right in its row of 16 lanes, cyclically)
-template <int N>
-__device__ __forceinline__ double ror_max(double x) {
+// op(x, x of the lane N to the right in its row of 16 lanes, cyclically)
+template <int N, class Op>
+__device__ __forceinline__ double ror_with(double x, Op op) {
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0x120 + N, 0xF, 0xF, false);
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0x120 + N, 0xF, 0xF, false);
-  return fmax(x, __hiloint2double(hi, lo));
+  return op(x, __hiloint2double(hi, lo));
 }
 
-// maximum over the wave, in every lane
-__device__ __forceinline__ double wave_max(double x) {
-  x = ror_max<8>(x);
-  x = ror_max<4>(x);
-  x = ror_max<2>(x);
-  x = ror_max<1>(x);
-  return swap_max<32>(swap_max<16>(x));
+// over the row of 16 lanes, in every lane
+template <class Op>
+__device__ __forceinline__ double row_reduce(double x, Op op) {
+  return ror_with<1>(ror_with<2>(ror_with<4>(ror_with<8>(x, op), op), op), op);
+}
+
+struct MaxOp {
+  __device__ __forceinline__ double operator()(double a, double b) const { return fmax(a, b); }
+};
+struct AddOp {
+  __device__ __forceinline__ double operator()(double a, double b) const { return a + b; }
+};
+
+// over the wave, in every lane
+template <class Op>
+__device__ __forceinline__ double wave_reduce(double x, Op op) {
+  return swap_with<32>(swap_with<16>(row_reduce(x, op), op), op);
 }
 
 // x of lane N of the row of 16 lanes
