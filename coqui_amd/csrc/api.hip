@@ -1454,19 +1454,20 @@ double nelec_at(thcgw_ctx* ctx, const c128* H0, const c128* F, const c128* S, co
 }
 
 // The same from the Hessenberg forms of H0 + F + Sigma(iw_n) in the orthonormal basis (hessenberg.hip);
-// false when some pivot is zero or not finite.
-bool nelec_from_hessenberg(thcgw_ctx* ctx, const c128* H, double mu, double* nel, hipStream_t s) {
+// false when some trace is not finite.
+bool nelec_from_hessenberg(thcgw_ctx* ctx, const c128* H, const c128* rsub, double mu, double* nel, hipStream_t s) {
   const int nw = ctx->d.nw_f, nk = ctx->nk;
   const size_t count = static_cast<size_t>(nw) * nk;
   c128* tr = ctx->buf<c128>("dg_tr", count);
   int* bad = ctx->buf<int>("dg_info", count);
-  c128* sums = ctx->buf<c128>("dg_sum", static_cast<size_t>(nw) + 1);
-  thcgw::hessenberg_traces(s, H, ctx->d_wn_f, ctx->d.beta, mu, nw, nk, ctx->d.no, tr, bad, sums);
-  std::vector<std::complex<double>> h(nw + 1);
+  c128* sums = ctx->buf<c128>("dg_sum", 2 * static_cast<size_t>(nw));
+  thcgw::hessenberg_traces(s, H, rsub, ctx->d_wn_f, ctx->d.beta, mu, nw, nk, ctx->d.no, tr, bad, sums);
+  std::vector<std::complex<double>> h(2 * nw);
   THCGW_HIP(hipMemcpyAsync(h.data(), sums, sizeof(c128) * h.size(), hipMemcpyDeviceToHost, s));
   THCGW_HIP(hipStreamSynchronize(s));
-  if (h[nw] != 0.0) return false;
-  h.pop_back();
+  for (int n = 0; n < nw; ++n)
+    if (h[nw + n] != 0.0) return false;
+  h.resize(nw);
   *nel = nelec_from_traces(ctx, h);
   return true;
 }
@@ -2121,17 +2122,18 @@ int thcgw_update_mu(thcgw_ctx* ctx, const double* H0, const double* F, const dou
     check_dyson_g_inputs(ctx, "thcgw_update_mu", H0, F, Sov, Sigma, s);
     c128* Sw = sigma_to_w(ctx, C(Sigma), s);
     // The Hessenberg forms cost about one evaluation by inverses and make each of the 3 to 200
-    // that follow cheap; with an overlap, beyond their order, or should a pivot be lost, by inverses.
-    const c128* H = nullptr;
+    // that follow cheap; with an overlap, beyond their order, or should a trace be lost, by inverses.
+    c128 *H = nullptr, *rsub = nullptr;
     if (!Sov && thcgw::hessenberg_fits(ctx->d.no)) {
       const int nw = ctx->d.nw_f, no = ctx->d.no;
-      c128* Hb = ctx->buf<c128>("dg_h", static_cast<size_t>(nw) * ctx->nk * no * no);
-      thcgw::hessenberg_reduce(s, C(H0), C(F), Sw, nw, ctx->nk, no, Hb);
-      H = Hb;
+      const size_t rows = static_cast<size_t>(nw) * ctx->nk * no;
+      H = ctx->buf<c128>("dg_h", rows * no);
+      rsub = ctx->buf<c128>("dg_hsub", rows);
+      thcgw::hessenberg_reduce(s, C(H0), C(F), Sw, nw, ctx->nk, no, H, rsub);
     }
     auto N = [&](double mu) {
       double nel;
-      if (H && nelec_from_hessenberg(ctx, H, mu, &nel, s)) return nel;
+      if (H && nelec_from_hessenberg(ctx, H, rsub, mu, &nel, s)) return nel;
       return nelec_at(ctx, C(H0), C(F), C(Sov), Sw, mu, s);
     };
     // scf_common.cpp:147-202: bracket in steps of 0.2, then bisect to |nel - target| < mu_tol

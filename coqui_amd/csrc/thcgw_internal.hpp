@@ -194,13 +194,14 @@ bool ir_transform_fits(int R, int I);
 void ir_transform(hipStream_t s, const c128* T, int R, int I, const c128* in, long ld_in, long bs_in, c128* out,
                   long ld_out, long bs_out, long cols, int batch, bool real_t = false);
 
-// hessenberg.hip: H[n, k] = the Hessenberg form of H0_k + F_k + Sw[n, k] (unitary similarity, order <= 128);
-// tr[n, k] = Tr[(iw_n + mu - H[n, k])^-1], bad[n, k] = 1 where a pivot is zero or not finite, and
-// sums[n] = the traces' average over k, sums[nw].x = the number of bad ones.
+// hessenberg.hip: H[n, k], rsub[n, k] = the Hessenberg form of H0_k + F_k + Sw[n, k] (unitary similarity,
+// order <= 128) as hessenberg_traces reads it: tr[n, k] = Tr[(iw_n + mu - H[n, k])^-1], bad[n, k] = 1 where
+// that is not finite, sums[n] = the average over k, sums[nw + n].x = the number of bad ones.
 bool hessenberg_fits(int no);
-void hessenberg_reduce(hipStream_t s, const c128* H0, const c128* F, const c128* Sw, int nw, int nk, int no, c128* H);
-void hessenberg_traces(hipStream_t s, const c128* H, const long* wn, double beta, double mu, int nw, int nk, int no,
-                       c128* tr, int* bad, c128* sums);
+void hessenberg_reduce(hipStream_t s, const c128* H0, const c128* F, const c128* Sw, int nw, int nk, int no, c128* H,
+                       c128* rsub);
+void hessenberg_traces(hipStream_t s, const c128* H, const c128* rsub, const long* wn, double beta, double mu, int nw,
+                       int nk, int no, c128* tr, int* bad, c128* sums);
 
 // matsubara.hip: Out[n, k] = [(iw_n + mu) S_k - H0_k - F_k - Sw[n, k]]^-1 or tr[n, k] = Tr of that
 // inverse times S_k (exactly one of Out and tr; S and H0 nullable) for orders up to 128;
