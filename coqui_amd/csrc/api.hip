@@ -2047,7 +2047,8 @@ int thcgw_solve_qp(thcgw_ctx* ctx, const double* Sigma, const double* Cmo, const
     const long dim = static_cast<long>(nk) * no;
     double* dE = ctx->buf<double>("qp_e", static_cast<size_t>(2 * dim));
     THCGW_HIP(hipMemcpyAsync(dE, E0, sizeof(double) * dim, hipMemcpyHostToDevice, s));
-    thcgw::qp_solve(s, dg, dg + static_cast<long>(nt) * dim, dE, ctx->d_Twt_ff, fit, nt, dim, mu, eta, tol, dE + dim);
+    c128* sw = ctx->buf<c128>("qp_sw", static_cast<size_t>(nfit) * dim);
+    thcgw::qp_solve(s, dg, dg + static_cast<long>(nt) * dim, dE, ctx->d_Twt_ff, fit, nt, dim, mu, eta, tol, sw, dE + dim);
     THCGW_HIP(hipMemcpyAsync(E_out, dE + dim, sizeof(double) * dim, hipMemcpyDeviceToHost, s));
     THCGW_HIP(hipStreamSynchronize(s));
   });

@@ -259,9 +259,10 @@ struct QpFit {
   double zim[QP_MAX_FIT];
 };
 // E_out[I] for I < dim from sig_t (nt, dim) diagonal Sigma_nn(tau), vhf (dim) diagonal Vhf_nn,
-// E0 (dim) starting energies (all device arrays); Twt (nw_f, nt) the fermionic table.
+// E0 (dim) starting energies (all device arrays); Twt (nw_f, nt) the fermionic table, sig_w
+// (nfit, dim) scratch.
 void qp_solve(hipStream_t s, const c128* sig_t, const c128* vhf, const double* E0, const c128* Twt, const QpFit& fit,
-              int nt, long dim, double mu, double eta, double tol, double* E_out);
+              int nt, long dim, double mu, double eta, double tol, c128* sig_w, double* E_out);
 // per block b' < nbx: max |A_ij - conj(A_ji)| and max |A_ij| over nb matrices of order n
 void herm_diff(hipStream_t s, const c128* A, int n, long nb, int nbx, double* out);
 // q-point symmetry map: W[w][q] = ph_q conj(ph_q)^T o W^[w][src q](perm_q, perm_q) for the q with
