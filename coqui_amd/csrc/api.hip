@@ -90,6 +90,7 @@ struct thcgw_ctx {
   long bz_o[10] = {};
   c128* d_bzD = nullptr;      // orbital rotations (nsym x nk_ibz x no x no)
   int vq() const { return dy_nq > 0 ? dy_nq : nk; }
+  bool pi_lower = false;    // the Dyson step at hand has the lower triangles of Pi only
   std::map<std::string, DevBuf> ws;
   std::string err;
   bool force_fallback = false;
@@ -389,10 +390,11 @@ void check_herm_g(thcgw_ctx* ctx, const c128* G, hipStream_t s, int nk_g = 0) {
                                           " against max |G| = " + sci(mag));
 }
 
-void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s) {
+// lower: of each Pi(q) only the lower triangle (flag 10); the rest of Pi keeps what it held.
+void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s, bool lower = false) {
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
-  const Proj proj = ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
+  const Proj proj = lower ? PROJ_LOWER : ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
   const long gs = static_cast<long>(nk) * no * no;
   const int P = choose_pair_chunk(ctx, 1);
   const c64* X64 = x_c64(ctx, X, s);
@@ -404,16 +406,17 @@ void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStrea
     const int c = std::min(P, nth - i0);
     project_p2a_f32(ctx, s, X64, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
     project_p2a_f32(ctx, s, X64, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, proj);
-    thcgw::pi_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP, GN, Pi + static_cast<long>(i0) * nk * M, M, scale, c);
+    thcgw::pi_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP, GN, Pi + static_cast<long>(i0) * nk * M, M, scale, c,
+                       lower ? nmu : 0);
   }
 }
 
-void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s) {
+void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s, bool lower = false) {
   check_herm_g(ctx, G, s);
-  if (ctx->precision != 0) return run_pi_f32(ctx, G, X, Pi, s);
+  if (ctx->precision != 0) return run_pi_f32(ctx, G, X, Pi, s, lower);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
-  const Proj proj = ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
+  const Proj proj = lower ? PROJ_LOWER : ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
   const long gs = static_cast<long>(nk) * no * no;  // one tau slice of G
   const int P = choose_pair_chunk(ctx, 2);
   c128* GP = ctx->buf<c128>("pi_gp", static_cast<size_t>(P) * nk * M);
@@ -425,16 +428,18 @@ void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t 
     project_p2a(ctx, s, X, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
     // G(beta - tau_i) = G[nt-1-i] for i in [i0, i0+c): tau slots [nt-i0-c, nt-i0), reversed
     project_p2a(ctx, s, X, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, proj);
-    thcgw::pi_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP, GN, Pi + static_cast<long>(i0) * nk * M, M, scale, c);
+    thcgw::pi_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP, GN, Pi + static_cast<long>(i0) * nk * M, M, scale, c,
+                   lower ? nmu : 0);
   }
 }
 
 // Pi(iW_n, q, PQ) = sum_i T+[n][i] Pi(tau_i, q, PQ): one GEMM (nw_half x nt_half) x (nt_half x N_q N_mu^2).
-void run_tau_to_w(thcgw_ctx* ctx, const c128* Pit, c128* Piw, hipStream_t s, int nq = 0) {
+// lower: the lower triangles at least.
+void run_tau_to_w(thcgw_ctx* ctx, const c128* Pit, c128* Piw, hipStream_t s, int nq = 0, bool lower = false) {
   const long cols = ctx->M * (nq > 0 ? nq : ctx->nk);
   if (thcgw::ir_transform_fits(ctx->nw_half, ctx->nt_half)) {
     thcgw::ir_transform(s, ctx->d_Tplus, ctx->nw_half, ctx->nt_half, Pit, cols, 0, Piw, cols, 0, cols, 1,
-                        ctx->real_Tplus);
+                        ctx->real_Tplus, lower ? ctx->d.nmu : 0);
     return;
   }
   THCGW_REQUIRE(cols < (1L << 31), "tau_to_w: N_q N_mu^2 too large for one GEMM");
@@ -706,6 +711,7 @@ void dyson_resolvent_lanes(thcgw_ctx* ctx, c128* PiW, const c128* V, const VFact
       resolvent_back(ctx, PiW, V, f.ldv, b0(c), cbn(c), d_ldet, solve, LU[l], Z[l], ls);
     } else {
       int* ipiv = ctx->buf<int>(l ? "dy_ipiv1" : "dy_ipiv", static_cast<size_t>(CH) * n);
+      if (ctx->pi_lower) thcgw::mirror_lower(ls, PiW + static_cast<long>(b0(c)) * M, M, n, cbn(c));
       dyson_chunk_lu(ctx, PiW, V, b0(c), cbn(c), d_trace, d_ldet, solve, pi_first, LU[l], Z[l], ipiv, info_all + b0(c),
                      ls);
     }
@@ -748,6 +754,7 @@ void dyson_matrices(thcgw_ctx* ctx, c128* PiW, const c128* V, const VFactors& f,
     }
     if (!ipiv) ipiv = ctx->buf<int>("dy_ipiv", static_cast<size_t>(CH) * n);
     if (solve && !Z) Z = ctx->buf<c128>("dy_z", static_cast<size_t>(CH) * M);
+    if (ctx->pi_lower) thcgw::mirror_lower(s, PiW + static_cast<long>(b0) * M, M, n, cb);
     dyson_chunk_lu(ctx, PiW, V, b0, cb, d_trace, d_ldet, solve, pi_first, LU, Z, ipiv, info_all + b0, s);
   }
 }
@@ -1314,9 +1321,20 @@ void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
   check_finite(ctx, "gw_iteration",
                {{G, ctx->d.nt * nk * no * no, "G_tskij"}, {X, nk * ctx->d.nmu * no, "X_skPa"}, {V, ctx->vq() * M, "V_qPQ"}},
                s);
-  run_pi(ctx, G, X, Pit, s);
-  run_tau_to_w(ctx, Pit, Piw, s);
-  run_dyson(ctx, Piw, V, dtr, dld, true, false, s);
+  // With a Hermitian G (flag 10) Pi is Hermitian, and the resolvent form reads its lower triangles
+  // only: the other halves are not formed, and mirrored should a chunk need the LU form after all.
+  // N_k = 64, N_mu = 480, 80 tau points, mixed precision: 58.8 -> 54.5 ms.
+  const bool lower = ctx->herm_g && ctx->dyson_algo == 2 && !ctx->trev && !ctx->sym;
+  run_pi(ctx, G, X, Pit, s, lower);
+  run_tau_to_w(ctx, Pit, Piw, s, 0, lower);
+  {
+    struct Restore {
+      thcgw_ctx* c;
+      ~Restore() { c->pi_lower = false; }
+    } restore{ctx};
+    ctx->pi_lower = lower;
+    run_dyson(ctx, Piw, V, dtr, dld, true, false, s);
+  }
   run_w_to_tau(ctx, Piw, Wqt, s);
   run_sigma(ctx, G, Wqt, X, Sig, herm, s, true);
 }

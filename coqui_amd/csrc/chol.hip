@@ -228,6 +228,16 @@ __global__ __launch_bounds__(256) void zero_upper_kernel(c128* A, long sA, int n
   if (c > r) A[static_cast<long>(blockIdx.y) * sA + e] = c128{0.0, 0.0};
 }
 
+// A[i][j] = conj(A[j][i]), j > i; on the way to the LU form only
+__global__ __launch_bounds__(256) void mirror_lower_kernel(c128* A, long sA, int n) {
+  c128* Ab = A + static_cast<long>(blockIdx.y) * sA;
+  const long e = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+  const int i = static_cast<int>(e / n), j = static_cast<int>(e % n);
+  if (i >= n || j <= i) return;
+  const c128 x = Ab[static_cast<long>(j) * n + i];
+  Ab[e] = c128{x.x, -x.y};
+}
+
 // ldet[b] = 2 sum_j ln Re L[j][j] (+ add[(b + aoff) % amod] when add is given)
 __global__ __launch_bounds__(256) void chol_logdet_kernel(const c128* L, long sL, int n, double* ldet,
                                                           const double* add, int amod, int aoff) {
@@ -547,6 +557,14 @@ void potrf_batched(hipStream_t s, c128* A, long sA, int lda, int n, int* info, i
   hipLaunchKernelGGL(fill_int0_kernel, dim3((batch + 255) / 256), dim3(256), 0, s, info, batch);
   THCGW_HIP(hipGetLastError());
   potrf_rec(s, A, sA, lda, 0, n, info, batch);
+}
+
+void mirror_lower(hipStream_t s, c128* A, long sA, int n, int batch) {
+  if (batch <= 0 || n <= 0) return;
+  const long nn = static_cast<long>(n) * n;
+  hipLaunchKernelGGL(mirror_lower_kernel, dim3(static_cast<unsigned>((nn + 255) / 256), batch), dim3(256), 0, s, A, sA,
+                     n);
+  THCGW_HIP(hipGetLastError());
 }
 
 void zero_upper(hipStream_t s, c128* A, long sA, int n, int batch) {

@@ -26,7 +26,7 @@ template <int RB, int KB, bool CT>
 __global__ __launch_bounds__(256) void ir_transform_kernel(const c128* __restrict__ T, int R, int I,
                                                            const c128* __restrict__ in, long ld_in, long bs_in,
                                                            c128* __restrict__ out, long ld_out, long bs_out,
-                                                           long cols) {
+                                                           long cols, int tri_n) {
   // T in A-fragment order: Tf[rb][kb][lane] = T[16 rb + lane % 16][4 kb + lane / 16] (zero padded)
   __shared__ c128 Tf[RB * KB * 64];
   for (int e = threadIdx.x; e < RB * KB * 64; e += 256) {
@@ -43,6 +43,11 @@ __global__ __launch_bounds__(256) void ir_transform_kernel(const c128* __restric
   const long nblk = (cols + 15) / 16;
   const long stride = static_cast<long>(gridDim.x) * 4;
   for (long cb = static_cast<long>(blockIdx.x) * 4 + (threadIdx.x >> 6); cb < nblk; cb += stride) {
+    if (tri_n > 0) {  // 16 columns of one row above the diagonal
+      const unsigned e = static_cast<unsigned>((cb * 16) % (static_cast<long>(tri_n) * tri_n));
+      const unsigned i = e / tri_n, j = e % tri_n;
+      if (j > i && j + 16 <= static_cast<unsigned>(tri_n)) continue;
+    }
     // Up to 27 fragments the compiler keeps T in registers for the whole loop (2-3 waves per
     // SIMD); beyond that the fragments are re-read from LDS per block, which keeps 3 waves
     // per SIMD instead of 1.
@@ -90,40 +95,42 @@ __global__ __launch_bounds__(256) void ir_transform_kernel(const c128* __restric
 
 template <int RB, int KB>
 void launch_irt(hipStream_t s, const c128* T, int R, int I, const c128* in, long ld_in, long bs_in, c128* out,
-                long ld_out, long bs_out, long cols, int batch, bool real_t) {
+                long ld_out, long bs_out, long cols, int batch, bool real_t, int tri_n) {
   const long nblk = (cols + 15) / 16;
   const long want = (nblk + 3) / 4;                  // one 16-column block per wave
   const long cap = std::max(1L, 4096L / batch);      // about 16 workgroups per CU in all
   const dim3 g(static_cast<unsigned>(std::min(want, cap)), batch);
   if (real_t)
     hipLaunchKernelGGL((ir_transform_kernel<RB, KB, false>), g, dim3(256), 0, s, T, R, I, in, ld_in, bs_in, out,
-                       ld_out, bs_out, cols);
+                       ld_out, bs_out, cols, tri_n);
   else
     hipLaunchKernelGGL((ir_transform_kernel<RB, KB, true>), g, dim3(256), 0, s, T, R, I, in, ld_in, bs_in, out,
-                       ld_out, bs_out, cols);
+                       ld_out, bs_out, cols, tri_n);
   THCGW_HIP(hipGetLastError());
 }
 
 }  // namespace
 
+// tri_n > 0: the columns are elements of matrices of that order, one after the other, of which only the
+// lower triangles are needed; blocks of 16 columns that lie above the diagonal are left out.
 // At most 3 row blocks (R <= 48) and 11 K blocks (I <= 44) of the MFMA; T takes up to 33 KB
 // of LDS.  The 80-point tables (nt_half = 40, nw_half = 41) need the eleventh K block for
 // the iW -> tau direction.
 bool ir_transform_fits(int R, int I) { return R >= 1 && I >= 1 && R <= 48 && I <= 44; }
 
 void ir_transform(hipStream_t s, const c128* T, int R, int I, const c128* in, long ld_in, long bs_in, c128* out,
-                  long ld_out, long bs_out, long cols, int batch, bool real_t) {
+                  long ld_out, long bs_out, long cols, int batch, bool real_t, int tri_n) {
   THCGW_REQUIRE(ir_transform_fits(R, I), "ir_transform: at most 48 rows and 44 columns of T");
   THCGW_REQUIRE(batch >= 1 && batch <= 65535, "ir_transform: batch out of range");
   if (cols <= 0) return;
   if (R <= 32 && I <= 24)
-    launch_irt<2, 6>(s, T, R, I, in, ld_in, bs_in, out, ld_out, bs_out, cols, batch, real_t);
+    launch_irt<2, 6>(s, T, R, I, in, ld_in, bs_in, out, ld_out, bs_out, cols, batch, real_t, tri_n);
   else if (I <= 36)
-    launch_irt<3, 9>(s, T, R, I, in, ld_in, bs_in, out, ld_out, bs_out, cols, batch, real_t);
+    launch_irt<3, 9>(s, T, R, I, in, ld_in, bs_in, out, ld_out, bs_out, cols, batch, real_t, tri_n);
   else if (I <= 40)
-    launch_irt<3, 10>(s, T, R, I, in, ld_in, bs_in, out, ld_out, bs_out, cols, batch, real_t);
+    launch_irt<3, 10>(s, T, R, I, in, ld_in, bs_in, out, ld_out, bs_out, cols, batch, real_t, tri_n);
   else
-    launch_irt<3, 11>(s, T, R, I, in, ld_in, bs_in, out, ld_out, bs_out, cols, batch, real_t);
+    launch_irt<3, 11>(s, T, R, I, in, ld_in, bs_in, out, ld_out, bs_out, cols, batch, real_t, tri_n);
 }
 
 }  // namespace thcgw

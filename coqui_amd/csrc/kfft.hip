@@ -174,9 +174,10 @@ constexpr int KT = 256;
 // caller passes scale = sp / N_k^2.  Arithmetic in the scalar type of RC; TG and TO are
 // the storage types of G and Pi.  One launch covers a batch of tau slices (grid.y): a launch per
 // slice left the chip half empty at small N_mu and drained at the end of every slice.
+// herm_n > 0 (matrices of order herm_n): only the lower triangles are read and written.
 template <int N1, int N2, int N3, int S, typename RC, typename TG, typename TO>
 __global__ __launch_bounds__(KT) void pi_kfft_kernel(const TG* __restrict__ Gp, const TG* __restrict__ Gn,
-                                                     TO* __restrict__ Pi, long M, double scale) {
+                                                     TO* __restrict__ Pi, long M, double scale, int herm_n) {
   constexpr int L = (N1 / S) * N2 * N3;
   const long ts = N1 * N2 * N3 * M;  // between tau slices; Gn's run backwards
   Gp += blockIdx.y * ts;
@@ -186,6 +187,7 @@ __global__ __launch_bounds__(KT) void pi_kfft_kernel(const TG* __restrict__ Gp, 
   const long col = gid / S;
   const int h = static_cast<int>(gid % S);
   if (col >= M) return;  // a column's S lanes are adjacent, so groups exit together
+  if (herm_n > 0 && col % herm_n > col / herm_n) return;
   RC a[L], b[L];
   load_col<N1, N2, N3, S>(a, Gp, M, col, h);
   load_col<N1, N2, N3, S>(b, Gn, M, col, h);
@@ -363,11 +365,11 @@ __global__ __launch_bounds__(FB_NK* FB_C) void kfft_fallback_kernel(int mode, Fb
 }
 
 template <int N1, int N2, int N3, int S, typename RC, typename TG, typename TO>
-void launch_pi(hipStream_t s, const TG* Gp, const TG* Gn, TO* Pi, long M, double scale, int slices) {
+void launch_pi(hipStream_t s, const TG* Gp, const TG* Gn, TO* Pi, long M, double scale, int slices, int herm_n) {
   const long threads = M * S;
   const unsigned grid = static_cast<unsigned>((threads + KT - 1) / KT);
   hipLaunchKernelGGL((pi_kfft_kernel<N1, N2, N3, S, RC, TG, TO>), dim3(grid, slices), dim3(KT), 0, s, Gp, Gn, Pi, M,
-                     scale);
+                     scale, herm_n);
 }
 
 template <int N1, int N2, int N3, int S, typename RC, typename TG, typename TW, typename TO>
@@ -401,14 +403,14 @@ FbGrid fallback_grid(const int* kg) {
 
 template <typename RC, typename TG, typename TO>
 void pi_kfft_t(hipStream_t s, const int* kgrid, bool force_fallback, const TG* Gp, const TG* Gn, TO* Pi, long M,
-               double scale, int slices) {
+               double scale, int slices, int herm_n) {
   if (slices <= 0) return;
   const int code = force_fallback ? 0 : grid_code(kgrid);
   switch (code) {
-    case 1: launch_pi<1, 1, 1, 1, RC>(s, Gp, Gn, Pi, M, scale, slices); break;
-    case 2: launch_pi<2, 2, 2, 1, RC>(s, Gp, Gn, Pi, M, scale, slices); break;
-    case 3: launch_pi<3, 3, 3, 1, RC>(s, Gp, Gn, Pi, M, scale, slices); break;
-    case 4: launch_pi<4, 4, 4, 4, RC>(s, Gp, Gn, Pi, M, scale, slices); break;
+    case 1: launch_pi<1, 1, 1, 1, RC>(s, Gp, Gn, Pi, M, scale, slices, herm_n); break;
+    case 2: launch_pi<2, 2, 2, 1, RC>(s, Gp, Gn, Pi, M, scale, slices, herm_n); break;
+    case 3: launch_pi<3, 3, 3, 1, RC>(s, Gp, Gn, Pi, M, scale, slices, herm_n); break;
+    case 4: launch_pi<4, 4, 4, 4, RC>(s, Gp, Gn, Pi, M, scale, slices, herm_n); break;
     default: {
       const unsigned grid = static_cast<unsigned>((M + FB_C - 1) / FB_C);
       hipLaunchKernelGGL((kfft_fallback_kernel<TG, TG, TO>), dim3(grid, slices), dim3(FB_NK * FB_C), 0, s, 0,
@@ -442,8 +444,8 @@ void sigma_kfft_t(hipStream_t s, const int* kgrid, bool force_fallback, const TG
 }  // namespace
 
 void pi_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128* Gp, const c128* Gn, c128* Pi,
-             long M, double scale, int slices) {
-  pi_kfft_t<c128>(s, kgrid, force_fallback, Gp, Gn, Pi, M, scale, slices);
+             long M, double scale, int slices, int herm_n) {
+  pi_kfft_t<c128>(s, kgrid, force_fallback, Gp, Gn, Pi, M, scale, slices, herm_n);
 }
 
 void sigma_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128* G1, const c128* G2,
@@ -452,8 +454,8 @@ void sigma_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128
 }
 
 void pi_kfft_f32(hipStream_t s, const int* kgrid, bool force_fallback, const c64* Gp, const c64* Gn, c128* Pi,
-                 long M, double scale, int slices) {
-  pi_kfft_t<c64>(s, kgrid, force_fallback, Gp, Gn, Pi, M, scale, slices);
+                 long M, double scale, int slices, int herm_n) {
+  pi_kfft_t<c64>(s, kgrid, force_fallback, Gp, Gn, Pi, M, scale, slices, herm_n);
 }
 
 void sigma_kfft_f32(hipStream_t s, const int* kgrid, bool force_fallback, const c64* G1, const c64* G2,

@@ -129,7 +129,7 @@ bool kfft_supported(const int* kgrid);
 // `slices` tau slices per call, N_k M elements apart (W's M apart): Gp, Pi, G1 and S1 forwards, Gn
 // backwards from the last slice, and G2, S2 for the first n2 slices, backwards from slice n2 - 1
 void pi_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128* Gp, const c128* Gn, c128* Pi,
-             long M, double scale, int slices = 1);
+             long M, double scale, int slices = 1, int herm_n = 0);
 // herm_n > 0: S Hermitian of order herm_n, only its lower half L (S = L + L^H) is written, and only
 // the lower triangle of G and W is used
 void sigma_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128* G1, const c128* G2,
@@ -137,7 +137,7 @@ void sigma_kfft(hipStream_t s, const int* kgrid, bool force_fallback, const c128
                 int slices = 1, int n2 = 1);
 // FP32 arithmetic (the generic-grid fallback computes in FP64), complex<float> G and Sigma.
 void pi_kfft_f32(hipStream_t s, const int* kgrid, bool force_fallback, const c64* Gp, const c64* Gn, c128* Pi,
-                 long M, double scale, int slices = 1);
+                 long M, double scale, int slices = 1, int herm_n = 0);
 void sigma_kfft_f32(hipStream_t s, const int* kgrid, bool force_fallback, const c64* G1, const c64* G2,
                     const c128* W, long w_kstride, c64* S1, c64* S2, long M, double scale, int herm_n = 0,
                     int slices = 1, int n2 = 1);
@@ -173,6 +173,8 @@ void trsm_right_lower_conj(hipStream_t s, const c128* L, long sL, int ldl, c128*
                            int batch);
 void trsm_right_lower_conj_f32(hipStream_t s, const c64* L, long sL, int ldl, c64* T, long sT, int ldt, int m,
                                int nb, int batch, int gemm_flags = 0);
+// A[i][j] = conj(A[j][i]) for j > i in each n x n matrix
+void mirror_lower(hipStream_t s, c128* A, long sA, int n, int batch);
 void zero_upper(hipStream_t s, c128* A, long sA, int n, int batch);
 void chol_logdet(hipStream_t s, const c128* L, long sL, int n, double* ldet, int batch, const double* add = nullptr,
                  int amod = 1, int aoff = 0);
@@ -192,7 +194,7 @@ void herm_finish(hipStream_t s, c128* W, long sW, const c128* V, long sV, int vm
 // and out ld_in / ld_out apart, matrices bs_in / bs_out apart); real_t: only Re T is used
 bool ir_transform_fits(int R, int I);
 void ir_transform(hipStream_t s, const c128* T, int R, int I, const c128* in, long ld_in, long bs_in, c128* out,
-                  long ld_out, long bs_out, long cols, int batch, bool real_t = false);
+                  long ld_out, long bs_out, long cols, int batch, bool real_t = false, int tri_n = 0);
 
 // hessenberg.hip: H[n, k], rsub[n, k] = the Hessenberg form of H0_k + F_k + Sw[n, k] (unitary similarity,
 // order <= 128) as hessenberg_traces reads it: tr[n, k] = Tr[(iw_n + mu - H[n, k])^-1], bad[n, k] = 1 where
