@@ -1,6 +1,7 @@
-// Inverses of the Matsubara matrices X(n, k) = (iw_n + mu) S_k - H0_k - F_k - Sigma(iw_n, k) of
-// order <= 128, one workgroup per matrix, or only the traces Tr[X^-1 S_k] that the electron
-// number needs (simple_dyson.cpp:65-78,130-172).
+// Inverses of order <= 128, one workgroup per matrix: of the Matsubara matrices X(n, k) =
+// (iw_n + mu) S_k - H0_k - F_k - Sigma(iw_n, k), or only the traces Tr[X^-1 S_k] that the electron
+// number needs (simple_dyson.cpp:65-78,130-172), and of the matrices 1 - V Pi of the Dyson
+// equation for W with the trace and the determinant that the RPA energy needs.
 //
 // The matrix is formed in registers and inverted there in place by Gauss-Jordan elimination
 // with partial pivoting: thread (r, c) of T x T holds the E x E elements (r + a T, c + b T).
@@ -37,22 +38,53 @@ namespace {
 
 __device__ __forceinline__ c128 cmul(c128 a, c128 b) { return c128{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
 
-template <int T, int E, bool TRACE>
+// INVERSE: Out = X^-1.  TRACES: tr_out = Tr[X^-1 S].  DYSON: X = Out, replaced by X^-1 - 1 if keep is
+// set; tr_out = Tr[1 - X] and ldet = ln |Re det X| where given.
+enum MatsubaraJob { INVERSE, TRACES, DYSON };
+
+template <int T, int E, MatsubaraJob JOB>
 __global__ __launch_bounds__(T* T) __attribute__((amdgpu_waves_per_eu(T == 32 ? 4 : E <= 4 ? 4 : 2)))
 void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn, double beta,
-                              double mu, int nk, int n, c128* Out, c128* tr_out, int* info) {
-  constexpr int N = T * E;
+                              double mu, int nk, int n, c128* Out, c128* tr_out, int* info, double* ldet, bool keep) {
+  constexpr int N = T * E, NW = T * T / 64;
   __shared__ c128 colv[2][N], rowv[N], scale[N];
   __shared__ double key[2][T * T / 64];
   __shared__ int perm[N], rowpos[N];
-  __shared__ double red[2][T * T / 64];
+  __shared__ double red[4][NW];
+  __shared__ c128 pivot[JOB == DYSON ? N : 1];
   __shared__ int bad;  // first zero or non-finite pivot column + 1
   const long b = blockIdx.x, m = static_cast<long>(n) * n;
   const long kofs = (b % nk) * m;
   const int r = threadIdx.x / T, c = threadIdx.x % T;
 
+  // sums over the workgroup, in its first thread
+  auto block_sum = [&](double x, double* sh) {
+    x = wave_reduce(x, AddOp{});
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
+  };
+  auto total = [&](const double* sh) {
+    double x = sh[0];
+    for (int q = 1; q < NW; ++q) x += sh[q];
+    return x;
+  };
+
   c128 v[E][E];
-  {
+  if constexpr (JOB == DYSON) {
+    double re = 0.0, im = 0.0;
+#pragma unroll
+    for (int a = 0; a < E; ++a)
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const int i = r + a * T, j = c + q * T;
+        v[a][q] = (i < n && j < n) ? Out[b * m + static_cast<long>(i) * n + j] : c128{0.0, 0.0};
+        if (i == j && i < n) {
+          re += 1.0 - v[a][q].x;
+          im -= v[a][q].y;
+        }
+      }
+    block_sum(re, red[0]);
+    block_sum(im, red[1]);
+  } else {
     const double wi = static_cast<double>(wn[b / nk]) * M_PI / beta;
 #pragma unroll
     for (int a = 0; a < E; ++a)
@@ -125,6 +157,7 @@ void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, cons
       if (c == 0) {
         colv[buf][p] = c128{0.0, 0.0};  // the stored row stays as it is
         scale[p] = s;
+        if constexpr (JOB == DYSON) pivot[k] = piv;
         const bool ok = isfinite(piv.x) && isfinite(piv.y) && (piv.x != 0.0 || piv.y != 0.0);
         if (!ok && bad == 0) bad = k + 1;
         perm[k] = p;
@@ -173,7 +206,7 @@ void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, cons
     }
   }
 
-  if constexpr (TRACE) {  // Tr[X^-1 S] = sum over this matrix of X^-1[k][p_j] S[p_j][k]
+  if constexpr (JOB == TRACES) {  // Tr[X^-1 S] = sum over this matrix of X^-1[k][p_j] S[p_j][k]
     double re = 0.0, im = 0.0;
 #pragma unroll
     for (int a = 0; a < E; ++a)
@@ -192,44 +225,74 @@ void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, cons
           }
         }
       }
-    for (int o = 32; o >= 1; o >>= 1) {
-      re += __shfl_xor(re, o);
-      im += __shfl_xor(im, o);
-    }
-    if ((threadIdx.x & 63) == 0) {
-      red[0][threadIdx.x >> 6] = re;
-      red[1][threadIdx.x >> 6] = im;
-    }
+    block_sum(re, red[0]);
+    block_sum(im, red[1]);
     __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int q = 1; q < T * T / 64; ++q) {
-        re += red[0][q];
-        im += red[1][q];
-      }
-      tr_out[b] = c128{re, im};
-    }
+    if (threadIdx.x == 0) tr_out[b] = c128{total(red[0]), total(red[1])};
   } else {
     c128* Ob = Out + b * m;
+    if (JOB == INVERSE || keep) {
 #pragma unroll
-    for (int a = 0; a < E; ++a)
+      for (int a = 0; a < E; ++a)
 #pragma unroll
-      for (int q = 0; q < E; ++q) {
-        const int i = r + a * T, j = c + q * T;
-        if (i < n && j < n) Ob[static_cast<long>(rowpos[i]) * n + perm[j]] = v[a][q];
+        for (int q = 0; q < E; ++q) {
+          const int i = r + a * T, j = c + q * T;
+          if (i < n && j < n) {
+            const int row = rowpos[i], col = perm[j];
+            const double one = JOB == DYSON && row == col ? 1.0 : 0.0;
+            Ob[static_cast<long>(row) * n + col] = c128{v[a][q].x - one, v[a][q].y};
+          }
+        }
+    }
+  }
+  if constexpr (JOB == DYSON) {
+    if (tr_out || ldet) {
+      double la = 0.0, ph = 0.0;  // a swap of rows turns the phase by pi, which |Re det| does not see
+      if (static_cast<int>(threadIdx.x) < n) {
+        const c128 p = pivot[threadIdx.x];
+        la = log(hypot(p.x, p.y));
+        ph = atan2(p.y, p.x);
       }
+      block_sum(la, red[2]);
+      block_sum(ph, red[3]);
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        if (tr_out) tr_out[b] = c128{total(red[0]), total(red[1])};
+        if (ldet) ldet[b] = total(red[2]) + log(fabs(cos(total(red[3]))));
+      }
+    }
   }
 }
 
-template <int T, int E>
-void launch_inverse(hipStream_t s, const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn,
-                    double beta, double mu, int nk, int n, int count, c128* Out, c128* tr, int* info) {
-  if (tr)
-    hipLaunchKernelGGL((matsubara_inverse_kernel<T, E, true>), dim3(count), dim3(T * T), 0, s, H0, F, S, Sw, wn, beta, mu,
-                       nk, n, Out, tr, info);
-  else
-    hipLaunchKernelGGL((matsubara_inverse_kernel<T, E, false>), dim3(count), dim3(T * T), 0, s, H0, F, S, Sw, wn, beta,
-                       mu, nk, n, Out, tr, info);
-  THCGW_HIP(hipGetLastError());
+struct InverseArgs {
+  const c128 *H0, *F, *S, *Sw;
+  const long* wn;
+  double beta, mu;
+  int nk;
+  c128 *Out, *tr;
+  int* info;
+  double* ldet;
+  bool keep;
+};
+
+template <MatsubaraJob JOB>
+void launch_inverse(hipStream_t s, const InverseArgs& x, int n, int count) {
+  auto go = [&](auto t, auto e) {
+    constexpr int T = t, E = e;
+    hipLaunchKernelGGL((matsubara_inverse_kernel<T, E, JOB>), dim3(count), dim3(T * T), 0, s, x.H0, x.F, x.S, x.Sw, x.wn,
+                       x.beta, x.mu, x.nk, n, x.Out, x.tr, x.info, x.ldet, x.keep);
+    THCGW_HIP(hipGetLastError());
+  };
+  using std::integral_constant;
+  switch ((n + 15) / 16) {
+    case 1: go(integral_constant<int, 16>{}, integral_constant<int, 1>{}); break;
+    case 2: go(integral_constant<int, 16>{}, integral_constant<int, 2>{}); break;
+    case 3: go(integral_constant<int, 16>{}, integral_constant<int, 3>{}); break;
+    case 4: go(integral_constant<int, 16>{}, integral_constant<int, 4>{}); break;
+    case 5: go(integral_constant<int, 16>{}, integral_constant<int, 5>{}); break;
+    case 6: go(integral_constant<int, 16>{}, integral_constant<int, 6>{}); break;
+    default: go(integral_constant<int, 32>{}, integral_constant<int, 4>{}); break;
+  }
 }
 
 }  // namespace
@@ -243,16 +306,16 @@ void matsubara_inverse(hipStream_t s, const c128* H0, const c128* F, const c128*
   const long count = static_cast<long>(nw) * nk;
   THCGW_REQUIRE(count < (1L << 30), "Dyson for G: too many matrices");
   if (count == 0) return;
-  const int nb = static_cast<int>(count);
-  switch ((no + 15) / 16) {
-    case 1: launch_inverse<16, 1>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
-    case 2: launch_inverse<16, 2>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
-    case 3: launch_inverse<16, 3>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
-    case 4: launch_inverse<16, 4>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
-    case 5: launch_inverse<16, 5>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
-    case 6: launch_inverse<16, 6>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
-    default: launch_inverse<32, 4>(s, H0, F, S, Sw, wn, beta, mu, nk, no, nb, Out, tr, info); break;
-  }
+  const InverseArgs x{H0, F, S, Sw, wn, beta, mu, nk, Out, tr, info, nullptr, true};
+  if (tr) launch_inverse<TRACES>(s, x, no, static_cast<int>(count));
+  else launch_inverse<INVERSE>(s, x, no, static_cast<int>(count));
+}
+
+void dyson_inverse(hipStream_t s, c128* A, int n, int batch, bool keep, c128* tr, double* ldet, int* info) {
+  THCGW_REQUIRE(matsubara_inverse_fits(n), "dyson_inverse: order must be in [1, 128]");
+  if (batch <= 0) return;
+  const InverseArgs x{nullptr, nullptr, nullptr, nullptr, nullptr, 0.0, 0.0, 1, A, tr, info, ldet, keep};
+  launch_inverse<DYSON>(s, x, n, batch);
 }
 
 }  // namespace thcgw
