@@ -108,6 +108,8 @@ struct thcgw_ctx {
                         // 2 = mixed with split-BF16 products in place of FP32 MFMA
   int tile32 = -1;      // FP32 tile shape chosen for this context (-1: process default)
   bool deferred = false;  // enqueue without host synchronisation (stream capture): checks run later
+  char* readback_p = nullptr;  // pinned memory for results that the host looks at while the stream goes on
+  size_t readback_bytes = 0;
   int nf_arrays = 0;      // arrays whose non-finite counts a deferred enqueue left in "nf_cnt"
   std::map<std::string, DevBuf>* pool = nullptr;  // scratch shared with the other systems of a batch
   // cgemm flags of this context: precision and FP32 tile shape
@@ -138,6 +140,17 @@ struct thcgw_ctx {
     }
     return static_cast<T*>(b.p);
   }
+  // Pinned host memory of at least `need` bytes; no copy into it may be pending.
+  char* readback(size_t need) {
+    if (readback_bytes < need) {
+      if (readback_p) THCGW_HIP(hipHostFree(readback_p));
+      readback_p = nullptr;
+      readback_bytes = 0;
+      THCGW_HIP(hipHostMalloc(reinterpret_cast<void**>(&readback_p), need, hipHostMallocDefault));
+      readback_bytes = need;
+    }
+    return readback_p;
+  }
   // Bytes currently held by workspace `name` (0 if not allocated).
   size_t held_bytes(const std::string& name) const {
     const std::map<std::string, DevBuf>& m = (pool && !private_buf(name)) ? *pool : ws;
@@ -148,6 +161,9 @@ struct thcgw_ctx {
     for (auto& kv : ws)
       if (kv.second.p) (void)hipFree(kv.second.p);
     ws.clear();
+    if (readback_p) (void)hipHostFree(readback_p);
+    readback_p = nullptr;
+    readback_bytes = 0;
     if (d_tau) (void)hipFree(d_tau);
     if (d_Tplus) (void)hipFree(d_Tplus);
     if (d_Tminus) (void)hipFree(d_Tminus);
@@ -933,7 +949,34 @@ struct FiniteArg {
 };
 constexpr int kNonfiniteBlocks = 1024;  // 16 waves per CU
 
-void check_finite(thcgw_ctx* ctx, const char* entry, std::initializer_list<FiniteArg> args, hipStream_t s) {
+// A check whose counts are on their way to pinned memory: refuse() waits for them.
+struct PendingFinite {
+  std::string entry;
+  std::vector<FiniteArg> a;
+  const int* h = nullptr;
+  hipEvent_t ready = nullptr;
+  PendingFinite() = default;
+  PendingFinite(const PendingFinite&) = delete;
+  PendingFinite& operator=(const PendingFinite&) = delete;
+  ~PendingFinite() {
+    if (ready) (void)hipEventDestroy(ready);
+  }
+  void refuse() const {
+    if (ready) THCGW_HIP(hipEventSynchronize(ready));
+    for (size_t i = 0; i < a.size(); ++i) {
+      long bad = 0;
+      for (int b = 0; b < kNonfiniteBlocks; ++b) bad += h[i * kNonfiniteBlocks + b];
+      if (bad > 0)
+        throw thcgw::Error(THCGW_ERR_NONFINITE, entry + ": " + a[i].name + " holds " + std::to_string(bad) +
+                                                    " NaN or infinite values");
+    }
+  }
+};
+
+// With `later` the counts go to the pinned memory at `pinned` (FINITE_MAX * kNonfiniteBlocks ints) and the
+// caller looks at them when it has enqueued more work.
+void check_finite(thcgw_ctx* ctx, const char* entry, std::initializer_list<FiniteArg> args, hipStream_t s,
+                  PendingFinite* later = nullptr, int* pinned = nullptr) {
   std::vector<FiniteArg> a;
   for (const FiniteArg& x : args)
     if (x.p && x.ncplx > 0) a.push_back(x);
@@ -950,16 +993,28 @@ void check_finite(thcgw_ctx* ctx, const char* entry, std::initializer_list<Finit
     ctx->nf_arrays = static_cast<int>(a.size());
     return;
   }
-  std::vector<int> h(a.size() * kNonfiniteBlocks);
-  THCGW_HIP(hipMemcpyAsync(h.data(), cnt, sizeof(int) * h.size(), hipMemcpyDeviceToHost, s));
-  THCGW_HIP(hipStreamSynchronize(s));
-  for (size_t i = 0; i < a.size(); ++i) {
-    long bad = 0;
-    for (int b = 0; b < kNonfiniteBlocks; ++b) bad += h[i * kNonfiniteBlocks + b];
-    if (bad > 0)
-      throw thcgw::Error(THCGW_ERR_NONFINITE, std::string(entry) + ": " + a[i].name + " holds " + std::to_string(bad) +
-                                                  " NaN or infinite values");
+  PendingFinite now;
+  PendingFinite& c = later ? *later : now;
+  c.entry = entry;
+  c.a = a;
+  std::vector<int> h(later ? 0 : a.size() * kNonfiniteBlocks);
+  c.h = later ? pinned : h.data();
+  THCGW_HIP(hipMemcpyAsync(const_cast<int*>(c.h), cnt, sizeof(int) * a.size() * kNonfiniteBlocks, hipMemcpyDeviceToHost, s));
+  if (later) {
+    THCGW_HIP(hipEventCreateWithFlags(&c.ready, hipEventDisableTiming));
+    THCGW_HIP(hipEventRecord(c.ready, s));
+  } else {
+    THCGW_HIP(hipStreamSynchronize(s));
+    c.refuse();
   }
+}
+
+void refuse_singular(const int* info, int total, int nq) {
+  for (int b = 0; b < total; ++b)
+    if (info[b] != 0)
+      throw thcgw::Error(THCGW_ERR_SINGULAR,
+                         "Dyson: (I - V Pi) is singular at (n, q) = (" + std::to_string(b / nq) + ", " +
+                             std::to_string(b % nq) + "), zero pivot " + std::to_string(info[b] - 1));
 }
 
 // In place Pi(iW) -> W(iW) - V; optional Tr(V Pi) and ln|Re det(I - V Pi)| per matrix
@@ -969,7 +1024,7 @@ void check_finite(thcgw_ctx* ctx, const char* entry, std::initializer_list<Finit
 // does not apply run the LU form.  With time reversal (flag 9) only the irreducible q are
 // solved.
 void run_dyson(thcgw_ctx* ctx, c128* PiW, const c128* V, c128* d_trace, double* d_ldet, bool solve, bool pi_first,
-               hipStream_t s) {
+               hipStream_t s, int* pinned_info = nullptr) {
   const int nq = ctx->nk;
   const int total = ctx->nw_half * nq;
   int* info_all = ctx->buf<int>("dy_info", static_cast<size_t>(total));
@@ -982,14 +1037,14 @@ void run_dyson(thcgw_ctx* ctx, c128* PiW, const c128* V, c128* d_trace, double* 
     dyson_matrices(ctx, PiW, V, f, total, d_trace, d_ldet, solve, pi_first, info_all, s);
   }
   if (ctx->deferred) return;  // check_deferred() reads the flags after the stream completes
+  if (pinned_info) {  // looked at by the caller, with refuse_singular
+    THCGW_HIP(hipMemcpyAsync(pinned_info, info_all, sizeof(int) * total, hipMemcpyDeviceToHost, s));
+    return;
+  }
   std::vector<int> info(total);
   THCGW_HIP(hipMemcpyAsync(info.data(), info_all, sizeof(int) * total, hipMemcpyDeviceToHost, s));
   THCGW_HIP(hipStreamSynchronize(s));
-  for (int b = 0; b < total; ++b)
-    if (info[b] != 0)
-      throw thcgw::Error(THCGW_ERR_SINGULAR,
-                         "Dyson: (I - V Pi) is singular at (n, q) = (" + std::to_string(b / nq) + ", " +
-                             std::to_string(b % nq) + "), zero pivot " + std::to_string(info[b] - 1));
+  refuse_singular(info.data(), total, nq);
 }
 
 // Ec from per-(n, q) Tr and ln|Re det| (thc_rpa.icc:130-173, q_weight = 1).
@@ -1320,8 +1375,12 @@ void run_iteration_ibz(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
 
 // ---- one iteration as enqueue + finish (the batch captures the enqueue part) -----------
 
+// finish: the iteration is completed and its results checked here (a single system).  The host does
+// not wait for the device between the stages then: the input check is looked at when Pi is enqueued, before any
+// factorisation, the Dyson flags and Ec at the end.  Each wait left the chip idle for 20 to 30 us.
+// N_mu = 24 iteration 262 -> 180 us, N_mu = 200 2.43 -> 2.35 ms.
 void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128* V, c128* Sig, c128* Wqt, bool want_ec,
-                       bool herm, hipStream_t s) {
+                       bool herm, hipStream_t s, double* Ec = nullptr, bool finish = false) {
   const long M = ctx->M;
   const int total = ctx->nw_half * ctx->nk;
   c128* Pit = Wqt;  // W_qtPQ doubles as Pi_tqPQ scratch (same size)
@@ -1329,9 +1388,23 @@ void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
   c128* dtr = want_ec ? ctx->buf<c128>("ec_tr", total) : nullptr;
   double* dld = want_ec ? ctx->buf<double>("ec_ld", total) : nullptr;
   const long nk = ctx->nk, no = ctx->d.no;
+  // Pinned: the counts of the input check, the Dyson flags and the terms of Ec
+  const size_t at_info = sizeof(int) * thcgw::FINITE_MAX * kNonfiniteBlocks, at_tr = at_info + sizeof(double) * total;
+  char* pin = nullptr;
+  struct Drain {  // no copy into the pinned memory outlives the call
+    hipStream_t s;
+    bool on;
+    ~Drain() {
+      if (on) (void)hipStreamSynchronize(s);
+    }
+  } drain{s, finish};
+  if (finish) pin = ctx->readback(at_tr + (sizeof(c128) + sizeof(double)) * total);
+  PendingFinite inputs;
+  // the check of flag 10 waits for its own result, after this one
+  const bool later = finish && !ctx->herm_g;
   check_finite(ctx, "gw_iteration",
                {{G, ctx->d.nt * nk * no * no, "G_tskij"}, {X, nk * ctx->d.nmu * no, "X_skPa"}, {V, ctx->vq() * M, "V_qPQ"}},
-               s);
+               s, later ? &inputs : nullptr, reinterpret_cast<int*>(pin));
   // With a Hermitian G (flag 10) Pi is Hermitian, and the resolvent form reads its lower triangles
   // only: the other halves are not formed, and mirrored should a chunk need the LU form after all.
   // N_k = 64, N_mu = 480, 80 tau points, mixed precision: 58.8 -> 54.5 ms.
@@ -1344,10 +1417,23 @@ void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
       ~Restore() { c->pi_lower = false; }
     } restore{ctx};
     ctx->pi_lower = lower;
-    run_dyson(ctx, Piw, V, dtr, dld, true, false, s);
+    if (later) inputs.refuse();
+    run_dyson(ctx, Piw, V, dtr, dld, true, false, s, finish ? reinterpret_cast<int*>(pin + at_info) : nullptr);
+  }
+  if (finish && want_ec) {
+    THCGW_HIP(hipMemcpyAsync(pin + at_tr, dtr, sizeof(c128) * total, hipMemcpyDeviceToHost, s));
+    THCGW_HIP(hipMemcpyAsync(pin + at_tr + sizeof(c128) * total, dld, sizeof(double) * total, hipMemcpyDeviceToHost, s));
   }
   run_w_to_tau(ctx, Piw, Wqt, s);
   run_sigma(ctx, G, Wqt, X, Sig, herm, s, true);
+  if (!finish) return;
+  THCGW_HIP(hipStreamSynchronize(s));
+  refuse_singular(reinterpret_cast<const int*>(pin + at_info), total, ctx->nk);
+  if (want_ec) {
+    const auto* tr = reinterpret_cast<const std::complex<double>*>(pin + at_tr);
+    const auto* ld = reinterpret_cast<const double*>(pin + at_tr + sizeof(c128) * total);
+    *Ec = assemble_ec(ctx, std::vector<std::complex<double>>(tr, tr + total), std::vector<double>(ld, ld + total));
+  }
 }
 
 // After a deferred enqueue has completed: Cholesky / LU flags of the Dyson step.
@@ -2041,9 +2127,7 @@ int thcgw_gw_iteration(thcgw_ctx* ctx, const double* G, const double* X, const d
   return guarded(ctx, [&] {
     THCGW_REQUIRE(G && X && V && Sig && Wqt, "thcgw_gw_iteration: null pointer");
     hipStream_t s = S(stream);
-    enqueue_iteration(ctx, C(G), C(X), C(V), Cm(Sig), Cm(Wqt), Ec != nullptr, herm != 0, s);
-    if (Ec) *Ec = finish_ec(ctx, s);
-    THCGW_HIP(hipStreamSynchronize(s));
+    enqueue_iteration(ctx, C(G), C(X), C(V), Cm(Sig), Cm(Wqt), Ec != nullptr, herm != 0, s, Ec, true);
   });
 }
 
