@@ -222,7 +222,7 @@ void hermitize(hipStream_t s, c128* A, int n, long nb, double scale = 1.0);
 void one_minus_trace(hipStream_t s, const c128* A, long sA, int n, c128* trace, int batch);
 void log_re_det(hipStream_t s, const c128* A, long sA, int n, const int* ipiv, double* ldet, int batch);
 // W = P Z - V: rows of Z in the order that undoes the LU column swaps, minus V (nullable).
-void dyson_finish(hipStream_t s, const c128* Z, long sZ, const c128* V, long sV, int vmod, const int* ipiv, int n,
+void dyson_finish(hipStream_t s, const c128* Z, long sZ, const c128* V, long sV, int vmod, int* ipiv, int n,
                   c128* W, long sW, int b0, int batch);
 void copy_batch(hipStream_t s, const c128* src, long sS, int smod, c128* dst, long sD, long per, int b0, int batch);
 void copy_batch(hipStream_t s, const c64* src, long sS, int smod, c64* dst, long sD, long per, int b0, int batch);
