@@ -222,7 +222,7 @@ int thcgw_rpa_ec(thcgw_ctx* ctx, const double* Pi_wqPQ, const double* V_qPQ, dou
  * scr_coulomb_t::update_w + gw_t::evaluate as called by scf_loop
  * (src/methods/SCF/scf_driver.cpp:119-122) and gw_t::rpa_energy (thc_rpa.cpp:22-61).
  * W_qtPQ (caller-owned, nk*nt_half*nmu^2 complex) receives W - V; it also serves as
- * scratch for Pi_tqPQ.  Synchronises the stream. */
+ * scratch for Pi_tqPQ, also in a call that is refused.  Synchronises the stream. */
 int thcgw_gw_iteration(thcgw_ctx* ctx, const double* G_tskij, const double* X_skPa, const double* V_qPQ,
                        double* Sigma_tskij, double* W_qtPQ, double* Ec, int hermitize, void* stream);
 
@@ -432,8 +432,10 @@ int thcgw_set_qsym(thcgw_ctx* ctx, const int* src, const int* perm, const double
  *           chunk's Z Z^H runs; 1 (default) = one stream.  Results are bit-identical.  A
  *           batch's captured graph keeps one stream per system;
  *   flag 10: G(tau, k) is Hermitian (as for any G built from a Hermitian H(k) and Fermi
- *           occupations): the projections X G X^H for chi0 and Sigma form their lower tiles
- *           and mirror them, half the work of that product, and Sigma's back-projection
+ *           occupations): the projections X G X^H for chi0 and Sigma form their lower tiles,
+ *           half the work of that product, and mirror them where whole matrices are read
+ *           (Sigma's k-grid transform, and in an iteration of the resolvent form all of Pi,
+ *           work on the lower triangles only), and Sigma's back-projection
  *           X^H S X of the then Hermitian S is formed as Y + Y^H, Y = X^H L X with L the
  *           lower half of S (Sigma is returned Hermitian).  thcgw_pi, thcgw_sigma and
  *           thcgw_gw_iteration refuse G with max |G - G^H| > 1e-12 max |G| (THCGW_ERR_ARG);
