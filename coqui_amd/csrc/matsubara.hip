@@ -19,7 +19,7 @@
 // Memory traffic is one read of Sigma(iw) and one write of the inverse.  T = 16 with E = n / 16
 // rounded up wastes little padding and leaves 2-8 workgroups per CU to hide the barriers; up to
 // E = 6 (n <= 96) the elements fit the registers (E = 7 spills 90 of them in every column step),
-// and n <= 128 takes T = 32, E = 4.
+// and n <= 128 takes T = 32, E = 4; many matrices of order <= 32 take T = 8, one wave each.
 // N(mu) over N_k = 64 and 80 frequencies (5120 inverses with the transform and the transfer of the
 // traces), batched LU with triangular solves and a row gather through memory -> this kernel:
 // order 16 1.34 -> 0.22 ms, 26 2.18 -> 0.33, 52 5.17 -> 1.00, 78 9.83 -> 2.12, 96 13.2 -> 2.99,
@@ -43,7 +43,7 @@ __device__ __forceinline__ c128 cmul(c128 a, c128 b) { return c128{a.x * b.x - a
 enum MatsubaraJob { INVERSE, TRACES, DYSON };
 
 template <int T, int E, MatsubaraJob JOB>
-__global__ __launch_bounds__(T* T) __attribute__((amdgpu_waves_per_eu(T == 32 ? 4 : E <= 4 ? 4 : 2)))
+__global__ __launch_bounds__(T* T) __attribute__((amdgpu_waves_per_eu(T == 16 && E > 4 ? 2 : 4)))
 void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn, double beta,
                               double mu, int nk, int n, c128* Out, c128* tr_out, int* info, double* ldet, bool keep) {
   constexpr int N = T * E, NW = T * T / 64;
@@ -119,7 +119,9 @@ void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, cons
       best = fmax(best, __hiloint2double(static_cast<int>(static_cast<unsigned>(__double2hiint(mag)) | off),
                                          static_cast<int>(lo)));
     }
-    if (T == 16) best = swap_with<16>(best, MaxOp{});  // four thread rows per wave, at lanes c, c + 16, c + 32, c + 48
+    // 64 / T thread rows per wave, T lanes apart
+    if (T == 8) best = ror_with<8>(best, MaxOp{});
+    if (T <= 16) best = swap_with<16>(best, MaxOp{});
     best = swap_with<32>(best, MaxOp{});
     if (c == cc) {
 #pragma unroll
@@ -284,6 +286,15 @@ void launch_inverse(hipStream_t s, const InverseArgs& x, int n, int count) {
     THCGW_HIP(hipGetLastError());
   };
   using std::integral_constant;
+  // Many small matrices: one wave each (T = 8), whose barriers cost nothing.  Electron number, T = 16 -> 8, on 5120
+  // matrices of order 16 163 -> 138 us, 24 249 -> 203, 32 316 -> 279; on 160 of order 16 104 -> 103,
+  // 24 111 -> 113, 32 117 -> 127: the line lies at one matrix per SIMD.
+  if (n <= 32 && count >= 1024) {
+    if (n <= 16) go(integral_constant<int, 8>{}, integral_constant<int, 2>{});
+    else if (n <= 24) go(integral_constant<int, 8>{}, integral_constant<int, 3>{});
+    else go(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+    return;
+  }
   switch ((n + 15) / 16) {
     case 1: go(integral_constant<int, 16>{}, integral_constant<int, 1>{}); break;
     case 2: go(integral_constant<int, 16>{}, integral_constant<int, 2>{}); break;

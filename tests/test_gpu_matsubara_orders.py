@@ -69,3 +69,36 @@ def test_singular_matrix_is_reported(no):
         ctx.dyson_g(z, sig, 0.0, S=z)
     assert e.value.code == 3
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 15, 16, 17, 24, 25, 31, 32, 33])
+def test_many_small_matrices(n):
+    """The same kernel with one wave per matrix (order <= 32, 1024 matrices or more): G of 2560
+    matrices and W of 1344, equal at every frequency."""
+    import torch
+
+    from coqui_amd import IAFT, ThcGW
+
+    rng = np.random.default_rng(n)
+    ia = IAFT.from_table(BETA, TABLE)
+    nk = 64
+    ctx = ThcGW((4, 4, 4), n, n, ia)
+    assert ctx.nw_half * nk >= 1024
+    F = _herm(rng, 1, nk, n, n) / np.sqrt(n)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.complex128)).cuda()  # noqa: E731
+    g, _ = ctx.dyson_g(dev(F), dev(np.zeros((ia.nt, 1, nk, n, n))), 0.13)
+    iw = 1j * ia.wn_mesh_f * np.pi / BETA + 0.13
+    X = iw[:, None, None, None] * np.eye(n) - F[0]
+    G = np.tensordot(ia.Ttw_ff * (np.sqrt(2.0) / BETA), np.linalg.inv(X), 1)
+    tol = 16 * n * EPS * float(np.max(np.linalg.cond(X)))
+    assert np.max(np.abs(g.cpu().numpy()[:, 0] - G)) <= tol * np.max(np.abs(G))
+
+    eye = np.eye(n)
+    A = rng.standard_normal((nk, n, n)) + 1j * rng.standard_normal((nk, n, n))
+    P = np.broadcast_to(eye - A, (ctx.nw_half, nk, n, n))
+    PiW = dev(P)
+    ctx.dyson_w(PiW, dev(np.broadcast_to(eye, (nk, n, n))))
+    ref = np.linalg.inv(A) - eye
+    tol = 16 * n * EPS * float(np.max(np.linalg.cond(A)))
+    assert np.max(np.abs(PiW.cpu().numpy() - ref)) <= tol * (1 + np.max(np.abs(ref)))
+    ctx.close()
