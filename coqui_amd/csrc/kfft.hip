@@ -272,7 +272,7 @@ __global__ __launch_bounds__(KT) void sigma_kfft_kernel(const TG* __restrict__ G
 // without a specialised kernel and as an independent check of the specialised ones.  Bound by
 // the LDS reads, one complex value per term.  One thread per column with a sincospi per term took
 // 20 us for one tau slice of the 2 x 2 x 1 grid at N_mu = 24 (nine workgroups); the 20 slices of
-// a 40-point table now take 6.8 us in one launch, and the N_mu = 24 iteration 0.37 ms instead of 1.18.
+// a 40-point table now take 6.8 us in one launch, and the N_mu = 24 iteration lost 0.8 of its 1.18 ms.
 // ---------------------------------------------------------------------------------
 constexpr int FB_C = 16;   // columns per workgroup
 constexpr int FB_NK = 16;  // largest N_k
