@@ -500,6 +500,11 @@ int choose_dyson_chunk(thcgw_ctx* ctx, int total) {
   return (total + nchunks - 1) / nchunks;
 }
 
+// Whether the LU form solves this system's matrices in registers (dyson_small.hip).
+bool dyson_small_form(const thcgw_ctx* ctx, bool solve) {
+  return thcgw::dyson_small_fits(ctx->d.nmu, static_cast<long>(ctx->nw_half) * ctx->vq(), solve);
+}
+
 // One chunk of matrices b0 .. b0+cb of the LU form: A = I - V Pi (or I - Pi V) -> getrf ->
 // ln|Re det|; with solve, (I - V Pi) Y = V and W - V = Y - V replace getri + GEMM
 // (scr_coulomb_t.cpp:180-196, thc_rpa.icc:141-163).
@@ -507,21 +512,14 @@ void dyson_chunk_lu(thcgw_ctx* ctx, c128* PiW, const c128* V, int b0, int cb, c1
                     bool solve, bool pi_first, c128* LU, c128* Z, int* ipiv, int* info, hipStream_t s) {
   const int n = ctx->d.nmu, nq = ctx->vq();
   const long M = ctx->M;
-  if (!pi_first)
-    thcgw::zgemm(s, thcgw::OP_N, thcgw::OP_N, n, n, n, kMinusOne, thcgw::bp(V, M, nq, 1, b0), n,
-                 thcgw::bp(PiW + static_cast<long>(b0) * M, M), n, kZero, LU, M, n, cb, kOne);
-  else
-    thcgw::zgemm(s, thcgw::OP_N, thcgw::OP_N, n, n, n, kMinusOne, thcgw::bp(PiW + static_cast<long>(b0) * M, M), n,
-                 thcgw::bp(V, M, nq, 1, b0), n, kZero, LU, M, n, cb, kOne);
-  if (thcgw::matsubara_inverse_fits(n)) {
-    // Small orders: W - V = [(I - V Pi)^-1 - I] V with the inverse formed in registers, three launches
-    // instead of about 15 whose panels and triangles have no work for the chip.  The whole step, LU
-    // -> inverse: 84 matrices of order 24 169 -> 110 us, 64 275 -> 177, 96 442 -> 273, 128 613 -> 411;
-    // 1344 matrices 223 -> 142, 689 -> 425, 1708 -> 1159, 2874 -> 2402.
-    thcgw::dyson_inverse(s, LU, n, cb, solve, d_trace ? d_trace + b0 : nullptr, d_ldet ? d_ldet + b0 : nullptr, info);
-    if (solve)
-      thcgw::zgemm(s, thcgw::OP_N, thcgw::OP_N, n, n, n, kOne, thcgw::bp(LU, M), n, thcgw::bp(V, M, nq, 1, b0), n, kZero,
-                   PiW + static_cast<long>(b0) * M, M, n, cb);
+  c128* P = PiW + static_cast<long>(b0) * M;
+  const bool small = dyson_small_form(ctx, solve);  // takes A - I, leaves Z and ipiv alone
+  const thcgw::BatchPtr v = thcgw::bp(V, M, nq, 1, b0), p = thcgw::bp(P, M);
+  thcgw::zgemm(s, thcgw::OP_N, thcgw::OP_N, n, n, n, kMinusOne, pi_first ? p : v, n, pi_first ? v : p, n, kZero, LU, M,
+               n, cb, small ? kZero : kOne);
+  if (small) {
+    thcgw::dyson_small(s, LU, V, nq, b0, n, cb, solve ? P : nullptr, d_trace ? d_trace + b0 : nullptr,
+                       d_ldet ? d_ldet + b0 : nullptr, info);
     return;
   }
   if (d_trace) thcgw::one_minus_trace(s, LU, M, n, d_trace + b0, cb);
@@ -737,7 +735,9 @@ void dyson_resolvent_lanes(thcgw_ctx* ctx, c128* PiW, const c128* V, const VFact
     if (!any_nonzero(info_all + b0(c), cbn(c), ls)) {
       resolvent_back(ctx, PiW, V, f.ldv, b0(c), cbn(c), d_ldet, solve, LU[l], Z[l], ls);
     } else {
-      int* ipiv = ctx->buf<int>(l ? "dy_ipiv1" : "dy_ipiv", static_cast<size_t>(CH) * n);
+      int* ipiv = dyson_small_form(ctx, solve)
+                      ? nullptr
+                      : ctx->buf<int>(l ? "dy_ipiv1" : "dy_ipiv", static_cast<size_t>(CH) * n);
       if (ctx->pi_lower) thcgw::mirror_lower(ls, PiW + static_cast<long>(b0(c)) * M, M, n, cbn(c));
       dyson_chunk_lu(ctx, PiW, V, b0(c), cbn(c), d_trace, d_ldet, solve, pi_first, LU[l], Z[l], ipiv, info_all + b0(c),
                      ls);
@@ -779,8 +779,9 @@ void dyson_matrices(thcgw_ctx* ctx, c128* PiW, const c128* V, const VFactors& f,
       if (!Z) Z = ctx->buf<c128>("dy_z", static_cast<size_t>(CH) * M);
       if (dyson_chunk_hpd(ctx, PiW, V, f.Lv, b0, cb, d_trace, d_ldet, solve, LU, Z, info_all + b0, s)) continue;
     }
-    if (!ipiv) ipiv = ctx->buf<int>("dy_ipiv", static_cast<size_t>(CH) * n);
-    if (solve && !Z) Z = ctx->buf<c128>("dy_z", static_cast<size_t>(CH) * M);
+    const bool small = dyson_small_form(ctx, solve);
+    if (!small && !ipiv) ipiv = ctx->buf<int>("dy_ipiv", static_cast<size_t>(CH) * n);
+    if (!small && solve && !Z) Z = ctx->buf<c128>("dy_z", static_cast<size_t>(CH) * M);
     if (ctx->pi_lower) thcgw::mirror_lower(s, PiW + static_cast<long>(b0) * M, M, n, cb);
     dyson_chunk_lu(ctx, PiW, V, b0, cb, d_trace, d_ldet, solve, pi_first, LU, Z, ipiv, info_all + b0, s);
   }

@@ -1,7 +1,6 @@
-// Inverses of order <= 128, one workgroup per matrix: of the Matsubara matrices X(n, k) =
-// (iw_n + mu) S_k - H0_k - F_k - Sigma(iw_n, k), or only the traces Tr[X^-1 S_k] that the electron
-// number needs (simple_dyson.cpp:65-78,130-172), and of the matrices 1 - V Pi of the Dyson
-// equation for W with the trace and the determinant that the RPA energy needs.
+// Inverses of the Matsubara matrices X(n, k) = (iw_n + mu) S_k - H0_k - F_k - Sigma(iw_n, k) of
+// order <= 128, one workgroup per matrix, or only the traces Tr[X^-1 S_k] that the electron
+// number needs (simple_dyson.cpp:65-78,130-172).
 //
 // The matrix is formed in registers and inverted there in place by Gauss-Jordan elimination
 // with partial pivoting: thread (r, c) of T x T holds the E x E elements (r + a T, c + b T).
@@ -38,20 +37,18 @@ namespace {
 
 __device__ __forceinline__ c128 cmul(c128 a, c128 b) { return c128{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
 
-// INVERSE: Out = X^-1.  TRACES: tr_out = Tr[X^-1 S].  DYSON: X = Out, replaced by X^-1 - 1 if keep is
-// set; tr_out = Tr[1 - X] and ldet = ln |Re det X| where given.
-enum MatsubaraJob { INVERSE, TRACES, DYSON };
+// INVERSE: Out = X^-1.  TRACES: tr_out = Tr[X^-1 S].
+enum MatsubaraJob { INVERSE, TRACES };
 
 template <int T, int E, MatsubaraJob JOB>
 __global__ __launch_bounds__(T* T) __attribute__((amdgpu_waves_per_eu(T == 16 && E > 4 ? 2 : 4)))
 void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn, double beta,
-                              double mu, int nk, int n, c128* Out, c128* tr_out, int* info, double* ldet, bool keep) {
+                              double mu, int nk, int n, c128* Out, c128* tr_out, int* info) {
   constexpr int N = T * E, NW = T * T / 64;
   __shared__ c128 colv[2][N], rowv[N], scale[N];
   __shared__ double key[2][T * T / 64];
   __shared__ int perm[N], rowpos[N];
-  __shared__ double red[4][NW];
-  __shared__ c128 pivot[JOB == DYSON ? N : 1];
+  __shared__ double red[2][NW];
   __shared__ int bad;  // first zero or non-finite pivot column + 1
   const long b = blockIdx.x, m = static_cast<long>(n) * n;
   const long kofs = (b % nk) * m;
@@ -69,22 +66,7 @@ void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, cons
   };
 
   c128 v[E][E];
-  if constexpr (JOB == DYSON) {
-    double re = 0.0, im = 0.0;
-#pragma unroll
-    for (int a = 0; a < E; ++a)
-#pragma unroll
-      for (int q = 0; q < E; ++q) {
-        const int i = r + a * T, j = c + q * T;
-        v[a][q] = (i < n && j < n) ? Out[b * m + static_cast<long>(i) * n + j] : c128{0.0, 0.0};
-        if (i == j && i < n) {
-          re += 1.0 - v[a][q].x;
-          im -= v[a][q].y;
-        }
-      }
-    block_sum(re, red[0]);
-    block_sum(im, red[1]);
-  } else {
+  {
     const double wi = static_cast<double>(wn[b / nk]) * M_PI / beta;
 #pragma unroll
     for (int a = 0; a < E; ++a)
@@ -159,7 +141,6 @@ void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, cons
       if (c == 0) {
         colv[buf][p] = c128{0.0, 0.0};  // the stored row stays as it is
         scale[p] = s;
-        if constexpr (JOB == DYSON) pivot[k] = piv;
         const bool ok = isfinite(piv.x) && isfinite(piv.y) && (piv.x != 0.0 || piv.y != 0.0);
         if (!ok && bad == 0) bad = k + 1;
         perm[k] = p;
@@ -233,36 +214,13 @@ void matsubara_inverse_kernel(const c128* H0, const c128* F, const c128* S, cons
     if (threadIdx.x == 0) tr_out[b] = c128{total(red[0]), total(red[1])};
   } else {
     c128* Ob = Out + b * m;
-    if (JOB == INVERSE || keep) {
 #pragma unroll
-      for (int a = 0; a < E; ++a)
+    for (int a = 0; a < E; ++a)
 #pragma unroll
-        for (int q = 0; q < E; ++q) {
-          const int i = r + a * T, j = c + q * T;
-          if (i < n && j < n) {
-            const int row = rowpos[i], col = perm[j];
-            const double one = JOB == DYSON && row == col ? 1.0 : 0.0;
-            Ob[static_cast<long>(row) * n + col] = c128{v[a][q].x - one, v[a][q].y};
-          }
-        }
-    }
-  }
-  if constexpr (JOB == DYSON) {
-    if (tr_out || ldet) {
-      double la = 0.0, ph = 0.0;  // a swap of rows turns the phase by pi, which |Re det| does not see
-      if (static_cast<int>(threadIdx.x) < n) {
-        const c128 p = pivot[threadIdx.x];
-        la = log(hypot(p.x, p.y));
-        ph = atan2(p.y, p.x);
+      for (int q = 0; q < E; ++q) {
+        const int i = r + a * T, j = c + q * T;
+        if (i < n && j < n) Ob[static_cast<long>(rowpos[i]) * n + perm[j]] = v[a][q];
       }
-      block_sum(la, red[2]);
-      block_sum(ph, red[3]);
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        if (tr_out) tr_out[b] = c128{total(red[0]), total(red[1])};
-        if (ldet) ldet[b] = total(red[2]) + log(fabs(cos(total(red[3]))));
-      }
-    }
   }
 }
 
@@ -273,8 +231,6 @@ struct InverseArgs {
   int nk;
   c128 *Out, *tr;
   int* info;
-  double* ldet;
-  bool keep;
 };
 
 template <MatsubaraJob JOB>
@@ -282,7 +238,7 @@ void launch_inverse(hipStream_t s, const InverseArgs& x, int n, int count) {
   auto go = [&](auto t, auto e) {
     constexpr int T = t, E = e;
     hipLaunchKernelGGL((matsubara_inverse_kernel<T, E, JOB>), dim3(count), dim3(T * T), 0, s, x.H0, x.F, x.S, x.Sw, x.wn,
-                       x.beta, x.mu, x.nk, n, x.Out, x.tr, x.info, x.ldet, x.keep);
+                       x.beta, x.mu, x.nk, n, x.Out, x.tr, x.info);
     THCGW_HIP(hipGetLastError());
   };
   using std::integral_constant;
@@ -317,16 +273,9 @@ void matsubara_inverse(hipStream_t s, const c128* H0, const c128* F, const c128*
   const long count = static_cast<long>(nw) * nk;
   THCGW_REQUIRE(count < (1L << 30), "Dyson for G: too many matrices");
   if (count == 0) return;
-  const InverseArgs x{H0, F, S, Sw, wn, beta, mu, nk, Out, tr, info, nullptr, true};
+  const InverseArgs x{H0, F, S, Sw, wn, beta, mu, nk, Out, tr, info};
   if (tr) launch_inverse<TRACES>(s, x, no, static_cast<int>(count));
   else launch_inverse<INVERSE>(s, x, no, static_cast<int>(count));
-}
-
-void dyson_inverse(hipStream_t s, c128* A, int n, int batch, bool keep, c128* tr, double* ldet, int* info) {
-  THCGW_REQUIRE(matsubara_inverse_fits(n), "dyson_inverse: order must be in [1, 128]");
-  if (batch <= 0) return;
-  const InverseArgs x{nullptr, nullptr, nullptr, nullptr, nullptr, 0.0, 0.0, 1, A, tr, info, ldet, keep};
-  launch_inverse<DYSON>(s, x, n, batch);
 }
 
 }  // namespace thcgw

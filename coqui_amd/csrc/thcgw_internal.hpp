@@ -208,12 +208,16 @@ void hessenberg_traces(hipStream_t s, const c128* H, const c128* rsub, const lon
 // matsubara.hip: Out[n, k] = [(iw_n + mu) S_k - H0_k - F_k - Sw[n, k]]^-1 or tr[n, k] = Tr of that
 // inverse times S_k (exactly one of Out and tr; S and H0 nullable) for orders up to 128;
 // info[n nk + k] = first zero or non-finite pivot column + 1, or 0
-// dyson_inverse: A[b] -> A[b]^-1 - 1 (keep) for packed matrices of order n <= 128, tr[b] = Tr[1 - A[b]] and
-// ldet[b] = ln |Re det A[b]| where given, info[b] = first lost pivot + 1.
 bool matsubara_inverse_fits(int no);
 void matsubara_inverse(hipStream_t s, const c128* H0, const c128* F, const c128* S, const c128* Sw, const long* wn,
                        double beta, double mu, int nw, int nk, int no, c128* Out, c128* tr, int* info);
-void dyson_inverse(hipStream_t s, c128* A, int n, int batch, bool keep, c128* tr, double* ldet, int* info);
+
+// dyson_small.hip: for matrices A[b] = 1 + D[b] of order n <= 96 (packed) and V[(b0 + b) % vmod]:
+// W[b] = A^-1 V - V (W may be null), tr[b] = -Tr D[b] and ldet[b] = ln |Re det A[b]| where given, info[b] = first lost pivot + 1.
+// dyson_small_fits: the rule of the Dyson step for a system of `total` matrices.
+bool dyson_small_fits(int n, long total, bool solve);
+void dyson_small(hipStream_t s, const c128* D, const c128* V, int vmod, int b0, int n, int batch, c128* W, c128* tr,
+                 double* ldet, int* info);
 
 // misc.hip
 void scale_mo(hipStream_t s, const c128* C, const double* E, const double* tau, double mu, double beta, int nt, int nk,
