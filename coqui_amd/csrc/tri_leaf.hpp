@@ -22,11 +22,11 @@ enum TriLeaf {
 // What bounds it: memory where there are thousands of vectors (batch x m), the chain of nb steps
 // where there are few.  16 lanes per vector give a hundred rows as many waves as one thread
 // per vector gives 1600, and keep a vector's elements in 8 registers instead of 128.
-// With L^H the product is rounded before it is subtracted: the forms that hold V^-1 multiply a
-// change in the last bits of V's factor by the condition of V.
+// A product is rounded before it is subtracted: one rounding at the size of the element, and the forms
+// that hold V^-1 multiply a change in the last bits of V's factor by the condition of V.
 // Against one thread per vector with the triangle read from LDS for each (per launch, order 32):
 // L^H with at most 1600 rows on 4 matrices 23.3 -> 6.2 us; all leaves of the LU form on 168 matrices
-// of order 200 616 -> 337 us, on 164 of order 800 4.30 -> 2.87 ms.  Order-64 leaves (100 us where two of
+// of order 200 616 -> 363 us, on 164 of order 800 4.30 -> 3.14 ms.  Order-64 leaves (100 us where two of
 // order 32 take 32 each and the product between them the rest) gained 1% on the latter and lost 4%
 // on order 24.
 template <typename RC, int NB, int V, TriLeaf KIND>
@@ -100,10 +100,8 @@ __global__ __launch_bounds__(256) void tri_leaf_kernel(const RC* A, long sA, int
               x[v][e].x -= xc[v].x * f[e].x + xc[v].y * f[e].y;
               x[v][e].y -= xc[v].y * f[e].x - xc[v].x * f[e].y;
             } else {
-              x[v][e].x -= xc[v].x * f[e].x;
-              x[v][e].y -= xc[v].x * f[e].y;
-              x[v][e].x += xc[v].y * f[e].y;
-              x[v][e].y -= xc[v].y * f[e].x;
+              x[v][e].x -= fma(xc[v].x, f[e].x, -(xc[v].y * f[e].y));
+              x[v][e].y -= fma(xc[v].x, f[e].y, xc[v].y * f[e].x);
             }
           }
     }
@@ -129,7 +127,7 @@ __global__ __launch_bounds__(256) void tri_leaf_kernel(const RC* A, long sA, int
 // Four vectors per 16 lanes read the triangle once for all four; below 16384 vectors (4 waves per SIMD
 // with one each) more waves are worth more: L^H with at most 1600 rows on 4 matrices 6.2 us with
 // one, 10.4 with four; order 24 on 84 matrices 4.8 and 6.7; order 200 on 168 matrices, the narrow blocks
-// below the line included, 337 us by this rule, 355 with four everywhere.
+// below the line included, 5% less by this rule than with four everywhere.
 template <TriLeaf KIND, int NB, typename RC>
 void tri_leaf(hipStream_t s, const RC* A, long sA, int lda, RC* T, long sT, int ldt, int m, int nb, int batch) {
   auto go = [&](auto v) {
