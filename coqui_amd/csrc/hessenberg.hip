@@ -192,7 +192,7 @@ void hessenberg_kernel(const c128* H0, const c128* F, const c128* Sw, int nk, in
 // bad[b] = 1 where the result is not finite.
 //
 // What bounds it: the read of H, n^2 / 2 complex numbers per matrix.  5120 matrices of order 78: 55 us,
-// 4.6 TB/s, against 1.26 ms for the inverses in registers and 156 us for an elimination of z - H with
+// 4.6 TB/s, against 1.36 ms for the inverses in registers and 156 us for an elimination of z - H with
 // pivoting (whose selects and divisions cost more than the read).
 template <int E>
 __global__ __launch_bounds__(64) void hessenberg_trace_kernel(const c128* H, const c128* rsub, const long* wn,
