@@ -10,6 +10,7 @@
 #include <complex>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -405,6 +406,9 @@ void check_herm_g(thcgw_ctx* ctx, const c128* G, hipStream_t s, int nk_g = 0) {
     throw thcgw::Error(THCGW_ERR_ARG, "flag 10 (Hermitian G): G is not Hermitian, max |G - G^H| = " + sci(diff) +
                                           " against max |G| = " + sci(mag));
 }
+
+// Called by a stage when its first kernels are enqueued, before the first one that writes the caller's array.
+using BeforeWrite = std::function<void()>;
 
 // lower: of each Pi(q) only the lower triangle (flag 10); the rest of Pi keeps what it held.
 void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s, bool lower = false) {
@@ -950,20 +954,32 @@ struct FiniteArg {
 };
 constexpr int kNonfiniteBlocks = 1024;  // 16 waves per CU
 
+// A point of a stream that the host can wait for.
+struct Event {
+  hipEvent_t e = nullptr;
+  Event() = default;
+  Event(const Event&) = delete;
+  Event& operator=(const Event&) = delete;
+  ~Event() {
+    if (e) (void)hipEventDestroy(e);
+  }
+  void record(hipStream_t s) {
+    if (!e) THCGW_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    THCGW_HIP(hipEventRecord(e, s));
+  }
+  void wait() const {  // at once where nothing was recorded
+    if (e) THCGW_HIP(hipEventSynchronize(e));
+  }
+};
+
 // A check whose counts are on their way to pinned memory: refuse() waits for them.
 struct PendingFinite {
   std::string entry;
   std::vector<FiniteArg> a;
   const int* h = nullptr;
-  hipEvent_t ready = nullptr;
-  PendingFinite() = default;
-  PendingFinite(const PendingFinite&) = delete;
-  PendingFinite& operator=(const PendingFinite&) = delete;
-  ~PendingFinite() {
-    if (ready) (void)hipEventDestroy(ready);
-  }
+  Event ready;
   void refuse() const {
-    if (ready) THCGW_HIP(hipEventSynchronize(ready));
+    ready.wait();
     for (size_t i = 0; i < a.size(); ++i) {
       long bad = 0;
       for (int b = 0; b < kNonfiniteBlocks; ++b) bad += h[i * kNonfiniteBlocks + b];
@@ -1002,8 +1018,7 @@ void check_finite(thcgw_ctx* ctx, const char* entry, std::initializer_list<Finit
   c.h = later ? pinned : h.data();
   THCGW_HIP(hipMemcpyAsync(const_cast<int*>(c.h), cnt, sizeof(int) * a.size() * kNonfiniteBlocks, hipMemcpyDeviceToHost, s));
   if (later) {
-    THCGW_HIP(hipEventCreateWithFlags(&c.ready, hipEventDisableTiming));
-    THCGW_HIP(hipEventRecord(c.ready, s));
+    c.ready.record(s);
   } else {
     THCGW_HIP(hipStreamSynchronize(s));
     c.refuse();
@@ -1074,7 +1089,7 @@ void fetch_ec_terms(thcgw_ctx* ctx, const c128* d_tr, const double* d_ld, std::v
 }
 
 void run_sigma_f32(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c128* Sig, bool herm,
-                   hipStream_t s) {
+                   hipStream_t s, const BeforeWrite& before_write) {
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
   const long gs = static_cast<long>(nk) * no * no;
@@ -1098,6 +1113,7 @@ void run_sigma_f32(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X
     thcgw::sigma_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP, c2 > 0 ? GN : nullptr,
                       Wqt + static_cast<long>(i0) * M, static_cast<long>(nth) * M, SP, c2 > 0 ? SN : nullptr, M, scale,
                       ctx->herm_g ? nmu : 0, c, c2);
+    if (i0 == 0 && before_write) before_write();
     project_a2p_f32(ctx, s, X64, SP, Sig + i0 * gs, static_cast<long>(c) * nk, Ab, ctx->herm_g);
     if (c2 > 0)
       project_a2p_f32(ctx, s, X64, SN, Sig + (nt - i0 - c2) * gs, static_cast<long>(c2) * nk, Ab, ctx->herm_g);
@@ -1108,9 +1124,9 @@ void run_sigma_f32(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X
 
 // g_checked: the caller's run_pi has checked the same G for flag 10.
 void run_sigma(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c128* Sig, bool herm, hipStream_t s,
-               bool g_checked = false) {
+               bool g_checked = false, const BeforeWrite& before_write = {}) {
   if (!g_checked) check_herm_g(ctx, G, s);
-  if (ctx->precision != 0) return run_sigma_f32(ctx, G, Wqt, X, Sig, herm, s);
+  if (ctx->precision != 0) return run_sigma_f32(ctx, G, Wqt, X, Sig, herm, s, before_write);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
   const long gs = static_cast<long>(nk) * no * no;
@@ -1131,6 +1147,7 @@ void run_sigma(thcgw_ctx* ctx, const c128* G, const c128* Wqt, const c128* X, c1
     thcgw::sigma_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP, c2 > 0 ? GN : nullptr,
                       Wqt + static_cast<long>(i0) * M, static_cast<long>(nth) * M, SP, c2 > 0 ? SN : nullptr, M, scale,
                       ctx->herm_g ? nmu : 0, c, c2);
+    if (i0 == 0 && before_write) before_write();
     if (ctx->herm_g) {
       project_a2p_herm(ctx, s, X, SP, Sig + i0 * gs, static_cast<long>(c) * nk, Ab);
       if (c2 > 0) project_a2p_herm(ctx, s, X, SN, Sig + (nt - i0 - c2) * gs, static_cast<long>(c2) * nk, Ab);
@@ -1376,10 +1393,11 @@ void run_iteration_ibz(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
 
 // ---- one iteration as enqueue + finish (the batch captures the enqueue part) -----------
 
-// finish: the iteration is completed and its results checked here (a single system).  The host does
-// not wait for the device between the stages then: the input check is looked at when Pi is enqueued, before any
-// factorisation, the Dyson flags and Ec at the end.  Each wait left the chip idle for 20 to 30 us.
-// N_mu = 24 iteration 262 -> 180 us, N_mu = 200 2.43 -> 2.35 ms.
+// finish: the iteration is completed and its results checked here (a single system).  In the plain form
+// without flag 10 the host never waits for an idle device then: it looks at the input check when Pi is
+// enqueued, at the Dyson flags when the first projections for Sigma are, before anything is
+// written to Sigma, and at Ec at the end.  (The Cholesky forms read the flags of every chunk, flag 10 the
+// result of its check.)  A wait between two stages left the chip idle for 20 to 30 us.
 void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128* V, c128* Sig, c128* Wqt, bool want_ec,
                        bool herm, hipStream_t s, double* Ec = nullptr, bool finish = false) {
   const long M = ctx->M;
@@ -1421,15 +1439,19 @@ void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
     if (later) inputs.refuse();
     run_dyson(ctx, Piw, V, dtr, dld, true, false, s, finish ? reinterpret_cast<int*>(pin + at_info) : nullptr);
   }
+  Event solved;
+  if (finish) solved.record(s);
   if (finish && want_ec) {
     THCGW_HIP(hipMemcpyAsync(pin + at_tr, dtr, sizeof(c128) * total, hipMemcpyDeviceToHost, s));
     THCGW_HIP(hipMemcpyAsync(pin + at_tr + sizeof(c128) * total, dld, sizeof(double) * total, hipMemcpyDeviceToHost, s));
   }
   run_w_to_tau(ctx, Piw, Wqt, s);
-  run_sigma(ctx, G, Wqt, X, Sig, herm, s, true);
+  run_sigma(ctx, G, Wqt, X, Sig, herm, s, true, finish ? BeforeWrite([&] {
+    solved.wait();
+    refuse_singular(reinterpret_cast<const int*>(pin + at_info), total, ctx->nk);
+  }) : BeforeWrite());
   if (!finish) return;
   THCGW_HIP(hipStreamSynchronize(s));
-  refuse_singular(reinterpret_cast<const int*>(pin + at_info), total, ctx->nk);
   if (want_ec) {
     const auto* tr = reinterpret_cast<const std::complex<double>*>(pin + at_tr);
     const auto* ld = reinterpret_cast<const double*>(pin + at_tr + sizeof(c128) * total);
