@@ -411,7 +411,8 @@ void check_herm_g(thcgw_ctx* ctx, const c128* G, hipStream_t s, int nk_g = 0) {
 using BeforeWrite = std::function<void()>;
 
 // lower: of each Pi(q) only the lower triangle (flag 10); the rest of Pi keeps what it held.
-void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s, bool lower = false) {
+void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s, bool lower,
+                const BeforeWrite& before_write) {
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
   const Proj proj = lower ? PROJ_LOWER : ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
@@ -426,14 +427,16 @@ void run_pi_f32(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStrea
     const int c = std::min(P, nth - i0);
     project_p2a_f32(ctx, s, X64, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
     project_p2a_f32(ctx, s, X64, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, proj);
+    if (i0 == 0 && before_write) before_write();
     thcgw::pi_kfft_f32(s, ctx->d.kgrid, ctx->force_fallback, GP, GN, Pi + static_cast<long>(i0) * nk * M, M, scale, c,
                        lower ? nmu : 0);
   }
 }
 
-void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s, bool lower = false) {
+void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t s, bool lower = false,
+            const BeforeWrite& before_write = {}) {
   check_herm_g(ctx, G, s);
-  if (ctx->precision != 0) return run_pi_f32(ctx, G, X, Pi, s, lower);
+  if (ctx->precision != 0) return run_pi_f32(ctx, G, X, Pi, s, lower, before_write);
   const int nk = ctx->nk, no = ctx->d.no, nmu = ctx->d.nmu, nt = ctx->d.nt, nth = ctx->nt_half;
   const long M = ctx->M;
   const Proj proj = lower ? PROJ_LOWER : ctx->herm_g ? PROJ_MIRROR : PROJ_FULL;
@@ -448,6 +451,7 @@ void run_pi(thcgw_ctx* ctx, const c128* G, const c128* X, c128* Pi, hipStream_t 
     project_p2a(ctx, s, X, G + i0 * gs, GP, static_cast<long>(c) * nk, Ab, proj);
     // G(beta - tau_i) = G[nt-1-i] for i in [i0, i0+c): tau slots [nt-i0-c, nt-i0), reversed
     project_p2a(ctx, s, X, G + (nt - i0 - c) * gs, GN, static_cast<long>(c) * nk, Ab, proj);
+    if (i0 == 0 && before_write) before_write();
     thcgw::pi_kfft(s, ctx->d.kgrid, ctx->force_fallback, GP, GN, Pi + static_cast<long>(i0) * nk * M, M, scale, c,
                    lower ? nmu : 0);
   }
@@ -1394,9 +1398,9 @@ void run_iteration_ibz(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
 // ---- one iteration as enqueue + finish (the batch captures the enqueue part) -----------
 
 // finish: the iteration is completed and its results checked here (a single system).  In the plain form
-// without flag 10 the host never waits for an idle device then: it looks at the input check when Pi is
-// enqueued, at the Dyson flags when the first projections for Sigma are, before anything is
-// written to Sigma, and at Ec at the end.  (The Cholesky forms read the flags of every chunk, flag 10 the
+// without flag 10 the host never waits for an idle device then: it looks at the input check when the first
+// projections for Pi are enqueued, at the Dyson flags when those for Sigma are, each before anything is
+// written to the caller's arrays, and at Ec at the end.  (The Cholesky forms read the flags of every chunk, flag 10 the
 // result of its check.)  A wait between two stages left the chip idle for 20 to 30 us.
 void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128* V, c128* Sig, c128* Wqt, bool want_ec,
                        bool herm, hipStream_t s, double* Ec = nullptr, bool finish = false) {
@@ -1428,7 +1432,7 @@ void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
   // only: the other halves are not formed, and mirrored should a chunk need the LU form after all.
   // N_k = 64, N_mu = 480, 80 tau points, mixed precision: 58.8 -> 54.5 ms.
   const bool lower = ctx->herm_g && ctx->dyson_algo == 2 && !ctx->trev && !ctx->sym;
-  run_pi(ctx, G, X, Pit, s, lower);
+  run_pi(ctx, G, X, Pit, s, lower, later ? BeforeWrite([&] { inputs.refuse(); }) : BeforeWrite());
   run_tau_to_w(ctx, Pit, Piw, s, 0, lower);
   {
     struct Restore {
@@ -1436,7 +1440,6 @@ void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
       ~Restore() { c->pi_lower = false; }
     } restore{ctx};
     ctx->pi_lower = lower;
-    if (later) inputs.refuse();
     run_dyson(ctx, Piw, V, dtr, dld, true, false, s, finish ? reinterpret_cast<int*>(pin + at_info) : nullptr);
   }
   Event solved;

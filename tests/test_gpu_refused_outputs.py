@@ -1,4 +1,5 @@
-"""What a refused iteration leaves in the caller's arrays: Sigma stays to the bit when 1 - V Pi is singular."""
+"""What a refused iteration leaves in the caller's arrays: Sigma stays to the bit when 1 - V Pi is singular,
+Sigma and W when an input is not finite."""
 import numpy as np
 import pytest
 
@@ -40,4 +41,22 @@ def test_singular_leaves_sigma(kgrid, no, nmu, flags):
     assert torch.equal(S, S0)
     S1, W1, _ = ctx.gw_iteration(G, X, V, Sigma=S, W_qt=W)  # and the context goes on
     assert torch.isfinite(torch.view_as_real(S1)).all() and torch.isfinite(torch.view_as_real(W1)).all()
+    ctx.close()
+
+
+@pytest.mark.parametrize("flags", [{}, {10: 1}, {6: 1, 7: 1}, {6: 2, 7: 1, 10: 1}, {2: 1}],
+                         ids=["plain", "hermitian-G", "mixed", "mixed-resolvent", "one-pair-per-batch"])
+@pytest.mark.parametrize("bad", ["G", "X", "V"])
+def test_nonfinite_input_leaves_both(bad, flags):
+    import torch
+
+    from coqui_amd import ThcgwError
+
+    ctx, G, X, V, S, W = _system((2, 2, 1), 4, 24, flags)
+    S0, W0 = S.clone(), W.clone()
+    {"G": G, "X": X, "V": V}[bad].view(-1)[-1] = float("nan")
+    with pytest.raises(ThcgwError) as e:
+        ctx.gw_iteration(G, X, V, Sigma=S, W_qt=W)
+    assert e.value.code == 6 and bad + "_" in str(e.value)
+    assert torch.equal(S, S0) and torch.equal(W, W0)
     ctx.close()
