@@ -732,7 +732,7 @@ void qsym_diff(hipStream_t s, const c128* A, int n, int nq, const int* src, cons
 
 void herm_diff(hipStream_t s, const c128* A, int n, long nb, int nbx, double* out) {
   // Whole matrices where there are as many as workgroups, else parts of at least 4096 elements: chi0 of one k
-  // point with 42 G(tau) of order 1000 takes 812 us, 1849 with a workgroup per matrix.
+  // point with 40 G(tau) of order 1000 takes 812 us, 1849 with a workgroup per matrix.
   const long parts = std::max(1L, std::min(nbx / std::max(nb, 1L), static_cast<long>(n) * n / 4096));
   const int rows = static_cast<int>((n + parts - 1) / parts);
   hipLaunchKernelGGL(herm_diff_kernel, dim3(nbx), dim3(T256), 0, s, A, n, nb, rows, out);
