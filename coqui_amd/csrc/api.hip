@@ -28,6 +28,22 @@ namespace {
 
 thread_local std::string g_create_error;
 
+// A point of a stream that the host can wait for.  Kept by the context: making one costs as much as a launch.
+struct Event {
+  hipEvent_t e = nullptr;
+  Event() = default;
+  Event(const Event&) = delete;
+  Event& operator=(const Event&) = delete;
+  ~Event() {
+    if (e) (void)hipEventDestroy(e);
+  }
+  void record(hipStream_t s) {
+    if (!e) THCGW_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    THCGW_HIP(hipEventRecord(e, s));
+  }
+  void wait() const { THCGW_HIP(hipEventSynchronize(e)); }
+};
+
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
@@ -111,6 +127,7 @@ struct thcgw_ctx {
   bool deferred = false;  // enqueue without host synchronisation (stream capture): checks run later
   char* readback_p = nullptr;  // pinned memory for results that the host looks at while the stream goes on
   size_t readback_bytes = 0;
+  Event inputs_checked, dyson_solved;  // of an iteration at hand
   int nf_arrays = 0;      // arrays whose non-finite counts a deferred enqueue left in "nf_cnt"
   std::map<std::string, DevBuf>* pool = nullptr;  // scratch shared with the other systems of a batch
   // cgemm flags of this context: precision and FP32 tile shape
@@ -958,32 +975,14 @@ struct FiniteArg {
 };
 constexpr int kNonfiniteBlocks = 1024;  // 16 waves per CU
 
-// A point of a stream that the host can wait for.
-struct Event {
-  hipEvent_t e = nullptr;
-  Event() = default;
-  Event(const Event&) = delete;
-  Event& operator=(const Event&) = delete;
-  ~Event() {
-    if (e) (void)hipEventDestroy(e);
-  }
-  void record(hipStream_t s) {
-    if (!e) THCGW_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    THCGW_HIP(hipEventRecord(e, s));
-  }
-  void wait() const {  // at once where nothing was recorded
-    if (e) THCGW_HIP(hipEventSynchronize(e));
-  }
-};
-
 // A check whose counts are on their way to pinned memory: refuse() waits for them.
 struct PendingFinite {
   std::string entry;
   std::vector<FiniteArg> a;
   const int* h = nullptr;
-  Event ready;
+  const Event* ready = nullptr;
   void refuse() const {
-    ready.wait();
+    if (ready) ready->wait();
     for (size_t i = 0; i < a.size(); ++i) {
       long bad = 0;
       for (int b = 0; b < kNonfiniteBlocks; ++b) bad += h[i * kNonfiniteBlocks + b];
@@ -1022,7 +1021,8 @@ void check_finite(thcgw_ctx* ctx, const char* entry, std::initializer_list<Finit
   c.h = later ? pinned : h.data();
   THCGW_HIP(hipMemcpyAsync(const_cast<int*>(c.h), cnt, sizeof(int) * a.size() * kNonfiniteBlocks, hipMemcpyDeviceToHost, s));
   if (later) {
-    c.ready.record(s);
+    ctx->inputs_checked.record(s);
+    c.ready = &ctx->inputs_checked;
   } else {
     THCGW_HIP(hipStreamSynchronize(s));
     c.refuse();
@@ -1442,15 +1442,14 @@ void enqueue_iteration(thcgw_ctx* ctx, const c128* G, const c128* X, const c128*
     ctx->pi_lower = lower;
     run_dyson(ctx, Piw, V, dtr, dld, true, false, s, finish ? reinterpret_cast<int*>(pin + at_info) : nullptr);
   }
-  Event solved;
-  if (finish) solved.record(s);
+  if (finish) ctx->dyson_solved.record(s);
   if (finish && want_ec) {
     THCGW_HIP(hipMemcpyAsync(pin + at_tr, dtr, sizeof(c128) * total, hipMemcpyDeviceToHost, s));
     THCGW_HIP(hipMemcpyAsync(pin + at_tr + sizeof(c128) * total, dld, sizeof(double) * total, hipMemcpyDeviceToHost, s));
   }
   run_w_to_tau(ctx, Piw, Wqt, s);
   run_sigma(ctx, G, Wqt, X, Sig, herm, s, true, finish ? BeforeWrite([&] {
-    solved.wait();
+    ctx->dyson_solved.wait();
     refuse_singular(reinterpret_cast<const int*>(pin + at_info), total, ctx->nk);
   }) : BeforeWrite());
   if (!finish) return;
