@@ -15,7 +15,7 @@
 //
 // The factorisation is recursive on the lower triangle: factor A11, A21 <- A21 L11^-H,
 // A22 <- A22 - A21 A21^H (lower tiles only), factor A22.  Leaves of order <= 32 are
-// factored in LDS by one workgroup per matrix.  Only the lower triangle of a factored
+// factored in registers by one workgroup per matrix.  Only the lower triangle of a factored
 // matrix is defined.
 #include "lri.hpp"
 #include "thcgw_internal.hpp"
@@ -529,8 +529,8 @@ void tri_inverse_conj(hipStream_t s, const c128* L, long sL, int ldl, c128* Z, l
 }
 
 // X L^H = T as trsm_right_lower_conj in FP32 arithmetic, T and L stored as complex<float>;
-// gemm_flags selects the product of the updates (0: FP32 MFMA, GEMM_SPLIT_BF16).  The leaves are 64 wide (64 complex<float> per thread), so that no
-// update product is narrower than the 64 x 64 GEMM tile.
+// gemm_flags selects the product of the updates (0: FP32 MFMA, GEMM_SPLIT_BF16).  The leaves are 64
+// wide (a vector over 16 lanes), so that no update product is narrower than the 64 x 64 GEMM tile.
 constexpr int CB32 = 64;
 
 void trsm_right_lower_conj_f32(hipStream_t s, const c64* L, long sL, int ldl, c64* T, long sT, int ldt, int m,

@@ -7,7 +7,12 @@
 // (Wilkinson, The Algebraic Eigenvalue Problem, 7.11) gives the determinant up to a factor that does
 // not depend on z: with x_{n-1} = 1, the rows i = n-1 .. 1 of (z - H) x = 0 give x_{i-1}, and row 0
 // leaves a number p proportional to det(z - H); differentiated along, p'/p is the trace, 8 n^2 flops.
-// Both steps are backward stable like the inverse.
+// The reflections are backward stable.  The recurrence and its derivative round independently, with an error of
+// order eps cond(z - A) for the trace, the inverse's.  N against extended precision (rms over 40 to 60 random
+// H(k) + Sigma and four mu, in 1e-16 n): inverses 4.4 at any order, this 4.6 at order 8, 5.7 at 32, 6.4 at 78:
+// 5e-14 there, against the mu_tol that ends the search (1e-9).  Sums of the recurrence with their rounding
+// errors took 40% longer and left it at 6.9: what remains is the rounding of x and its derivative.
+// Where p underflows the trace is not finite, and that mu goes to the inverses.
 // Search of 34 evaluations at N_k = 64, 80 frequencies, order 78, with G(tau) at its end: 48.9 ->
 // 7.9 ms.
 #include "thcgw_internal.hpp"

@@ -47,8 +47,9 @@ __device__ __forceinline__ dd mul_d(dd x, double y) {
   p.lo += x.lo * y;
   return quick_two_sum(p.hi, p.lo);
 }
-// a / y with r = 1 / y rounded: the quotient a r corrected by its remainder is a / y correctly rounded
-// (Markstein, IBM J. Res. Dev. 34, 1990)
+// a / y with r = 1 / y rounded: the quotient a r corrected by its remainder (Markstein, IBM J. Res. Dev.
+// 34, 1990), which is a / y correctly rounded where a r is within one ulp of it and nearly so elsewhere.  The
+// double-double quotient takes its remainders from these values, whatever their last bit.
 __device__ __forceinline__ double quotient(double a, double y, double r) {
   const double q = a * r;
   return fma(fma(-q, y, a), r, q);

@@ -24,7 +24,8 @@ struct Cplx {
   double re, im;
 };
 
-enum Op : int { OP_N = 0, OP_T = 1, OP_C = 2 };
+// The profile's classes are 3 op(A) + op(B); 1, a transpose without conjugation, is not built.
+enum Op : int { OP_N = 0, OP_C = 2 };
 
 struct Error : std::runtime_error {
   int code;

@@ -3,7 +3,7 @@
 // or complex<float> independently of the arithmetic (conversion happens on the way
 // through LDS and in the epilogue).
 //
-//   C[b] = alpha * op(A[b]) * op(B[b]) + beta * C[b] + gamma * I,   op in {N, T, C}
+//   C[b] = alpha * op(A[b]) * op(B[b]) + beta * C[b] + gamma * I,   op in {N, C}
 //
 // All matrices are row-major with explicit leading dimensions.  One 256-thread
 // workgroup (four waves, 2 x 2) computes a BM x BN tile of C; each wave owns every other
@@ -954,8 +954,8 @@ void launch_f32(hipStream_t s, Args a) {
 
 std::atomic<int> g_tile_mode{0};  // 0 = automatic, else shape + 1
 
-// 64 x 64 tiles by default: at three waves per SIMD they hide load latency better than
-// the larger shapes at one wave per SIMD (measured on the N_k = 64, N_mu = 800 iteration: 45.8 vs 26.4 TFLOP/s).
+// 64 x 64 tiles by default: at four waves per SIMD (three with three products) they hide load latency
+// better than the larger shapes at one wave per SIMD (measured on the N_k = 64, N_mu = 800 iteration: 45.8 vs 26.4 TFLOP/s).
 int tile_shape(int, int, int) {
   const int forced = g_tile_mode.load();
   return forced > 0 ? forced - 1 : 0;
