@@ -482,7 +482,12 @@ def main():
         "roofline": {"kernel": "%s (GEMM class %s of the %s form)" % (gemm_kernel_name(cls, bool(FORMS[args.headline][3] and args.g3_mask & 1)),
                                                                        cls, args.headline),
                      "bound": "mfma", "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
-                     "frac": round(achieved / peak, 4), "traffic": traffic, "traffic_source": traffic_src,
+                     "frac": round(achieved / peak, 4),
+                     # achieved counts 8 flops per complex multiply-add, of which the three-product FP64 kernels
+                     # execute 6: the share of the peak that the matrix cores work at
+                     "executed_frac": (round(achieved / peak * (0.75 if FORMS[args.headline][3] and args.g3_mask & 1 else 1.0), 4)
+                                       if peak == FP64_PEAK_TFLOPS else None),
+                     "traffic": traffic, "traffic_source": traffic_src,
                      "algorithmic_bytes_per_launch": round(g_by / max(g_n, 1)),
                      "flops_per_launch": round(g_fl / max(g_n, 1)),
                      "launches": g_n, "avg_launch_ms": round(g_ms / max(g_n, 1), 4),

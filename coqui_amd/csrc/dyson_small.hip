@@ -43,7 +43,8 @@ __device__ __forceinline__ void csub(c128& c, c128 a, c128 b) {
 // SOLVE: W[b] = A^-1 V - V with V's member (b0 + b) % vmod; otherwise the trace and the determinant only.
 template <int T, int E, bool SOLVE>
 __global__ __launch_bounds__(T* T) __attribute__((amdgpu_waves_per_eu(!SOLVE || T == 32 || E < 3 ? 4 : E == 3 ? 3 : 2)))
-void dyson_small_kernel(const c128* D, const c128* V, int vmod, int b0, int n, c128* W, c128* tr, double* ldet, int* info) {
+void dyson_small_kernel(const c128* D, const c128* V, int vmod, int b0, int n, c128* W, c128* tr, double* ldet,
+                        int* info) {
   constexpr int N = T * E, NW = T * T / 64, EB = SOLVE ? E : 1;
   __shared__ c128 colv[2][N], rowv[N], scale[N], pivot[N];
   __shared__ c128 delta[N];  // element (k, k) of D before step k
@@ -116,7 +117,8 @@ void dyson_small_kernel(const c128* D, const c128* V, int vmod, int b0, int n, c
       // fmin: a NaN or an infinity becomes a pivot by its place and is found by its value then
       const double mag = fmin(fabs(v[a][q].x) + fabs(v[a][q].y), DBL_MAX);
       const unsigned off = (used << (31 - a)) & 0x80000000u;  // negative: loses every maximum
-      const unsigned lo = (static_cast<unsigned>(__double2loint(mag)) & ~127u) | static_cast<unsigned>(127 - (r + a * T));
+      const unsigned lo =
+          (static_cast<unsigned>(__double2loint(mag)) & ~127u) | static_cast<unsigned>(127 - (r + a * T));
       best = fmax(best, __hiloint2double(static_cast<int>(static_cast<unsigned>(__double2hiint(mag)) | off),
                                          static_cast<int>(lo)));
     }
@@ -265,8 +267,8 @@ void dyson_small(hipStream_t s, const c128* D, const c128* V, int vmod, int b0, 
   auto go = [&](auto t, auto e) {
     constexpr int T = t, E = e;
     if (W)
-      hipLaunchKernelGGL((dyson_small_kernel<T, E, true>), dim3(batch), dim3(T * T), 0, s, D, V, vmod, b0, n, W, tr, ldet,
-                         info);
+      hipLaunchKernelGGL((dyson_small_kernel<T, E, true>), dim3(batch), dim3(T * T), 0, s, D, V, vmod, b0, n, W, tr,
+                         ldet, info);
     else
       hipLaunchKernelGGL((dyson_small_kernel<T, E, false>), dim3(batch), dim3(T * T), 0, s, D, V, vmod, b0, n, W, tr,
                          ldet, info);

@@ -14,7 +14,7 @@
 // errors took 40% longer and left it at 6.9: what remains is the rounding of x and its derivative.
 // Where p underflows the trace is not finite, and that mu goes to the inverses.
 // Search of 34 evaluations at N_k = 64, 80 frequencies, order 78, with G(tau) at its end: 48.9 ->
-// 7.9 ms.
+// 8.2 ms.
 #include "thcgw_internal.hpp"
 #include "wave.hpp"
 
