@@ -222,8 +222,9 @@ int thcgw_rpa_ec(thcgw_ctx* ctx, const double* Pi_wqPQ, const double* V_qPQ, dou
  * scr_coulomb_t::update_w + gw_t::evaluate as called by scf_loop
  * (src/methods/SCF/scf_driver.cpp:119-122) and gw_t::rpa_energy (thc_rpa.cpp:22-61).
  * W_qtPQ (caller-owned, nk*nt_half*nmu^2 complex) receives W - V; it also serves as
- * scratch for Pi_tqPQ.  A call refused for its arguments or inputs leaves both output arrays
- * as they were; one refused as singular leaves Sigma_tskij.  Synchronises the stream. */
+ * scratch for Pi_tqPQ.  A call refused for a NaN or infinity in its inputs or for flag 10 leaves
+ * both output arrays as they were; one refused as singular, or for the symmetry of flag 9 or
+ * thcgw_set_qsym, leaves Sigma_tskij.  Synchronises the stream. */
 int thcgw_gw_iteration(thcgw_ctx* ctx, const double* G_tskij, const double* X_skPa, const double* V_qPQ,
                        double* Sigma_tskij, double* W_qtPQ, double* Ec, int hermitize, void* stream);
 
